@@ -317,13 +317,13 @@ def batched_kernel(M, N, K):
     projection (the selection in csrc/capi.hip linear_w4 and csrc/w4_mfma.hip
     w4_mfma): M = 3..16 takes the small-batch f16-MFMA limb kernel (exact
     products from f16 limbs of x), except M = 16 with N and K at most 4096,
-    which stays on FP32 MFMA; from M = 17 (K a multiple of 128) the batched
-    limb GEMM.  Every entry's frac_fp32_mfma_peak is its f32-contraction rate
-    over the FP32-MFMA peak; the limb kernels get there on f16 MFMA."""
+    which stays on FP32 MFMA; from M = 17 the batched f16-limb GEMM.  Every
+    entry's frac_fp32_mfma_peak is its f32-contraction rate over the FP32-MFMA
+    peak; the limb kernels get there on f16 MFMA."""
     if 3 <= M <= 16 and not (M == 16 and N <= 4096 and K <= 4096):
         return "k_limb_prep + k_w4_limb (f16 MFMA on exact limbs of x) + k_limb_reduce"
-    if M >= 17 and K % 128 == 0:
-        return "k_lgemm_prep + k_w4_lgemm (f16 MFMA on exact limbs of x, 16-row slabs) + k_mfma_reduce"
+    if M >= 17:
+        return "k_qsplit + k_qgemm (f16 MFMA on two f16 limbs of x) + k_qreduce"
     return "k_w4_mfma (FP32 MFMA) + k_mfma_reduce"
 
 
@@ -584,7 +584,7 @@ def prefill_run(dec, cfg, n):
     return {"tokens": n, "ms": round(sec * 1e3, 3), "tok_s": round(n / sec, 1),
             "tflops": round(fl / sec / 1e12, 2), "flops": fl,
             "mfma_fp32_frac": round(fl / sec / 1e12 / MFMA_F32_PEAK, 4),
-            "kernel": "k_w4_lgemm (f16 MFMA on exact limbs of x) for the projections; "
+            "kernel": "k_qgemm (f16 MFMA on two f16 limbs of x) for the projections; "
                       "mfma_fp32_frac is the f32-contraction rate over the FP32-MFMA peak"}
 
 

@@ -1,0 +1,108 @@
+"""The batched f16-limb projection (17 or more rows) at the edges of its tiles:
+rows around 32 and 64, column blocks of 128 and 256, K that is no whole number
+of 128-element stages, K splits, every scale form, and rows of extreme or
+non-finite activations.  Against float64; the bound follows the kernel: two f16
+limbs hold an activation to 2^-22, and every sum is f32, one addition per 32
+elements of K plus the splits', so an output is off by at most
+(K / 32 + 16) 2^-24 sum |w x|."""
+import numpy as np
+import pytest
+import torch
+
+import torchburn_amd as tb
+from torchburn_amd import _lib, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def deq4(w, s, gs):
+    q = np.stack((w & 15, w >> 4), -1).reshape(w.shape[0], -1).astype(np.float64) - 8
+    return q * (np.repeat(s.astype(np.float64), gs, 1) if s.ndim == 2 else s.astype(np.float64)[:, None])
+
+
+def check(y, x, w, bias=None, res=None):
+    """y against x w^T (+ bias) (+ res) within the bound above, row by row where finite."""
+    xd = x.astype(np.float64)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = xd @ w.T
+        mag = np.abs(xd) @ np.abs(w).T
+    for t in (bias, res):
+        if t is not None:
+            ref = ref + t.astype(np.float64)
+            mag = mag + np.abs(t)
+    bound = (x.shape[1] / 32 + 16) * 2.0 ** -24 * mag + 1e-37
+    fin = np.isfinite(x).all(1)
+    assert np.isfinite(y[fin]).all()
+    assert (np.abs(y[fin] - ref[fin]) <= bound[fin]).all()
+    assert not np.isfinite(y[~fin]).any()
+    assert (np.isnan(y[~fin]) == np.isnan(ref[~fin])).all()
+    inf = ~np.isnan(ref[~fin])
+    assert (y[~fin][inf] == ref[~fin][inf].astype(np.float32)).all()
+
+
+@pytest.mark.parametrize("m,n,k,gs,v2", [
+    (17, 33, 160, 32, False), (32, 128, 128, 64, False), (33, 257, 2080, 32, False),
+    (64, 300, 4096, 128, False), (65, 130, 96, 32, False), (130, 515, 1600, 64, False),
+    (19, 70, 224, 0, False), (48, 129, 64, 64, True), (200, 65, 1600, 64, True)])
+def test_w4_projection_edges(cuda, m, n, k, gs, v2):
+    print(f"case qgemm w4 m={m} n={n} k={k} gs={gs} v2={v2}", flush=True)
+    g = synth.rng(71, m, n, k)
+    x = synth.activations(g, m, k)
+    x[:, 3::37] *= 50.0
+    b = synth.activations(g, n)
+    w, s = synth.int4_weight(g, n, k, gs or k)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    if gs == 0:
+        s = s.reshape(-1)
+        y = tb.w4a32_linear(T(x), T(w), T(s), T(b))
+    elif v2:
+        s = s.astype(np.float16).astype(np.float32)
+        y = tb.w4a32_grouped_linear_v2(T(x), tb.pack_rows_w4a32_group64_v1_to_v2(T(w), T(s), k), T(b))
+    else:
+        y = tb.w4a32_grouped_linear(T(x), T(w), T(s), T(b), group_size=gs)
+    check(y.cpu().numpy(), x, deq4(w, s, gs or k), b)
+
+
+def test_w4_extreme_and_nonfinite_rows(cuda):
+    m, n, k, gs = 40, 130, 1152, 32
+    g = synth.rng(72, m)
+    x = synth.activations(g, m, k)
+    x[1] *= 2.0 ** 100
+    x[2] *= 2.0 ** -110
+    x[3] = 0.0
+    x[4, :k // 2] *= 2.0 ** 60
+    x[33, 7] = np.inf
+    x[34, 100] = -np.inf
+    x[34, 1100] = np.inf
+    x[35, 64] = np.nan
+    w, s = synth.int4_weight(g, n, k, gs)
+    r = synth.activations(g, m, n)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    y = tb.w4a32_grouped_linear_residual(T(x), T(w), T(s), T(r), group_size=gs)
+    check(y.cpu().numpy(), x, deq4(w, s, gs), res=r)
+
+
+@pytest.mark.parametrize("m,k,inter,gs", [
+    (40, 2048, 4096, 32),    # limbs and partials within the scratch the entry point counts
+    (20, 4128, 64, 32)])     # limbs larger than that count: the FP32-MFMA form
+def test_noalloc_mlp_at_17_rows_or_more(cuda, m, k, inter, gs):
+    print(f"case qgemm noalloc m={m} k={k} inter={inter}", flush=True)
+    g = synth.rng(73, m, k)
+    x, r = synth.activations(g, m, k), synth.activations(g, m, k)
+    wts = [synth.int4_weight(g, n, kk, gs) for n, kk in ((inter, k), (inter, k), (k, inter))]
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    t = [T(a) for p in wts for a in p]
+    dx, dr = T(x), T(r)
+    P = lambda a: a.data_ptr()
+    outs = []
+    for name in ("tb_fused_swiglu_mlp_w4a32_noalloc", "tb_fused_swiglu_mlp_w4a32"):
+        out = torch.empty((m, k), device=cuda)
+        _lib.check(getattr(_lib.lib(), name)(
+            P(dx), P(t[0]), P(t[1]), None, P(t[2]), P(t[3]), None, P(t[4]), P(t[5]), None, P(dr),
+            P(out), m, k, inter, k, gs, torch.cuda.current_stream(cuda).cuda_stream))
+        outs.append(out.cpu().numpy())
+    gw, uw, dw = (deq4(w, s, gs) for w, s in wts)
+    a, u = x.astype(np.float64) @ gw.T, x.astype(np.float64) @ uw.T
+    ref = (a / (1 + np.exp(-a)) * u) @ dw.T + r
+    for o in outs:
+        assert np.abs(o - ref).max() / np.abs(ref).max() < 2e-6

@@ -44,9 +44,10 @@ HOST_SANITIZE_FLAGS = [
 ]
 
 
-# Per-source extra flags.  w4_limb: MFMA results in VGPRs (the kernel scales
+# Per-source extra flags.  w4_limb, qgemm: MFMA results in VGPRs (the kernels scale
 # every result with VALU; accumulators in AGPRs would cost a copy each).
 EXTRA_FLAGS = {
+    "qgemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "w4_limb.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 

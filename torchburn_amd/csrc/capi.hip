@@ -174,10 +174,11 @@ static MfmaParams mfma_params(const float *x, const uint8_t *w, const float *s, 
 // The MFMA projection with its split-K partials in the library workspace.
 static int mfma_ws(const MfmaParams &p, int epi, hipStream_t st) {
     WsLease lease;
-    int rc = workspace(w4_mfma_partials_bytes(p.m, p.n, p.k, p.w1 != nullptr), st, lease);
+    const size_t bytes = w4_mfma_scratch_bytes(p.m, p.n, p.k, p.w1 != nullptr);
+    int rc = workspace(bytes, st, lease);
     if (rc) return rc;
     void *ws = lease.ptr;
-    return w4_mfma(p, epi, static_cast<float *>(ws), st);
+    return w4_mfma(p, epi, static_cast<float *>(ws), bytes, st);
 }
 
 // Shapes of the small-batch f16-MFMA projection: limb_min_m() <= m <= limb_max_m(),
@@ -276,7 +277,7 @@ static int linear_w4(const float *x, const uint8_t *w, const float *s, bool v2,
     const size_t rest = any_shape ? 0
                         : lb ? up256(limb_records_bytes((int)m, (int)k)) +
                                    limb_partials_bytes((int)m, (int)n, (int)k, false)
-                        : mf ? w4_mfma_partials_bytes((int)m, (int)n, (int)k, false)
+                        : mf ? w4_mfma_scratch_bytes((int)m, (int)n, (int)k, false, v2)
                              : xq_bytes(m, k);
     const float *xin = x;
     void *tail = nullptr;
@@ -308,7 +309,7 @@ static int linear_w4(const float *x, const uint8_t *w, const float *s, bool v2,
         q.res = res;
         q.v2 = v2 ? 1 : 0;
         q.scale_mode = scale_mode;
-        return w4_mfma(q, epi, static_cast<float *>(tail), st);
+        return w4_mfma(q, epi, static_cast<float *>(tail), rest, st);
     }
     W4Params p = w4_params(xin, w, s, bias, out, m, n, k, gs);
     p.res = res;
@@ -397,6 +398,7 @@ struct MlpW4 {
     const float *down_s, *down_b, *residual;
     float *out;
     int64_t m, k, inter, n_out, gs;
+    size_t part_cap;   // the batched projections' scratch is at most this
 };
 
 static int mlp_w4_check(const MlpW4 &a, const char *op) {
@@ -409,7 +411,7 @@ static int mlp_w4_check(const MlpW4 &a, const char *op) {
     return TB_OK;
 }
 
-// 0: any-shape GEMVs; 1: FP32-MFMA pair; 2: GEMV passes; 3: small-batch f16 MFMA
+// 0: any-shape GEMVs; 1: batched pair (w4_mfma); 2: GEMV passes; 3: small-batch f16 MFMA
 static int mlp_w4_path(const MlpW4 &a) {
     if (limb_fast(a.x, a.gate_w, a.m, a.inter, a.k, a.gs, false, true) &&
         aligned(a.up_w, 16) &&
@@ -421,7 +423,7 @@ static int mlp_w4_path(const MlpW4 &a) {
     return a.m >= mfma_min_m() ? 1 : 2;
 }
 
-// Scratch: h [m, inter] f32, then the MFMA split-K partials (path 1), the
+// Scratch: h [m, inter] f32, then the batched projections' scratch (path 1), the
 // chunk records of x and of h (path 2) or their f16-limb records (path 3).
 // W4A8 semantics (tb_set_vnni_semantics) at group 64: the reference rounds x to
 // bytes before the gate / up pair (fused_ops.rs:215-232) and h before the down
@@ -430,12 +432,22 @@ static bool mlp_a8(const MlpW4 &a) { return a.gs == 64 && vnni_semantics(); }
 
 static size_t mlp_w4_scratch_main(const MlpW4 &a);
 
+static size_t mlp_part_bytes(const MlpW4 &a) {
+    return std::min(
+        a.part_cap,
+        std::max(w4_mfma_scratch_bytes((int)a.m, (int)a.inter, (int)a.k, true),
+                 w4_mfma_scratch_bytes((int)a.m, (int)a.n_out, (int)a.inter, false)));
+}
+
 // [path scratch | x' (m x k) | h' (m x inter)], the last two under W4A8 only.
-static size_t mlp_w4_scratch_bytes(const MlpW4 &a) {
-    const size_t main = mlp_w4_scratch_main(a);
+static size_t mlp_w4_with_a8(const MlpW4 &a, size_t main) {
     if (!mlp_a8(a)) return main;
     return up256(main) + up256((size_t)a.m * (size_t)a.k * sizeof(float)) +
            up256((size_t)a.m * (size_t)a.inter * sizeof(float));
+}
+
+static size_t mlp_w4_scratch_bytes(const MlpW4 &a) {
+    return mlp_w4_with_a8(a, mlp_w4_scratch_main(a));
 }
 
 static size_t mlp_w4_scratch_main(const MlpW4 &a) {
@@ -448,11 +460,7 @@ static size_t mlp_w4_scratch_main(const MlpW4 &a) {
                    std::max(limb_partials_bytes((int)a.m, (int)a.inter, (int)a.k, true),
                             limb_partials_bytes((int)a.m, (int)a.n_out, (int)a.inter, false));
         }
-        case 1: {
-            const size_t pg = w4_mfma_partials_bytes((int)a.m, (int)a.inter, (int)a.k, true);
-            const size_t pd = w4_mfma_partials_bytes((int)a.m, (int)a.n_out, (int)a.inter, false);
-            return hb + std::max(pg, pd);
-        }
+        case 1: return hb + mlp_part_bytes(a);
         default: return hb + up256(xq_bytes(a.m, a.k)) + xq_bytes(a.m, a.inter);
     }
 }
@@ -510,13 +518,14 @@ static int mlp_w4_run(const MlpW4 &a, void *ws, hipStream_t st) {
     }
     if (path == 1) {
         float *part = reinterpret_cast<float *>(static_cast<char *>(ws) + hb);
+        const size_t pb = mlp_part_bytes(a);
         MfmaParams g = mfma_params(x, a.gate_w, a.gate_s, a.gate_b, h, m, inter, k, gs);
         g.w1 = a.up_w; g.s1 = a.up_s; g.b1 = a.up_b;
-        if ((rc = w4_mfma(g, EPI_SWIGLU, part, st))) return rc;
+        if ((rc = w4_mfma(g, EPI_SWIGLU, part, pb, st))) return rc;
         if (a8 && (rc = act_u8(h, ha, m, inter, st))) return rc;
         MfmaParams d = mfma_params(hin, a.down_w, a.down_s, a.down_b, a.out, m, n_out, inter, gs);
         d.res = a.residual;
-        return w4_mfma(d, a.residual ? EPI_RESID : EPI_PLAIN, part, st);
+        return w4_mfma(d, a.residual ? EPI_RESID : EPI_PLAIN, part, pb, st);
     }
     uint32_t *xq = reinterpret_cast<uint32_t *>(static_cast<char *>(ws) + hb);
     uint32_t *hq = reinterpret_cast<uint32_t *>(static_cast<char *>(ws) + hb +
@@ -550,6 +559,20 @@ static int mlp_w4_run(const MlpW4 &a, void *ws, hipStream_t st) {
 // stand-in of the array; its device address (per device) comes from
 // hipGetSymbolAddress and is the only form passed to kernels.
 constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
+
+// Bytes that the entry point counts for a batched projection of m rows: split-K
+// partials of 64-row tiles in about 512 blocks and, from 17 rows at K % 128 ==
+// 0, 8224 bytes per 16 rows and 128 of K.  The sizes it takes are a promise of
+// its header, so this count stays what it was, whatever the kernels use of it.
+static size_t noalloc_part_bytes(int64_t m, int64_t n, int64_t k, bool dual) {
+    const int64_t tiles = (m + 15) / 16, mz = (tiles + std::min<int64_t>(tiles, 4) - 1) /
+                                              std::min<int64_t>(tiles, 4);
+    const int64_t blocks = (n + 63) / 64 * (dual ? 2 : 1) * mz, steps = (k + 127) / 128;
+    const int64_t want = std::max<int64_t>(1, std::min((512 + blocks - 1) / blocks, steps));
+    const int64_t klen = (steps + want - 1) / want * 128, splits = (k + klen - 1) / klen;
+    const size_t pb = up256((size_t)(dual ? 2 : 1) * splits * m * n * sizeof(float));
+    return pb + (m >= 17 && k % 128 == 0 ? (size_t)tiles * (k / 128) * 8224 : 0);
+}
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -823,7 +846,7 @@ int tb_fused_swiglu_mlp_w4a32(const float *x, const uint8_t *gate_w, const float
                               int64_t m, int64_t k, int64_t inter, int64_t n_out,
                               int64_t group_size, void *stream) {
     const MlpW4 a{x, gate_w, gate_s, gate_b, up_w, up_s, up_b, down_w, down_s, down_b,
-                  residual, out, m, k, inter, n_out, group_size};
+                  residual, out, m, k, inter, n_out, group_size, SIZE_MAX};
     int rc = mlp_w4_check(a, "fused_swiglu_mlp_w4a32");
     if (rc || m == 0 || n_out == 0) return rc;
     hipStream_t st = (hipStream_t)stream;
@@ -839,11 +862,18 @@ int tb_fused_swiglu_mlp_w4a32_noalloc(const float *x, const uint8_t *gate_w,
                                       const float *down_b, const float *residual, float *out,
                                       int64_t m, int64_t k, int64_t inter, int64_t n_out,
                                       int64_t group_size, void *stream) {
-    const MlpW4 a{x, gate_w, gate_s, gate_b, up_w, up_s, up_b, down_w, down_s, down_b,
-                  residual, out, m, k, inter, n_out, group_size};
+    MlpW4 a{x, gate_w, gate_s, gate_b, up_w, up_s, up_b, down_w, down_s, down_b,
+            residual, out, m, k, inter, n_out, group_size, SIZE_MAX};
     int rc = mlp_w4_check(a, "fused_swiglu_mlp_w4a32_noalloc");
     if (rc || m == 0 || n_out == 0) return rc;
-    const size_t need = mlp_w4_scratch_bytes(a);
+    size_t need = 0;
+    if (mlp_w4_path(a) == 1) {
+        a.part_cap = std::max(noalloc_part_bytes(m, inter, k, true),
+                              noalloc_part_bytes(m, n_out, inter, false));
+        need = mlp_w4_with_a8(a, up256((size_t)m * (size_t)inter * sizeof(float)) + a.part_cap);
+    } else {
+        need = mlp_w4_scratch_bytes(a);
+    }
     TB_REQUIRE(need <= kNoAllocScratchBytes, TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: fused_swiglu_mlp_w4a32_noalloc: this shape needs " +
                    std::to_string(need) + " bytes of scratch; the static scratch holds " +

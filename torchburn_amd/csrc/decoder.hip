@@ -568,16 +568,17 @@ struct Decoder {
     static constexpr int kPrefillRows = 256;
     float *pf_x = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr, *pf_q = nullptr,
           *pf_a = nullptr, *pf_h = nullptr, *pf_part = nullptr;
+    size_t pf_part_bytes = 0;
     int *pf_tok = nullptr;
 
     int prefill_alloc() {
         if (pf_x) return TB_OK;
         const int R = kPrefillRows;
         const size_t nq = (size_t)(hq + 2 * hkv) * hd;
-        size_t part = w4_mfma_partials_bytes(R, (int)nq, H, false);
-        part = std::max(part, w4_mfma_partials_bytes(R, H, hq * hd, false));
-        part = std::max(part, w4_mfma_partials_bytes(R, I, H, true));
-        part = std::max(part, w4_mfma_partials_bytes(R, H, I, false));
+        size_t part = w4_mfma_scratch_upto(R, (int)nq, H, false);
+        part = std::max(part, w4_mfma_scratch_upto(R, H, hq * hd, false));
+        part = std::max(part, w4_mfma_scratch_upto(R, I, H, true));
+        part = std::max(part, w4_mfma_scratch_upto(R, H, I, false));
         // 3..16 rows (verify_tokens, short chunks) take the small-batch
         // projection: records + split partials of the largest of its shapes
         size_t lb = 0;
@@ -600,6 +601,7 @@ struct Decoder {
             (lb && (rc = alloc(&pf_hrec, limb_records_bytes(kLimbMaxM, I)))))
             return rc;
         pf_limb_bytes = lb;
+        pf_part_bytes = part;
         return TB_OK;
     }
 
@@ -659,7 +661,7 @@ struct Decoder {
         p.w0 = static_cast<const uint8_t *>(w); p.s0 = s; p.b0 = b;
         p.w1 = static_cast<const uint8_t *>(w2); p.s1 = s2;
         p.res = res; p.y = y; p.m = m; p.n = n; p.k = k; p.gshift = gshift(gs);
-        return w4_mfma(p, epi, pf_part, st);
+        return w4_mfma(p, epi, pf_part, pf_part_bytes, st);
     }
 
     // Positions start .. start + n - 1 attend every earlier position (the
@@ -690,16 +692,15 @@ struct Decoder {
             if (M <= 8 && limb_gemm(xr, lm_w, lm_s, nullptr, nullptr, nullptr, nullptr, y, M, V, H,
                                     rc))
                 return rc;
-            if (!pf_lmpart &&
-                (rc = alloc(&pf_lmpart, w4_mfma_partials_bytes(64, V, H, false))))
-                return rc;
+            const size_t lb = w4_mfma_scratch_upto(64, V, H, false);
+            if (!pf_lmpart && (rc = alloc(&pf_lmpart, lb))) return rc;
             for (int r0 = 0; r0 < M; r0 += 64) {
                 MfmaParams p{};
                 p.x = xr + (size_t)r0 * H;
                 p.w0 = static_cast<const uint8_t *>(lm_w); p.s0 = lm_s;
                 p.y = y + (size_t)r0 * V; p.m = std::min(64, M - r0); p.n = V; p.k = H;
                 p.gshift = gshift(gs);
-                if ((rc = w4_mfma(p, EPI_PLAIN, pf_lmpart, st))) return rc;
+                if ((rc = w4_mfma(p, EPI_PLAIN, pf_lmpart, lb, st))) return rc;
             }
             return TB_OK;
         }

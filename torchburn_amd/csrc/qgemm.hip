@@ -1,0 +1,658 @@
+// Batched quantized projection Y[M, N] = X[M, K] . deq(W)^T on f16 MFMA
+// (v_mfma_f32_32x32x16_f16) for INT4 (v1 nibbles, v2 blocks) and INT8 weights.
+//
+// Replaces the M > 1 path of the reference's w4a32_grouped_linear
+// (src/quantization/packed_v2.rs:557-624 -> gemm_w4a32_grouped,
+// src/quantization/gemv.rs:1690-1725), w8a32_linear (gemv.rs:974-1061) and the
+// batched SwiGLU of fused_swiglu_mlp_batched_w4a32
+// (src/quantization/fused_ops.rs:1267-1319), which run one GEMV per activation
+// row; here a weight byte is read once per block of activation rows.
+//
+// Arithmetic.  A stored weight is a small integer, exact in f16: the nibble q
+// becomes (1024 + q) - 1032 (one AND-OR and half a packed subtraction; a nibble
+// at bits 4-7 becomes 16 (q - 8), and its activation is divided by 16), an INT8
+// code b becomes (1024 + b + 128) - 1152.  An activation is scaled by a power
+// of two 2^e (the largest magnitude of its row in the block's K range lands in
+// [2^14, 2^15)) and split into two f16 limbs, x 2^e = h1 + h2 + r with
+// |r| <= 2^-22 |x 2^e| (or 2^-25 absolute, 2^-39 of the row's largest).  Both
+// limbs accumulate in one f32 MFMA chain over 32 elements, smaller limb first;
+// the chain's result takes the group scale and is added in f32, and the row's
+// 2^-e is applied once at the end.
+// Inf and NaN travel through the first limb, as in the reference's
+// unpack-and-fma.
+//
+// Why two limbs on f16: f32 MFMA runs at 1/16 of the f16 rate, three int8
+// limbs at twice the f16 rate would need an integer-to-float conversion per
+// result and group, and one exponent per row instead of one per 64 elements
+// leaves a single multiply-add per result and group on the vector ALUs.
+//
+// Tiling.  A block is four waves side by side along N, each 32 MT activation
+// rows x 32 NT weight rows.  The limbs of the block's rows go to LDS by direct
+// global-to-LDS loads, one K stage (SG groups of 32) ahead, and are read by
+// all four waves; a lane's weights (one 16-byte chunk per 32 rows x 64 K) and
+// scales go straight to registers, one stage ahead, and are expanded there.
+// Lane (i, h) = (l % 32, l / 32) loads group 2 j + h of weight row i;
+// v_permlane32_swap then leaves dwords 2 h and 2 h + 1 of each group in half
+// h, so K slot (u, h, e) of a group (step u of two) is element
+// 16 h + 8 u + e, and the records hold x in that order.
+//
+// Bound: the matrix cores, at the clock this card holds under a dense f16
+// product (a large library product in bf16 runs at 1.2 PFLOP/s, half the
+// nominal rate).  Measured on whole calls, against the kernel on fixed-point
+// limbs with an exponent per 64 elements and two more MFMAs per group for the
+// -8 of the weights that this one replaced:
+//   Llama-3-8B gate/up pair, 512 rows, group 32    271 us, 444 TFLOP/s (888 in
+//                                                  MFMA work)
+//   Llama-3-8B MLP, 512 rows, group 64             951 -> 504 us
+//   64 rows, N = 14336, K = 4096, group 32         54.6 -> 33.7 us
+// and the error against 64 bits went from 6.2e-7 to 1.5e-7 (activations with
+// large channels; the limbs follow each element's own size).
+#include <math.h>
+
+#include <algorithm>
+
+#include "gemv_common.hpp"
+#include "qgemm.hpp"
+#include "tb_common.hpp"
+
+namespace tb {
+
+using namespace gemv;
+
+namespace {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+constexpr int kSlab = 32;            // activation rows of one MFMA tile
+constexpr int kGroupBytes = 4096;    // one slab x 32 K: 2 steps x 2 limbs x 1 KiB
+constexpr int kPad = 128;            // K is padded to whole stages in the records
+
+// K slot e of a step's 8 holds element slot_elem(e): the order in which a dword
+// of nibbles expands; slots with (e & 2) hold 16 x weights.
+__host__ __device__ constexpr int slot_elem(int e) { return (e >> 1) | ((e & 1) << 2); }
+
+__device__ __forceinline__ h8 expand_w4(uint32_t d) {
+    const uint32_t u = d >> 8, o = 0x64006400u;
+    const u32x4 v = {(d & 0x000F000Fu) | o, (d & 0x00F000F0u) | o, (u & 0x000F000Fu) | o,
+                     (u & 0x00F000F0u) | o};
+    const h8 c = {(_Float16)-1032.f, (_Float16)-1032.f, (_Float16)-1152.f, (_Float16)-1152.f,
+                  (_Float16)-1032.f, (_Float16)-1032.f, (_Float16)-1152.f, (_Float16)-1152.f};
+    return __builtin_bit_cast(h8, v) + c;
+}
+
+__device__ __forceinline__ h8 expand_w8(uint32_t d0, uint32_t d1) {
+    const uint32_t a = d0 ^ 0x80808080u, b = d1 ^ 0x80808080u, o = 0x64646464u;
+    const u32x4 v = {__builtin_amdgcn_perm(a, o, 0x00050004u), __builtin_amdgcn_perm(a, o, 0x00070006u),
+                     __builtin_amdgcn_perm(b, o, 0x00050004u), __builtin_amdgcn_perm(b, o, 0x00070006u)};
+    const _Float16 m = (_Float16)-1152.f;
+    return __builtin_bit_cast(h8, v) + h8{m, m, m, m, m, m, m, m};
+}
+
+struct QArgs {
+    const uint8_t *rec;    // split activations
+    const float *inv;      // [splits][slabs * 32] 2^-e
+    const uint8_t *w0, *w1;
+    const float *s0, *s1, *b0, *b1, *res;
+    float *y;              // [m, n], or the partials [splits][pair ? 2 : 1][m][n]
+    int m, n, k;
+    int scols, gshift, s0_len, s1_len;
+    int slabs, groups;     // 32-row slabs, padded 32-K groups of the records
+    int mz, nbx, splits, slen;   // row blocks, column blocks, K splits, groups per split
+};
+
+// SM: 0 a scale per 32-element group, 1 per 64 or more, 2 one per row (applied
+// in the epilogue).
+template <int FMT, int MT, int NT, int SM, bool PAIR>
+struct QTile {
+    static constexpr int SG = FMT == Q_W8 ? 2 : 4;   // groups per stage
+    static constexpr int LD = 2;                     // 16-byte chunks per lane and column tile
+    static constexpr int NDW = FMT == Q_V2 ? 5 : 4;
+    static constexpr int NS = SM == 0 ? 4 : 2;       // scales per column tile and stage
+
+    struct Stage {
+        uint32_t q[NT][LD][NDW];
+        float s[NT][NS];
+    };
+
+    const QArgs &a;
+    int lane, wave, i, h;
+    const uint8_t *wp[NT];   // the lane's weight row
+    const float *sp[NT];
+    uint32_t vrow[NT];       // byte offset of the lane's row (v2)
+    int chunks;              // 32-element chunks of a row
+
+    __device__ __forceinline__ QTile(const QArgs &aa) : a(aa) {
+        lane = threadIdx.x & 63;
+        wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        i = lane & 31;
+        h = lane >> 5;
+        chunks = a.k >> 5;
+    }
+
+    __device__ __forceinline__ int col(int bx, int nt) const {
+        return PAIR ? bx * 128 + 32 * wave + i : bx * (128 * NT) + 32 * (NT * wave + nt) + i;
+    }
+
+    __device__ __forceinline__ void rows(int bx) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const int c = col(bx, nt);
+            const size_t row = c < a.n ? c : 0;   // rows past n read row 0, never stored
+            const bool second = PAIR && nt == 1;
+            const uint8_t *w = second ? a.w1 : a.w0;
+            vrow[nt] = (uint32_t)row * (uint32_t)((a.k >> 6) * kV2Block);
+            wp[nt] = FMT == Q_V2 ? w : w + row * (size_t)(FMT == Q_W8 ? a.k : a.k >> 1);
+            sp[nt] = SM == 2 || FMT == Q_V2
+                         ? nullptr
+                         : (second ? a.s1 : a.s0) + row * (size_t)a.scols;
+        }
+    }
+
+    // Weights and scales of the stage at group g0.  Chunks past the row (K not
+    // a multiple of the stage) re-read its last chunk: their activations are 0.
+    __device__ __forceinline__ void load(int g0, Stage &st) const {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+            for (int j = 0; j < LD; ++j) {
+                if constexpr (FMT == Q_W8) {
+                    const int c = min(g0 + j, chunks - 1);
+                    const u32x4 v = *reinterpret_cast<const u32x4 *>(wp[nt] + 32 * (size_t)c + 16 * h);
+                    st.q[nt][j][0] = v.x; st.q[nt][j][1] = v.y; st.q[nt][j][2] = v.z; st.q[nt][j][3] = v.w;
+                } else if constexpr (FMT == Q_V2) {
+                    const int c = min(g0 + 2 * j + h, chunks - 1);
+                    const uint32_t o = vrow[nt] + (uint32_t)(c >> 1) * kV2Block + (uint32_t)(c & 1) * 16u;
+                    const uint32_t *p = reinterpret_cast<const uint32_t *>(wp[nt] + (o & ~3u));
+#pragma unroll
+                    for (int d = 0; d < 5; ++d) st.q[nt][j][d] = p[d];
+                } else {
+                    const int c = min(g0 + 2 * j + h, chunks - 1);
+                    const u32x4 v = *reinterpret_cast<const u32x4 *>(wp[nt] + 16 * (size_t)c);
+                    st.q[nt][j][0] = v.x; st.q[nt][j][1] = v.y; st.q[nt][j][2] = v.z; st.q[nt][j][3] = v.w;
+                }
+            }
+            if constexpr (FMT == Q_V2) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int b = min((g0 >> 1) + j, (chunks >> 1) - 1);
+                    st.s[nt][j] = __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t *>(
+                        wp[nt] + vrow[nt] + (uint32_t)b * kV2Block + 32u));
+                }
+            } else if constexpr (SM == 0) {
+                if (g0 + 3 < chunks) {
+                    const f32x4u v = *reinterpret_cast<const f32x4u *>(sp[nt] + g0);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) st.s[nt][t] = v[t];
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        st.s[nt][t] = g0 + t < chunks ? sp[nt][g0 + t] : 0.f;
+                }
+            } else if constexpr (SM == 1) {
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    st.s[nt][t] = g0 + 2 * t < chunks ? sp[nt][(32 * (g0 + 2 * t)) >> a.gshift] : 0.f;
+            }
+        }
+    }
+
+    // The two B operands (steps u = 0, 1) of group g of the stage.
+    __device__ __forceinline__ void expand(const Stage &st, int nt, int g, int g0, h8 (&B)[2]) const {
+        if constexpr (FMT == Q_W8) {
+            const uint32_t *q = st.q[nt][g];
+            B[0] = expand_w8(q[0], q[1]);
+            B[1] = expand_w8(q[2], q[3]);
+        } else {
+            const int j = g >> 1;
+            uint32_t d[4];
+            if constexpr (FMT == Q_V2) {
+                const int c = min(g0 + 2 * j + h, chunks - 1);
+                const uint32_t o = vrow[nt] + (uint32_t)(c >> 1) * kV2Block;
+                const uint32_t sh = (o & 2u) * 8u;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    d[t] = __builtin_amdgcn_alignbit(st.q[nt][j][t + 1], st.q[nt][j][t], sh);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) d[t] = st.q[nt][j][t];
+            }
+            const auto s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
+            const auto s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
+            B[0] = expand_w4((g & 1) ? s0[1] : s0[0]);
+            B[1] = expand_w4((g & 1) ? s1[1] : s1[0]);
+        }
+    }
+
+    __device__ __forceinline__ float scale(const Stage &st, int nt, int g) const {
+        if (SM == 0) return st.s[nt][g & 3];
+        if (FMT == Q_V2) return f16_bits_to_f32(__float_as_uint(st.s[nt][g >> 1]));
+        return SM == 1 ? st.s[nt][g >> 1] : 1.0f;
+    }
+
+    // One stage: acc += scale * chain, a chain per 32 K.
+    __device__ __forceinline__ void compute(const uint8_t *lds, int g0, const Stage &st,
+                                            f32x16 (&acc)[MT][NT]) const {
+#pragma unroll
+        for (int g = 0; g < SG; ++g) {
+            h8 B[NT][2];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) expand(st, nt, g, g0, B[nt]);
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                h8 A[2][2];   // [step][limb]
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int l = 0; l < 2; ++l)
+                        A[u][l] = *reinterpret_cast<const h8 *>(
+                            lds + (mt * SG + g) * kGroupBytes + (2 * u + l) * 1024 + lane * 16);
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    f32x16 D = {};
+#pragma unroll
+                    for (int l = 1; l >= 0; --l)
+#pragma unroll
+                        for (int u = 0; u < 2; ++u)
+                            D = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[u][l], B[nt][u], D, 0, 0, 0);
+                    if constexpr (SM == 2) {
+                        acc[mt][nt] += D;
+                    } else {
+                        const float s = scale(st, nt, g);
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) acc[mt][nt][r] = fmaf(D[r], s, acc[mt][nt][r]);
+                    }
+                }
+            }
+        }
+    }
+};
+
+template <int FMT, int MT, int NT, int SM, bool PAIR>
+__global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
+    using T = QTile<FMT, MT, NT, SM, PAIR>;
+    constexpr int SG = T::SG;
+    constexpr int kStage = MT * SG * kGroupBytes;
+    static_assert(!PAIR || NT == 2, "a pair's column tiles are gate and up");
+    __shared__ __align__(16) uint8_t lds0[kStage];
+    __shared__ __align__(16) uint8_t lds1[kStage];
+    // Consecutive tiles (row blocks of the same columns first) on one XCD:
+    // blocks go to the 8 XCDs round robin.
+    const int per = gridDim.x >> 3;
+    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    if (tile >= a.mz * a.nbx * a.splits) return;
+    const int mz = tile % a.mz, rest = tile / a.mz;
+    const int bx = rest % a.nbx, split = rest / a.nbx;
+    const int gb = split * a.slen, ge = min(gb + a.slen, a.groups);
+
+    T t(a);
+    t.rows(bx);
+    const int slab0 = mz * MT;
+
+    auto stage_x = [&](uint8_t *lds, int g0) {
+        constexpr int kChunks = MT * SG * 4;   // KiB pieces of a stage
+#pragma unroll
+        for (int c0 = 0; c0 < kChunks; c0 += 4) {
+            const int c = c0 + t.wave, mt = c / (SG * 4), o = c - mt * (SG * 4);
+            const int slab = min(slab0 + mt, a.slabs - 1);   // slabs past the last are not stored
+            const uint8_t *src = a.rec + ((size_t)slab * a.groups + g0) * kGroupBytes + o * 1024 +
+                                 t.lane * 16;
+            __builtin_amdgcn_global_load_lds(src, lds + c * 1024, 16, 0, 0);
+        }
+    };
+    auto landed = [&] {   // this wave's copies landed, then everybody's
+        __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));   // vmcnt(0)
+        __syncthreads();
+    };
+
+    f32x16 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.f;
+
+    typename T::Stage sa, sb;
+    stage_x(lds0, gb);
+    t.load(gb, sa);
+    landed();
+    for (int g = gb; g < ge; g += 2 * SG) {
+        if (g + SG < ge) {
+            stage_x(lds1, g + SG);
+            t.load(g + SG, sb);
+        }
+        t.compute(lds0, g, sa, acc);
+        landed();
+        if (g + SG >= ge) break;
+        if (g + 2 * SG < ge) {
+            stage_x(lds0, g + 2 * SG);
+            t.load(g + 2 * SG, sa);
+        }
+        t.compute(lds1, g + SG, sb, acc);
+        landed();
+    }
+
+    // Register r of lane (i, h) is row 8 (r / 4) + 4 h + r % 4 of weight row i.
+    const bool split_k = a.splits > 1;
+    const size_t plane = (size_t)a.m * a.n;
+    float *y = a.y + (split_k ? (size_t)split * (PAIR ? 2 : 1) * plane : 0);
+    const float *inv = a.inv + (size_t)split * a.slabs * kSlab;
+    auto row_scale = [&](const float *s, int len, int c) {
+        return SM == 2 ? s[len > 1 ? c : 0] : 1.0f;
+    };
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int slab = slab0 + mt;
+        if (slab >= a.slabs) break;
+        f32x4 f[4];
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+            f[r4] = *reinterpret_cast<const f32x4 *>(inv + slab * kSlab + 8 * r4 + 4 * t.h);
+#pragma unroll
+        for (int nt = 0; nt < (PAIR ? 1 : NT); ++nt) {
+            const int c = t.col(bx, nt);
+            if (c >= a.n) continue;
+            const float rs0 = row_scale(a.s0, a.s0_len, c);
+            const float rs1 = PAIR ? row_scale(a.s1, a.s1_len, c) : 1.0f;
+            const float b0 = !split_k && a.b0 ? a.b0[c] : 0.f;
+            const float b1 = PAIR && !split_k && a.b1 ? a.b1[c] : 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = slab * kSlab + 8 * (r >> 2) + 4 * t.h + (r & 3);
+                if (row >= a.m) continue;
+                const size_t o = (size_t)row * a.n + c;
+                const float fr = f[r >> 2][r & 3];
+                const float g = acc[mt][nt][r] * fr * rs0;
+                if constexpr (PAIR) {
+                    const float u = acc[mt][NT - 1][r] * fr * rs1;
+                    if (split_k) {
+                        y[o] = g;
+                        y[plane + o] = u;
+                    } else {
+                        y[o] = silu(g + b0) * (u + b1);
+                    }
+                } else {
+                    float v = g;
+                    if (!split_k) {
+                        if (a.b0) v += b0;
+                        if (a.res) v += a.res[o];
+                    }
+                    y[o] = v;
+                }
+            }
+        }
+    }
+}
+
+// The limbs of x [m, k] for one K split of 8 rows: slab s, group g at
+// rec + (s groups + g) 4096, then [step][limb][lane (i, h)][8 slots].  A thread
+// takes pieces of 8 elements of row t % 8; rows past m and K past k are 0.
+// W4: slots in nibble order, the ones that meet 16 x weights divided by 16.
+template <bool W4>
+__global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
+                                                 uint8_t *__restrict__ rec,
+                                                 float *__restrict__ inv, int m, int k, int slabs,
+                                                 int groups, int slen) {
+    constexpr int PC = 4;   // pieces kept in registers
+    __shared__ float red[16][8];
+    const int t = threadIdx.x, tpr = blockDim.x >> 3;
+    const int row = blockIdx.x * 8 + (t & 7), split = blockIdx.y;
+    const int k0 = split * slen * 32, k1 = min(k0 + slen * 32, groups * 32);
+    const int pieces = (k1 - k0) >> 3;
+    const float *xr = x + (size_t)row * k;
+    auto fetch = [&](int p, f32x4 &a, f32x4 &b) {
+        const int kk = k0 + 8 * p;
+        a = b = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (row < m && kk < k) {
+            a = *reinterpret_cast<const f32x4 *>(xr + kk);
+            b = *reinterpret_cast<const f32x4 *>(xr + kk + 4);
+        }
+    };
+    float mx = 0.f;
+    auto see = [&](const f32x4 &a, const f32x4 &b) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float u = fabsf(a[e]), v = fabsf(b[e]);
+            mx = fmaxf(mx, u < INFINITY ? u : 0.f);
+            mx = fmaxf(mx, v < INFINITY ? v : 0.f);
+        }
+    };
+    f32x4 ra[PC], rb[PC];
+#pragma unroll
+    for (int c = 0; c < PC; ++c) {
+        const int p = (t >> 3) + c * tpr;
+        ra[c] = rb[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (p < pieces) fetch(p, ra[c], rb[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < PC; ++c) see(ra[c], rb[c]);
+    for (int p = (t >> 3) + PC * tpr; p < pieces; p += tpr) {
+        f32x4 a, b;
+        fetch(p, a, b);
+        see(a, b);
+    }
+#pragma unroll
+    for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((t & 63) < 8) red[t >> 6][t & 7] = mx;
+    __syncthreads();
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t & 7]);
+    int E = 0;
+    (void)frexpf(mx, &E);   // mx = f 2^E, f in [0.5, 1)
+    const int e = mx > 0.f ? min(15 - E, 126) : 0;
+    const float up = ldexpf(1.f, e);
+    if (t < 8) inv[(size_t)split * slabs * kSlab + row] = ldexpf(1.f, -e);
+    auto put = [&](int p, const f32x4 &a, const f32x4 &b) {
+        const int kk = k0 + 8 * p, g = kk >> 5, q = (kk >> 3) & 3;
+        h8 l1, l2;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int el = W4 ? slot_elem(j) : j;
+            const float v = el < 4 ? a[el & 3] : b[el & 3];
+            const float s = v * ((W4 && (j & 2)) ? up * 0.0625f : up);
+            const _Float16 u = (_Float16)s;
+            const float r = s - (float)u;
+            l1[j] = u;
+            l2[j] = fabsf(s) < INFINITY ? (_Float16)r : (_Float16)0.f;
+        }
+        uint8_t *d = rec + ((size_t)(row >> 5) * groups + g) * kGroupBytes +
+                     (size_t)(q & 1) * 2048 + (size_t)((q >> 1) * 32 + (row & 31)) * 16;
+        *reinterpret_cast<h8 *>(d) = l1;
+        *reinterpret_cast<h8 *>(d + 1024) = l2;
+    };
+#pragma unroll
+    for (int c = 0; c < PC; ++c) {
+        const int p = (t >> 3) + c * tpr;
+        if (p < pieces) put(p, ra[c], rb[c]);
+    }
+    for (int p = (t >> 3) + PC * tpr; p < pieces; p += tpr) {
+        f32x4 a, b;
+        fetch(p, a, b);
+        put(p, a, b);
+    }
+}
+
+// Sum of the split-K partials in split order, then the epilogue.  res may be y
+// (each element is read before the same thread writes it).
+template <bool PAIR, int VEC>
+__global__ __launch_bounds__(256) void k_qreduce(const float *__restrict__ part, int splits,
+                                                 int m, int n, const float *__restrict__ b0,
+                                                 const float *__restrict__ b1, const float *res,
+                                                 float *y) {
+    typedef float vec __attribute__((ext_vector_type(VEC)));
+    const size_t plane = (size_t)m * n, total = plane / VEC;
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
+         e += (size_t)gridDim.x * blockDim.x) {
+        const size_t o = e * VEC;
+        const int c = (int)(o % (size_t)n);
+        vec g = {}, u = {}, r = {}, bg = {}, bu = {};
+        if (res) r = *reinterpret_cast<const vec *>(res + o);
+        if (b0) bg = *reinterpret_cast<const vec *>(b0 + c);
+        if (PAIR && b1) bu = *reinterpret_cast<const vec *>(b1 + c);
+#pragma unroll 4
+        for (int s = 0; s < splits; ++s) {
+            g += *reinterpret_cast<const vec *>(part + (size_t)s * (PAIR ? 2 : 1) * plane + o);
+            if (PAIR) u += *reinterpret_cast<const vec *>(part + (size_t)(2 * s + 1) * plane + o);
+        }
+        vec v;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            if (PAIR) {
+                v[j] = silu(g[j] + bg[j]) * (u[j] + bu[j]);
+            } else {
+                float w = g[j];
+                if (b0) w += bg[j];
+                if (res) w += r[j];
+                v[j] = w;
+            }
+        }
+        *reinterpret_cast<vec *>(y + o) = v;
+    }
+}
+
+constexpr int kCUs = 256;
+constexpr int kMaxSplits = 16;
+
+struct Plan {
+    int mt, nt, mz, nbx, splits, slen, slabs, groups;
+};
+
+size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+size_t rec_bytes(const Plan &pl) { return (size_t)pl.slabs * pl.groups * kGroupBytes; }
+size_t inv_bytes(const Plan &pl, int splits) {
+    return up256((size_t)splits * pl.slabs * kSlab * sizeof(float));
+}
+size_t scratch_of(const Plan &pl, int splits, int m, int n, bool pair) {
+    return rec_bytes(pl) + inv_bytes(pl, splits) +
+           (splits > 1 ? (size_t)splits * (pair ? 2 : 1) * (size_t)m * n * sizeof(float) : 0);
+}
+
+// Tile and K split by a small cost model, in us, fitted to sweeps of (MT, NT,
+// splits) at M = 17..512 and N, K = 900..14336, which it meets within about 10%:
+//   * a CU finishes one 128-K stage of a block in 0.56 MT NT when other blocks
+//     hide its waits, and a block alone takes 0.9 + 0.45 MT NT (INT8 a third
+//     more: twice the weight bytes per stage);
+//   * K splits cost the reduce kernel and the partials' way through memory.
+// splits == 0 in the result: no plan fits the scratch.
+Plan plan(int m, int n, int k, int fmt, bool pair, size_t cap) {
+    Plan pl{};
+    pl.slabs = (m + kSlab - 1) / kSlab;
+    pl.groups = (k + kPad - 1) / kPad * (kPad / 32);
+    const int stages = pl.groups / 4;
+    double best = 1e30;
+    for (int mt = 1; mt <= (pl.slabs > 1 ? 2 : 1); ++mt)
+        for (int nt = pair ? 2 : 1; nt <= 2; ++nt) {
+            const int mz = (pl.slabs + mt - 1) / mt;
+            const int nbx = pair ? (n + 127) / 128 : (n + 128 * nt - 1) / (128 * nt);
+            const double busy = 0.56 * mt * nt;
+            const double alone = (0.9 + 0.45 * mt * nt) * (fmt == Q_W8 ? 1.35 : 1.0);
+            for (int s = 1; s <= stages && s <= kMaxSplits; ++s) {
+                const int len = (stages + s - 1) / s;
+                if ((stages + len - 1) / len != s) continue;
+                const long per_cu = ((long)mz * nbx * s + kCUs - 1) / kCUs;
+                double t = len * std::max((double)per_cu * busy, alone);
+                if (s > 1) t += 3.0 + (double)(pair ? 2 : 1) * s * m * n * (8.0 / 5e6);
+                if (t < best && scratch_of(pl, s, m, n, pair) <= cap) {
+                    best = t;
+                    pl.mt = mt; pl.nt = nt; pl.mz = mz; pl.nbx = nbx;
+                    pl.splits = s; pl.slen = len * 4;
+                }
+            }
+        }
+    return pl;
+}
+
+template <int FMT, int SM>
+int launch(const QArgs &a, const Plan &pl, bool pair, hipStream_t st) {
+    const long tiles = (long)pl.mz * pl.nbx * pl.splits;
+    const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
+    if (pair) {
+        if (pl.mt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 1, 2, SM, true>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_qgemm<FMT, 2, 2, SM, true>), grid, block, 0, st, a);
+    } else {
+        if (pl.nt == 1 && pl.mt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 1, 1, SM, false>), grid, block, 0, st, a);
+        else if (pl.nt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 2, 1, SM, false>), grid, block, 0, st, a);
+        else if (pl.mt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 1, 2, SM, false>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k_qgemm<FMT, 2, 2, SM, false>), grid, block, 0, st, a);
+    }
+    TB_LAUNCHED();
+    return TB_OK;
+}
+
+}  // namespace
+
+bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt) {
+    if (m < 1 || n < 1 || k < 32 || k % (fmt == Q_V2 ? 64 : 32) != 0) return false;
+    return k <= (int64_t)1 << 24 && m < (int64_t)1 << 24 && n < (int64_t)1 << 30;
+}
+
+size_t qgemm_scratch_bytes(int m, int n, int k, int fmt, bool pair) {
+    const Plan pl = plan(m, n, k, fmt, pair, SIZE_MAX);
+    return scratch_of(pl, pl.splits, m, n, pair);
+}
+
+bool qgemm_fits(int64_t m, int64_t n, int64_t k, int fmt, bool pair, size_t cap) {
+    return qgemm_shape_ok(m, n, k, fmt) &&
+           plan((int)m, (int)n, (int)k, fmt, pair, cap).splits > 0;
+}
+
+int qgemm(const QGemmParams &p, void *scratch, size_t cap, hipStream_t st) {
+    const bool pair = p.w1 != nullptr;
+    TB_REQUIRE(qgemm_shape_ok(p.m, p.n, p.k, p.fmt), TB_ERR_UNSUPPORTED,
+               "TB_UNSUPPORTED: batched projection needs K % 32 == 0");
+    const Plan pl = plan(p.m, p.n, p.k, p.fmt, pair, cap);
+    TB_REQUIRE(pl.splits > 0, TB_ERR_UNSUPPORTED,
+               "TB_UNSUPPORTED: batched projection: scratch too small");
+    uint8_t *rec = static_cast<uint8_t *>(scratch);
+    float *inv = reinterpret_cast<float *>(rec + rec_bytes(pl));
+    float *part = reinterpret_cast<float *>(rec + rec_bytes(pl) + inv_bytes(pl, pl.splits));
+    const dim3 pg((unsigned)(pl.slabs * 4), (unsigned)pl.splits);
+    const unsigned threads = pl.slen * 32 <= 1024 ? 256 : pl.slen * 32 <= 2048 ? 512 : 1024;
+    if (p.fmt == Q_W8)
+        hipLaunchKernelGGL((k_qsplit<false>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m, p.k,
+                           pl.slabs, pl.groups, pl.slen);
+    else
+        hipLaunchKernelGGL((k_qsplit<true>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m, p.k,
+                           pl.slabs, pl.groups, pl.slen);
+    TB_LAUNCHED();
+    QArgs a{};
+    a.rec = rec; a.inv = inv;
+    a.w0 = static_cast<const uint8_t *>(p.w0);
+    a.w1 = static_cast<const uint8_t *>(p.w1);
+    a.s0 = p.s0; a.s1 = p.s1; a.b0 = p.b0; a.b1 = p.b1; a.res = p.res;
+    a.y = pl.splits > 1 ? part : p.y;
+    a.m = p.m; a.n = p.n; a.k = p.k;
+    a.scols = p.grouped ? p.k >> p.gshift : 0;
+    a.gshift = p.gshift; a.s0_len = p.s0_len; a.s1_len = p.s1_len;
+    a.slabs = pl.slabs; a.groups = pl.groups;
+    a.mz = pl.mz; a.nbx = pl.nbx; a.splits = pl.splits; a.slen = pl.slen;
+    int rc;
+    if (p.fmt == Q_W8) rc = launch<Q_W8, 2>(a, pl, pair, st);
+    else if (p.fmt == Q_V2) rc = launch<Q_V2, 1>(a, pl, pair, st);
+    else if (!p.grouped) rc = launch<Q_W4, 2>(a, pl, pair, st);
+    else if (p.gshift == 5) rc = launch<Q_W4, 0>(a, pl, pair, st);
+    else rc = launch<Q_W4, 1>(a, pl, pair, st);
+    if (rc || pl.splits == 1) return rc;
+    const size_t total = (size_t)p.m * p.n;
+    const bool v4 = p.n % 4 == 0 && !(((uintptr_t)p.y | (uintptr_t)p.b0 | (uintptr_t)p.b1 |
+                                       (uintptr_t)p.res) & 15);
+    const unsigned rb = (unsigned)std::min<size_t>((total / (v4 ? 4 : 1) + 255) / 256, 4096);
+#define TB_QRED(PAIR_, VEC_)                                                                     \
+    hipLaunchKernelGGL((k_qreduce<PAIR_, VEC_>), dim3(rb), dim3(256), 0, st, part, pl.splits,    \
+                       p.m, p.n, p.b0, p.b1, p.res, p.y)
+    if (pair) {
+        if (v4) TB_QRED(true, 4);
+        else TB_QRED(true, 1);
+    } else {
+        if (v4) TB_QRED(false, 4);
+        else TB_QRED(false, 1);
+    }
+#undef TB_QRED
+    TB_LAUNCHED();
+    return TB_OK;
+}
+
+}  // namespace tb

@@ -1,22 +1,23 @@
-// Batched grouped-INT4 projection Y[M, N] = X[M, K] . deq(W)^T on FP32 MFMA
-// (v_mfma_f32_16x16x4_f32), for batches of M >= 5 rows (16-row tiles), where
-// the work is a dense contraction.
+// Grouped-INT4 projection Y[M, N] = X[M, K] . deq(W)^T on FP32 MFMA
+// (v_mfma_f32_16x16x4_f32) for 5 to 16 activation rows, where the weights'
+// stream and not the contraction sets the time; from 17 rows the calls go on to
+// the f16-limb kernel (qgemm.hip).
 //
 // Replaces the M > 1 path of the reference's w4a32_grouped_linear
 // (src/quantization/packed_v2.rs:557-624 -> gemm_w4a32_grouped,
 // src/quantization/gemv.rs:1690-1725), which runs one full GEMV per activation
-// row and so reads the weights M times; here every weight byte is read once per
-// 64 activation rows.  The batched SwiGLU of fused_swiglu_mlp_batched_w4a32
-// (src/quantization/fused_ops.rs:1267-1319: gate GEMM, up GEMM, silu * up,
-// down GEMM) maps onto the dual launch plus the SwiGLU reduce epilogue.
+// row and so reads the weights M times.  The batched SwiGLU of
+// fused_swiglu_mlp_batched_w4a32 (src/quantization/fused_ops.rs:1267-1319:
+// gate GEMM, up GEMM, silu * up, down GEMM) maps onto the dual launch plus the
+// SwiGLU reduce epilogue.
 //
-// Tiling.  A block (4 waves) owns 64 weight rows (16 per wave) x up to 64
-// activation rows (MT tiles of 16) x a K range of `klen` (split-K over blocks,
-// partial sums reduced by k_mfma_reduce in a fixed order, so results are
-// deterministic).  Per 128-wide K step:
-//   * X [16*MT, 128] is staged once per block in LDS (row pitch 132 floats,
-//     so the 16 rows of an MFMA operand read fall on distinct banks) and read
-//     by all four waves;
+// Tiling.  A block (4 waves) owns 64 weight rows (16 per wave) x 16 activation
+// rows x a K range of `klen` (split-K over blocks, partial sums reduced by
+// k_mfma_reduce in a fixed order, so results are deterministic).  Per 128-wide
+// K step:
+//   * X [16, 128] is staged once per block in LDS (row pitch 132 floats, so the
+//     16 rows of an MFMA operand read fall on distinct banks) and read by all
+//     four waves;
 //   * each lane loads one 16-byte chunk of its weight row (32 nibbles = one
 //     group at g32, half of one at g64) plus the group scale, and dequantizes
 //     it in registers straight into the MFMA B operand: (nib - 8) * s as
@@ -30,18 +31,18 @@
 //   * the next step's X tile, weight chunk and scale are loaded into registers
 //     before the current step's MFMAs are issued; X tiles alternate between two
 //     LDS buffers, so each step needs one barrier;
-//   * up to four independent accumulators per 16-row tile keep dependent MFMAs
-//     apart (small M has few tiles to interleave).
+//   * four independent accumulators keep dependent MFMAs apart.
 //   * V2: weights in the v2 stream (34-byte group-64 blocks with f16 scales,
 //     packed_v2.rs:26-143): a lane's 16-byte chunk is one half of a block,
 //     read with dword-aligned loads and a funnel shift (load_v2_chunk).
-#include <float.h>
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "gemv_common.hpp"
+#include "qgemm.hpp"
 #include "tb_common.hpp"
 #include "w4_gemv.hpp"
-#include "w4_limb.hpp"
 #include "w4_mfma.hpp"
 
 namespace tb {
@@ -57,7 +58,7 @@ constexpr int kTargetBlocks = 512;   // split-K target (TB_MFMA_BLOCKS overrides
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-template <int MT, bool V2>
+template <bool V2>
 __global__ __launch_bounds__(256) void k_w4_mfma(const float *__restrict__ x,
                                                  const uint8_t *__restrict__ w0,
                                                  const float *__restrict__ s0,
@@ -66,17 +67,16 @@ __global__ __launch_bounds__(256) void k_w4_mfma(const float *__restrict__ x,
                                                  float *__restrict__ part, int m, int n, int k,
                                                  int scols, int gshift, int klen, int nbx,
                                                  int splits) {
-    constexpr int XV = MT * 2;             // float4 of the X tile per thread
-    constexpr int NACC = MT <= 2 ? 4 : 2;  // independent accumulation chains per M tile
-    constexpr int NB = MT <= 2 ? 2 : 1;    // X tile buffers (two cost occupancy at MT >= 3)
-    __shared__ float xs[NB][MT * 16 * kXP];
+    constexpr int XV = 2;     // float4 of the X tile per thread
+    constexpr int NACC = 4;   // independent accumulation chains
+    __shared__ float xs[2][16 * kXP];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int bx = blockIdx.x;
     const int second = bx >= nbx ? 1 : 0;   // dual launch: blocks of the up projection
     bx -= second * nbx;
     const uint8_t *w = second ? w1 : w0;
     const float *s = second ? s1 : s0;
-    const int m0 = blockIdx.z * MT * 16;
+    const int m0 = blockIdx.z * 16;
     const int kb = blockIdx.y * klen;
     const int ke = min(k, kb + klen);
     const int row = bx * kBN + wave * 16 + (lane & 15);
@@ -114,19 +114,15 @@ __global__ __launch_bounds__(256) void k_w4_mfma(const float *__restrict__ x,
         }
     };
 
-    f32x4 acc[MT][NACC];
+    f32x4 acc[NACC];
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-        for (int c = 0; c < NACC; ++c) acc[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < NACC; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     load_step(kb);
     int buf = 0;
-    for (int k0 = kb; k0 < ke; k0 += kBK, buf ^= (NB - 1)) {
+    for (int k0 = kb; k0 < ke; k0 += kBK, buf ^= 1) {
+        // `buf` was last read two steps ago, before the previous step's barrier
         float *xb = xs[buf];
-        // With two buffers, `buf` was last read two steps ago, before the
-        // previous step's barrier; with one, wait for this step's readers.
-        if (NB == 1) __syncthreads();
 #pragma unroll
         for (int i = 0; i < XV; ++i) {
             const int f = tid + 256 * i;
@@ -140,15 +136,10 @@ __global__ __launch_bounds__(256) void k_w4_mfma(const float *__restrict__ x,
         const uint32_t dws[4] = {cw.x, cw.y, cw.z, cw.w};
 #pragma unroll
         for (int d = 0; d < 4; ++d) {
-            float a[MT][8];
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                const float *xa = xb + (t * 16 + (lane & 15)) * kXP + 32 * q + 8 * d;
-                const float4 a0 = *reinterpret_cast<const float4 *>(xa);
-                const float4 a1 = *reinterpret_cast<const float4 *>(xa + 4);
-                a[t][0] = a0.x; a[t][1] = a0.y; a[t][2] = a0.z; a[t][3] = a0.w;
-                a[t][4] = a1.x; a[t][5] = a1.y; a[t][6] = a1.z; a[t][7] = a1.w;
-            }
+            const float *xa = xb + (lane & 15) * kXP + 32 * q + 8 * d;
+            const float4 a0 = *reinterpret_cast<const float4 *>(xa);
+            const float4 a1 = *reinterpret_cast<const float4 *>(xa + 4);
+            const float a[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
             const uint32_t lo = dws[d] & 0x0F0F0F0Fu, hi = (dws[d] >> 4) & 0x0F0F0F0Fu;
             float b[8];
 #pragma unroll
@@ -158,26 +149,21 @@ __global__ __launch_bounds__(256) void k_w4_mfma(const float *__restrict__ x,
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    acc[t][e % NACC] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        a[t][e], b[e], acc[t][e % NACC], 0, 0, 0);
+                acc[e % NACC] =
+                    __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], acc[e % NACC], 0, 0, 0);
         }
     }
 
     const int col = bx * kBN + wave * 16 + (lane & 15);
     if (col >= n) return;
     float *pb = part + (size_t)(second * splits + blockIdx.y) * (size_t)m * n;
+    f32x4 v = acc[0];
 #pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        f32x4 v = acc[t][0];
+    for (int c = 1; c < NACC; ++c) v += acc[c];
 #pragma unroll
-        for (int c = 1; c < NACC; ++c) v += acc[t][c];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int mr = m0 + t * 16 + 4 * q + r;
-            if (mr < m) pb[(size_t)mr * n + col] = v[r];
-        }
+    for (int r = 0; r < 4; ++r) {
+        const int mr = m0 + 4 * q + r;
+        if (mr < m) pb[(size_t)mr * n + col] = v[r];
     }
 }
 
@@ -208,7 +194,7 @@ __global__ __launch_bounds__(256) void k_mfma_reduce(const float *__restrict__ p
 }
 
 struct Plan {
-    int mt, mz, nbx, klen, splits;
+    int mz, nbx, klen, splits;
 };
 
 int target_blocks() {
@@ -222,9 +208,7 @@ int target_blocks() {
 
 Plan plan(int m, int n, int k, bool dual) {
     Plan pl;
-    const int tiles = (m + 15) / 16;
-    pl.mt = tiles < 4 ? tiles : 4;
-    pl.mz = (tiles + pl.mt - 1) / pl.mt;
+    pl.mz = (m + 15) / 16;
     pl.nbx = (n + kBN - 1) / kBN;
     const int blocks = pl.nbx * (dual ? 2 : 1) * pl.mz;
     const int steps = (k + kBK - 1) / kBK;
@@ -237,17 +221,14 @@ Plan plan(int m, int n, int k, bool dual) {
     return pl;
 }
 
-// From 17 rows the projection runs on the exact f16 limbs of x (k_w4_lgemm,
-// w4_limb.hip) when K is whole 128-element batches and a 32-element group has
-// one scale (16-row projections measured 14.7 against 14.4 us on FP32 MFMA);
-// TB_MFMA_LIMB=0 keeps the FP32-MFMA kernel (measurement only).
-bool use_limbs(int m, int k, bool v2, int scale_mode, int gshift) {
-    static const bool on = [] {
-        const char *e = getenv("TB_MFMA_LIMB");
-        return !(e && e[0] == '0');
-    }();
-    return on && m >= 17 && !v2 && k % kBK == 0 && (scale_mode != 0 || gshift >= 5);
-}
+// From 17 rows the projection runs on the f16-limb kernel: at 17 rows, N = K =
+// 4096 the two take 17 and 15 us, from there this kernel's second 16-row tile
+// doubles its contraction (64 rows, N = 14336: 81 against 36 us); at 16 rows
+// and K = N = 4096 both take 14.4 us and below that this one is ahead (no
+// kernel that prepares the activations).
+constexpr int kQGemmMinM = 17;
+
+int qfmt(int v2) { return v2 ? Q_V2 : Q_W4; }
 
 size_t partials_only(int m, int n, int k, bool dual) {
     const Plan pl = plan(m, n, k, dual);
@@ -256,13 +237,18 @@ size_t partials_only(int m, int n, int k, bool dual) {
 
 }  // namespace
 
-size_t w4_mfma_partials_bytes(int m, int n, int k, bool dual) {
-    // partials, then (256-byte aligned) room for the limb records of x
-    const size_t pb = (partials_only(m, n, k, dual) + 255) & ~(size_t)255;
-    return pb + (m >= 17 && k % kBK == 0 ? lgemm_records_bytes(m, k) : 0);
+size_t w4_mfma_scratch_bytes(int m, int n, int k, bool dual, bool v2) {
+    if (m >= kQGemmMinM && qgemm_shape_ok(m, n, k, qfmt(v2)))
+        return qgemm_scratch_bytes(m, n, k, qfmt(v2), dual);
+    return partials_only(m, n, k, dual);
 }
 
-int w4_mfma(const MfmaParams &p, int epi, float *part, hipStream_t st) {
+size_t w4_mfma_scratch_upto(int m, int n, int k, bool dual) {
+    return std::max(w4_mfma_scratch_bytes(m, n, k, dual, false),
+                    partials_only(std::min(m, kQGemmMinM - 1), n, k, dual));
+}
+
+int w4_mfma(const MfmaParams &p, int epi, float *part, size_t cap, hipStream_t st) {
     const bool dual = p.w1 != nullptr;
     TB_REQUIRE(p.k % 32 == 0 && p.m >= 1 && p.n >= 1, TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: MFMA projection needs K % 32 == 0");
@@ -273,44 +259,31 @@ int w4_mfma(const MfmaParams &p, int epi, float *part, hipStream_t st) {
                    TB_ERR_UNSUPPORTED,
                    "TB_UNSUPPORTED: v2 blocks need K % 64 == 0, a 4-byte aligned stream "
                    "under 4 GiB");
+    if (p.m >= kQGemmMinM && qgemm_fits(p.m, p.n, p.k, qfmt(p.v2), dual, cap)) {
+        QGemmParams q{};
+        q.x = p.x; q.w0 = p.w0; q.s0 = p.s0; q.b0 = p.b0;
+        q.w1 = p.w1; q.s1 = p.s1; q.b1 = p.b1;
+        q.res = epi == EPI_RESID ? p.res : nullptr;
+        q.y = p.y; q.m = p.m; q.n = p.n; q.k = p.k;
+        q.fmt = qfmt(p.v2);
+        q.grouped = p.v2 || p.scale_mode == 0;
+        q.gshift = p.gshift;
+        q.s0_len = q.s1_len = p.scale_mode == 1 ? p.n : 1;
+        return qgemm(q, part, cap, st);
+    }
+    TB_REQUIRE(partials_only(p.m, p.n, p.k, dual) <= cap, TB_ERR_UNSUPPORTED,
+               "TB_UNSUPPORTED: MFMA projection: scratch too small");
     const Plan pl = plan(p.m, p.n, p.k, dual);
     dim3 grid(pl.nbx * (dual ? 2 : 1), pl.splits, pl.mz);
     const int scols = p.scale_mode == 0 ? p.k >> p.gshift : (p.scale_mode == 1 ? 1 : 0);
     const int gsh = p.scale_mode == 0 ? p.gshift : 31;
-    if (use_limbs(p.m, p.k, p.v2, p.scale_mode, p.gshift)) {
-        LGemmArgs a;
-        a.x = p.x;
-        a.rec = reinterpret_cast<uint8_t *>(part) +
-                ((partials_only(p.m, p.n, p.k, dual) + 255) & ~(size_t)255);
-        a.w0 = p.w0; a.s0 = p.s0; a.w1 = p.w1; a.s1 = p.s1;
-        a.part = part;
-        a.m = p.m; a.n = p.n; a.k = p.k;
-        a.scols = scols; a.gshift = gsh;
-        a.klen = pl.klen; a.nbx = pl.nbx; a.splits = pl.splits;
-        a.batches = p.k / kBK;
-        a.nslabs = (p.m + 15) / 16;
-        int rc = lgemm_prep(p.x, const_cast<uint8_t *>(a.rec), p.m, p.k, st);
-        if (rc) return rc;
-        if ((rc = lgemm_launch(a, pl.mt, grid, st))) return rc;
-    } else {
-#define TB_MFMA_LAUNCH(MT)                                                                   \
-    if (p.v2)                                                                                \
-        hipLaunchKernelGGL((k_w4_mfma<MT, true>), grid, dim3(256), 0, st, p.x, p.w0, p.s0,   \
-                           p.w1, p.s1, part, p.m, p.n, p.k, scols, gsh, pl.klen, pl.nbx,     \
-                           pl.splits);                                                       \
-    else                                                                                     \
-        hipLaunchKernelGGL((k_w4_mfma<MT, false>), grid, dim3(256), 0, st, p.x, p.w0, p.s0,  \
-                           p.w1, p.s1, part, p.m, p.n, p.k, scols, gsh, pl.klen, pl.nbx,     \
-                           pl.splits)
-    switch (pl.mt) {
-        case 1: TB_MFMA_LAUNCH(1); break;
-        case 2: TB_MFMA_LAUNCH(2); break;
-        case 3: TB_MFMA_LAUNCH(3); break;
-        default: TB_MFMA_LAUNCH(4); break;
-    }
-#undef TB_MFMA_LAUNCH
+    if (p.v2)
+        hipLaunchKernelGGL((k_w4_mfma<true>), grid, dim3(256), 0, st, p.x, p.w0, p.s0, p.w1, p.s1,
+                           part, p.m, p.n, p.k, scols, gsh, pl.klen, pl.nbx, pl.splits);
+    else
+        hipLaunchKernelGGL((k_w4_mfma<false>), grid, dim3(256), 0, st, p.x, p.w0, p.s0, p.w1, p.s1,
+                           part, p.m, p.n, p.k, scols, gsh, pl.klen, pl.nbx, pl.splits);
     TB_LAUNCHED();
-    }
     const size_t total = (size_t)p.m * p.n;
     size_t blocks = (total + 255) / 256;
     if (blocks > 4096) blocks = 4096;

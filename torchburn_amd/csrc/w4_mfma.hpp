@@ -1,4 +1,5 @@
-// Internal launcher of the batched INT4 projection on FP32 MFMA (w4_mfma.hip).
+// Internal launcher of the batched INT4 projection (w4_mfma.hip): FP32 MFMA up
+// to 16 rows, the f16-limb kernel (qgemm.hip) from 17.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -24,13 +25,18 @@ struct MfmaParams {
                          // (f16 scales inside, s0 / s1 unused)
 };
 
-// Bytes of split-K partials w4_mfma needs for this shape (dual = SwiGLU pair).
-size_t w4_mfma_partials_bytes(int m, int n, int k, bool dual);
+// Scratch of the fastest form for this shape (dual = SwiGLU pair).
+size_t w4_mfma_scratch_bytes(int m, int n, int k, bool dual, bool v2 = false);
 
-// y = epilogue(x . deq(w)^T) for any m >= 1 (the MFMA tile is 16 rows; rows
-// beyond m are padding).  epi: EPI_PLAIN, EPI_RESID, or EPI_SWIGLU when w1 is
-// set.  part: device scratch of w4_mfma_partials_bytes().  Shapes validated by
-// the caller (K % 32 == 0, K % group == 0, 16-byte aligned rows).
-int w4_mfma(const MfmaParams &p, int epi, float *part, hipStream_t st);
+// Scratch that serves every row count from 1 to m (v1 weights): below its own
+// fastest plan a call takes one that fits.
+size_t w4_mfma_scratch_upto(int m, int n, int k, bool dual);
+
+// y = epilogue(x . deq(w)^T) for any m >= 1.  epi: EPI_PLAIN, EPI_RESID, or
+// EPI_SWIGLU when w1 is set.  part: cap bytes of device scratch, 256-byte
+// aligned: w4_mfma_scratch_bytes(), or less (fewer K splits, or the FP32-MFMA
+// form where the f16 limbs of x do not fit).  Shapes validated by the caller
+// (K % 32 == 0, K % group == 0, 16-byte aligned rows).
+int w4_mfma(const MfmaParams &p, int epi, float *part, size_t cap, hipStream_t st);
 
 }  // namespace tb

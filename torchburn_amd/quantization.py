@@ -405,8 +405,8 @@ def fused_swiglu_mlp_batched_w4a32(
     """Prefill SwiGLU MLP over x (batch, T, K) -> (batch, T, N_down)
     (reference quantization_ffi.rs:511-570 -> fused_ops.rs:1267-1319: gate GEMM,
     up GEMM, silu(g) * u, down GEMM; one row delegates to the per-token path).
-    Both cases go through tb_fused_swiglu_mlp_w4a32, which runs rows >= 5 as the
-    FP32-MFMA GEMM pair and fewer as GEMV passes."""
+    Both cases go through tb_fused_swiglu_mlp_w4a32, which picks the kernels by
+    the row count."""
     if x.dim() < 1:
         raise UnsupportedOpError(
             f"{_lib.UNSUPPORTED_MARKER} fused_swiglu_mlp_batched_w4a32: x needs >= 1 dim")
@@ -510,8 +510,7 @@ def fused_swiglu_mlp_w8a32(
 def fused_swiglu_mlp_batched(x: torch.Tensor, gate: Any, up: Any, down: Any) -> torch.Tensor:
     """Prefill SwiGLU MLP over three QuantizedLinear modules (reference
     quantization.py:358-405, called at python/torchburn/llm/model.py:359): INT4
-    runs fused_swiglu_mlp_batched_w4a32 (all T rows as one FP32-MFMA GEMM pair
-    from 5 rows), INT8 the per-token fused_swiglu_mlp."""
+    runs fused_swiglu_mlp_batched_w4a32 over all T rows, INT8 fused_swiglu_mlp."""
     if gate.bits != 4:
         return fused_swiglu_mlp(x, gate, up, down)
     return fused_swiglu_mlp_batched_w4a32(
