@@ -1,4 +1,4 @@
-"""The batched f16-limb projection (17 or more rows) at the edges of its tiles:
+"""The batched f16-limb projection (INT4 from 17 rows, INT8 from 3 or 5) at the edges of its tiles:
 rows around 32 and 64, column blocks of 128 and 256, K that is no whole number
 of 128-element stages, K splits, every scale form, and rows of extreme or
 non-finite activations.  Against float64; the bound follows the kernel: two f16
@@ -61,6 +61,43 @@ def test_w4_projection_edges(cuda, m, n, k, gs, v2):
     else:
         y = tb.w4a32_grouped_linear(T(x), T(w), T(s), T(b), group_size=gs)
     check(y.cpu().numpy(), x, deq4(w, s, gs or k), b)
+
+
+@pytest.mark.parametrize("m,n,k,per_row", [
+    (3, 8200, 4096, True),   # 32 Mi weights: from 3 rows
+    (5, 33, 160, True), (32, 129, 992, False), (33, 300, 2080, True), (130, 260, 4160, True),
+    (6, 40, 16416, True)])   # K past the streaming GEMV's range
+def test_w8_projection_edges(cuda, m, n, k, per_row):
+    print(f"case qgemm w8 m={m} n={n} k={k}", flush=True)
+    g = synth.rng(74, m, n, k)
+    x = synth.activations(g, m, k)
+    x[:, 3::37] *= 50.0
+    x[m - 1, 5] = np.inf
+    b = synth.activations(g, n)
+    w, s = synth.int8_weight(g, n, k)
+    w[:, 5] = np.where(w[:, 5] == 0, 1, w[:, 5])   # inf * w has one sign or the other
+    s = s if per_row else s[:1]
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    y = tb.w8a32_linear(T(x), T(w), T(s), T(b))
+    check(y.cpu().numpy(), x, w.astype(np.float64) * s.astype(np.float64)[:, None], b)
+
+
+@pytest.mark.parametrize("m,k,inter", [(5, 96, 160), (40, 992, 1056), (130, 256, 4128)])
+def test_w8_mlp_rows(cuda, m, k, inter):
+    print(f"case qgemm w8 mlp m={m} k={k} inter={inter}", flush=True)
+    g = synth.rng(75, m, k, inter)
+    x, r = synth.activations(g, m, k), synth.activations(g, m, k)
+    wts = [synth.int8_weight(g, n, kk) for n, kk in ((inter, k), (inter, k), (k, inter))]
+    gb, ub, db = (synth.activations(g, n) for n in (inter, inter, k))
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    (gw, gs), (uw, us), (dw, ds) = wts
+    us = us[:1]
+    y = tb.fused_swiglu_mlp_w8a32(T(x), T(gw), T(gs), T(gb), T(uw), T(us), T(ub), T(dw), T(ds),
+                                  T(db), residual=T(r)).cpu().numpy()
+    D = lambda w, s: w.astype(np.float64) * s.astype(np.float64)[:, None]
+    a, u = x.astype(np.float64) @ D(gw, gs).T + gb, x.astype(np.float64) @ D(uw, us).T + ub
+    ref = (a / (1 + np.exp(-a)) * u) @ D(dw, ds).T + db + r
+    assert np.abs(y - ref).max() / np.abs(ref).max() < 2e-6
 
 
 def test_w4_extreme_and_nonfinite_rows(cuda):

@@ -23,6 +23,7 @@
 #include "w4_limb.hpp"
 #include "w4_mfma.hpp"
 #include "v2_layout.hpp"
+#include "qgemm.hpp"
 #include "quantize.hpp"
 #include "sample.hpp"
 
@@ -277,7 +278,8 @@ static int linear_w4(const float *x, const uint8_t *w, const float *s, bool v2,
     const size_t rest = any_shape ? 0
                         : lb ? up256(limb_records_bytes((int)m, (int)k)) +
                                    limb_partials_bytes((int)m, (int)n, (int)k, false)
-                        : mf ? w4_mfma_scratch_bytes((int)m, (int)n, (int)k, false, v2)
+                        : mf ? w4_mfma_scratch_bytes((int)m, (int)n, (int)k, false, v2,
+                                                    v2 || scale_mode == 0)
                              : xq_bytes(m, k);
     const float *xin = x;
     void *tail = nullptr;
@@ -385,6 +387,37 @@ static int generic(const float *x, const void *w0, const float *s0, int mode0, c
     g.res = res; g.y = y; g.m = m; g.n = n; g.k = k; g.group = gs;
     g.scale_mode0 = mode0; g.scale_mode1 = mode1; g.bits = bits;
     return gemv_generic(g, st);
+}
+
+// One INT8 projection, or a SwiGLU pair (p.w1 set), over m rows.  GEMV passes
+// take 2 rows each and re-read the weights; from 5 rows, or 3 on weights of
+// 32 Mi elements, the batched kernel reads them once (us, passes against
+// batched: 4096 x 4096 at 3 rows 12.2 / 13.6 and at 5 17 / 14; 14336 x 4096 at
+// 2 rows 14.0 / 22.7 and at 3 25.4 / 23.5; 4864 x 896 at 4 rows 9.3 / 11.1).
+static bool w8_batched(const DenseParams &p, int64_t m) {
+    const int64_t elems = (int64_t)p.n * p.k * (p.w1 ? 2 : 1);
+    return (m >= 5 || (m >= 3 && elems >= (int64_t)1 << 25)) && aligned(p.x, 16) &&
+           aligned(p.w0, 16) && aligned(p.w1, 16) && qgemm_shape_ok(m, p.n, p.k, Q_W8);
+}
+
+static size_t w8_scratch_bytes(const DenseParams &p, int64_t m) {
+    return w8_batched(p, m) ? qgemm_scratch_bytes((int)m, p.n, p.k, Q_W8, false, p.w1 != nullptr) : 0;
+}
+
+static int w8_rows(const DenseParams &p, int64_t m, void *scratch, size_t cap, hipStream_t st) {
+    if (w8_batched(p, m)) {
+        QGemmParams q{};
+        q.x = p.x; q.w0 = p.w0; q.s0 = p.rs0; q.b0 = p.b0;
+        q.w1 = p.w1; q.s1 = p.rs1; q.b1 = p.b1;
+        q.res = p.res; q.y = p.y; q.m = (int)m; q.n = p.n; q.k = p.k;
+        q.fmt = Q_W8;
+        q.s0_len = p.rs0_len; q.s1_len = p.rs1_len;
+        return qgemm(q, scratch, cap, st);
+    }
+    if (w8_fast(p.x, p.w0, p.k) && aligned(p.w1, 16))
+        return dense_rows(p, W_I8, p.w1 ? EPI_SWIGLU : (p.res ? EPI_RESID : EPI_PLAIN), m, st);
+    return generic(p.x, p.w0, p.rs0, p.rs0_len > 1 ? 1 : 2, p.b0, p.w1, p.rs1,
+                   p.rs1_len > 1 ? 1 : 2, p.b1, p.res, p.y, m, p.n, p.k, 1, 8, st);
 }
 
 // ---- fused SwiGLU MLP (INT4), shared by the workspace and no-alloc entries ----
@@ -975,13 +1008,13 @@ int tb_w8a32_linear(const float *x, const int8_t *w, const float *scales, int64_
     if (rc) return rc;
     TB_REQUIRE(out, TB_ERR_UNSUPPORTED, "TB_UNSUPPORTED: w8a32_linear: null output");
     if (m == 0 || n == 0) return TB_OK;
-    if (!w8_fast(x, w, k))
-        return generic(x, w, scales, s_len > 1 ? 1 : 2, bias, nullptr, nullptr, 0, nullptr,
-                       nullptr, out, m, n, k, 1, 8, (hipStream_t)stream);
     DenseParams p{};
     p.x = x; p.w0 = w; p.rs0 = scales; p.rs0_len = (int)s_len; p.b0 = bias; p.y = out;
     p.m = (int)m; p.n = (int)n; p.k = (int)k;
-    return dense_rows(p, W_I8, EPI_PLAIN, m, (hipStream_t)stream);
+    const size_t bytes = w8_scratch_bytes(p, m);
+    WsLease lease;
+    if (bytes && (rc = workspace(bytes, (hipStream_t)stream, lease))) return rc;
+    return w8_rows(p, m, lease.ptr, bytes, (hipStream_t)stream);
 }
 
 int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float *gate_s,
@@ -1002,29 +1035,26 @@ int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float 
     // down reads h [m, inter] from the workspace (x stands in for its checks)
     rc = check_w8(x, down_w, down_s, down_s_len, m, n_out, inter, "fused_swiglu_mlp_w8a32 down");
     if (rc) return rc;
-    WsLease lease;
-    rc = workspace((size_t)m * (size_t)inter * sizeof(float), (hipStream_t)stream, lease);
-    if (rc) return rc;
-    void *ws = lease.ptr;
-    float *h = static_cast<float *>(ws);
-    hipStream_t st = (hipStream_t)stream;
-    if (!w8_fast(x, gate_w, k) || !aligned(up_w, 16) || !w8_fast(h, down_w, inter)) {
-        rc = generic(x, gate_w, gate_s, gate_s_len > 1 ? 1 : 2, gate_b, up_w, up_s,
-                     up_s_len > 1 ? 1 : 2, up_b, nullptr, h, m, inter, k, 1, 8, st);
-        if (rc) return rc;
-        return generic(h, down_w, down_s, down_s_len > 1 ? 1 : 2, down_b, nullptr, nullptr, 0,
-                       nullptr, residual, out, m, n_out, inter, 1, 8, st);
-    }
     DenseParams p{};
     p.x = x; p.w0 = gate_w; p.rs0 = gate_s; p.rs0_len = (int)gate_s_len; p.b0 = gate_b;
     p.w1 = up_w; p.rs1 = up_s; p.rs1_len = (int)up_s_len; p.b1 = up_b;
-    p.y = h; p.m = (int)m; p.n = (int)inter; p.k = (int)k;
-    rc = dense_rows(p, W_I8, EPI_SWIGLU, m, st);
-    if (rc) return rc;
+    p.m = (int)m; p.n = (int)inter; p.k = (int)k;
     DenseParams d{};
-    d.x = h; d.w0 = down_w; d.rs0 = down_s; d.rs0_len = (int)down_s_len; d.b0 = down_b;
+    d.w0 = down_w; d.rs0 = down_s; d.rs0_len = (int)down_s_len; d.b0 = down_b;
     d.res = residual; d.y = out; d.m = (int)m; d.n = (int)n_out; d.k = (int)inter;
-    return dense_rows(d, W_I8, residual ? EPI_RESID : EPI_PLAIN, m, st);
+    // workspace: h, 16-byte aligned as x must be, then the batched projections'
+    // scratch (d.x is null here: aligned like the h it will be)
+    const size_t hb = up256((size_t)m * (size_t)inter * sizeof(float));
+    const size_t sb = std::max(w8_scratch_bytes(p, m), w8_scratch_bytes(d, m));
+    hipStream_t st = (hipStream_t)stream;
+    WsLease lease;
+    if ((rc = workspace(hb + sb, st, lease))) return rc;
+    float *h = static_cast<float *>(lease.ptr);
+    void *scratch = static_cast<char *>(lease.ptr) + hb;
+    p.y = h;
+    d.x = h;
+    if ((rc = w8_rows(p, m, scratch, sb, st))) return rc;
+    return w8_rows(d, m, scratch, sb, st);
 }
 
 }  // extern "C"

@@ -19,7 +19,10 @@
 // the chain's result takes the group scale and is added in f32, and the row's
 // 2^-e is applied once at the end.
 // Inf and NaN travel through the first limb, as in the reference's
-// unpack-and-fma.
+// unpack-and-fma.  An MFMA step rounds its sum down, which over a long row adds
+// up (a mean error of 1.3e-7 of the results' size at K = 14336): the records
+// hold every other group negated and its chain is subtracted, so that one
+// group's bias cancels another's (negated()).
 //
 // Why two limbs on f16: f32 MFMA runs at 1/16 of the f16 rate, three int8
 // limbs at twice the f16 rate would need an integer-to-float conversion per
@@ -43,10 +46,13 @@
 // -8 of the weights that this one replaced:
 //   Llama-3-8B gate/up pair, 512 rows, group 32    271 us, 444 TFLOP/s (888 in
 //                                                  MFMA work)
-//   Llama-3-8B MLP, 512 rows, group 64             951 -> 504 us
-//   64 rows, N = 14336, K = 4096, group 32         54.6 -> 33.7 us
-// and the error against 64 bits went from 6.2e-7 to 1.5e-7 (activations with
-// large channels; the limbs follow each element's own size).
+//   Llama-3-8B MLP, 512 rows, group 64             949 -> 449 us
+//   64 rows, N = 14336, K = 4096, group 32         54.2 -> 38.8 us
+//   Llama-3-8B MLP in INT8, 128 rows               2562 -> 158 us, against GEMV
+//                                                  passes of 2 rows each
+// The error against 64 bits went from 6.2e-7 to 1.4e-7 for INT4 (activations
+// with large channels: the limbs follow each element's own size) and from
+// 2.3e-7 to 2.1e-7 for the INT8 MLP.
 #include <math.h>
 
 #include <algorithm>
@@ -68,11 +74,16 @@ typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kSlab = 32;            // activation rows of one MFMA tile
 constexpr int kGroupBytes = 4096;    // one slab x 32 K: 2 steps x 2 limbs x 1 KiB
+constexpr int kRun = 512;            // K per level of the row-scale sums
 constexpr int kPad = 128;            // K is padded to whole stages in the records
 
 // K slot e of a step's 8 holds element slot_elem(e): the order in which a dword
 // of nibbles expands; slots with (e & 2) hold 16 x weights.
 __host__ __device__ constexpr int slot_elem(int e) { return (e >> 1) | ((e & 1) << 2); }
+
+// The groups held negated: every other one, starting anew each 4 groups (so
+// that large channels a power of two apart meet both signs).
+__host__ __device__ constexpr bool negated(int g) { return ((g ^ (g >> 2)) & 1) != 0; }
 
 __device__ __forceinline__ h8 expand_w4(uint32_t d) {
     const uint32_t u = d >> 8, o = 0x64006400u;
@@ -232,9 +243,15 @@ struct QTile {
         return SM == 1 ? st.s[nt][g >> 1] : 1.0f;
     }
 
-    // One stage: acc += scale * chain, a chain per 32 K.
+    // One stage, a fresh chain per 32 K.  With group scales acc += scale *
+    // chain; with one scale per row (SM 2) run += chain, and flush() adds run
+    // to acc every kRun elements: two levels of sums keep a long row as exact
+    // as the GEMV's lane tree (INT8, K = 4096, error against 64 bits: 1.3e-7
+    // there; a chain that runs on for 128 K 1.5e-7, for 1024 K 3e-7; two levels
+    // 1.1e-7).
     __device__ __forceinline__ void compute(const uint8_t *lds, int g0, const Stage &st,
-                                            f32x16 (&acc)[MT][NT]) const {
+                                            f32x16 (&acc)[MT][NT], f32x16 (&run)[MT][NT]) const {
+        const float sgn = negated(g0) ? -1.f : 1.f;   // g0 is even: group g's is that of g & 1
 #pragma unroll
         for (int g = 0; g < SG; ++g) {
             h8 B[NT][2];
@@ -257,15 +274,28 @@ struct QTile {
 #pragma unroll
                         for (int u = 0; u < 2; ++u)
                             D = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[u][l], B[nt][u], D, 0, 0, 0);
+                    const float s = (g & 1) ? -sgn * scale(st, nt, g) : sgn * scale(st, nt, g);
                     if constexpr (SM == 2) {
-                        acc[mt][nt] += D;
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) run[mt][nt][r] = fmaf(D[r], s, run[mt][nt][r]);
                     } else {
-                        const float s = scale(st, nt, g);
 #pragma unroll
                         for (int r = 0; r < 16; ++r) acc[mt][nt][r] = fmaf(D[r], s, acc[mt][nt][r]);
                     }
                 }
             }
+        }
+    }
+
+    __device__ __forceinline__ static void flush(f32x16 (&acc)[MT][NT], f32x16 (&run)[MT][NT]) {
+        if constexpr (SM == 2) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    acc[mt][nt] += run[mt][nt];
+                    run[mt][nt] = f32x16{};
+                }
         }
     }
 };
@@ -307,13 +337,7 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
         __syncthreads();
     };
 
-    f32x16 acc[MT][NT];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0.f;
+    f32x16 acc[MT][NT] = {}, run[MT][NT] = {};
 
     typename T::Stage sa, sb;
     stage_x(lds0, gb);
@@ -324,16 +348,18 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
             stage_x(lds1, g + SG);
             t.load(g + SG, sb);
         }
-        t.compute(lds0, g, sa, acc);
+        t.compute(lds0, g, sa, acc, run);
         landed();
         if (g + SG >= ge) break;
         if (g + 2 * SG < ge) {
             stage_x(lds0, g + 2 * SG);
             t.load(g + 2 * SG, sa);
         }
-        t.compute(lds1, g + SG, sb, acc);
+        t.compute(lds1, g + SG, sb, acc, run);
+        if (((g - gb) & (kRun / 32 - 1)) == kRun / 32 - 2 * SG) T::flush(acc, run);
         landed();
     }
+    T::flush(acc, run);
 
     // Register r of lane (i, h) is row 8 (r / 4) + 4 h + r % 4 of weight row i.
     const bool split_k = a.splits > 1;
@@ -446,12 +472,13 @@ __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
     if (t < 8) inv[(size_t)split * slabs * kSlab + row] = ldexpf(1.f, -e);
     auto put = [&](int p, const f32x4 &a, const f32x4 &b) {
         const int kk = k0 + 8 * p, g = kk >> 5, q = (kk >> 3) & 3;
+        const float sup = negated(g) ? -up : up;
         h8 l1, l2;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const int el = W4 ? slot_elem(j) : j;
             const float v = el < 4 ? a[el & 3] : b[el & 3];
-            const float s = v * ((W4 && (j & 2)) ? up * 0.0625f : up);
+            const float s = v * ((W4 && (j & 2)) ? sup * 0.0625f : sup);
             const _Float16 u = (_Float16)s;
             const float r = s - (float)u;
             l1[j] = u;
@@ -532,12 +559,13 @@ size_t scratch_of(const Plan &pl, int splits, int m, int n, bool pair) {
 
 // Tile and K split by a small cost model, in us, fitted to sweeps of (MT, NT,
 // splits) at M = 17..512 and N, K = 900..14336, which it meets within about 10%:
-//   * a CU finishes one 128-K stage of a block in 0.56 MT NT when other blocks
-//     hide its waits, and a block alone takes 0.9 + 0.45 MT NT (INT8 a third
-//     more: twice the weight bytes per stage);
+//   * a CU finishes one 128-K stage of a block in 0.25 + 0.55 MT NT when other
+//     blocks hide its waits, and a block alone takes 0.9 + 0.45 MT NT (INT8 a
+//     third more: twice the weight bytes per stage); past one block per CU the
+//     last, partly filled round costs half a round at a time;
 //   * K splits cost the reduce kernel and the partials' way through memory.
 // splits == 0 in the result: no plan fits the scratch.
-Plan plan(int m, int n, int k, int fmt, bool pair, size_t cap) {
+Plan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
     Plan pl{};
     pl.slabs = (m + kSlab - 1) / kSlab;
     pl.groups = (k + kPad - 1) / kPad * (kPad / 32);
@@ -545,15 +573,17 @@ Plan plan(int m, int n, int k, int fmt, bool pair, size_t cap) {
     double best = 1e30;
     for (int mt = 1; mt <= (pl.slabs > 1 ? 2 : 1); ++mt)
         for (int nt = pair ? 2 : 1; nt <= 2; ++nt) {
+            if (!grouped && mt * nt > 2) continue;   // two sums per result: registers
             const int mz = (pl.slabs + mt - 1) / mt;
             const int nbx = pair ? (n + 127) / 128 : (n + 128 * nt - 1) / (128 * nt);
-            const double busy = 0.56 * mt * nt;
+            const double busy = 0.25 + 0.55 * mt * nt;
             const double alone = (0.9 + 0.45 * mt * nt) * (fmt == Q_W8 ? 1.35 : 1.0);
             for (int s = 1; s <= stages && s <= kMaxSplits; ++s) {
                 const int len = (stages + s - 1) / s;
                 if ((stages + len - 1) / len != s) continue;
-                const long per_cu = ((long)mz * nbx * s + kCUs - 1) / kCUs;
-                double t = len * std::max((double)per_cu * busy, alone);
+                const double halves = (double)(((long)mz * nbx * s * 2 + kCUs - 1) / kCUs);
+                const double per_cu = std::max(1.0, halves * 0.5);
+                double t = len * std::max(per_cu * busy, alone);
                 if (s > 1) t += 3.0 + (double)(pair ? 2 : 1) * s * m * n * (8.0 / 5e6);
                 if (t < best && scratch_of(pl, s, m, n, pair) <= cap) {
                     best = t;
@@ -569,15 +599,21 @@ template <int FMT, int SM>
 int launch(const QArgs &a, const Plan &pl, bool pair, hipStream_t st) {
     const long tiles = (long)pl.mz * pl.nbx * pl.splits;
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
-    if (pair) {
-        if (pl.mt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 1, 2, SM, true>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_qgemm<FMT, 2, 2, SM, true>), grid, block, 0, st, a);
-    } else {
-        if (pl.nt == 1 && pl.mt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 1, 1, SM, false>), grid, block, 0, st, a);
-        else if (pl.nt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 2, 1, SM, false>), grid, block, 0, st, a);
-        else if (pl.mt == 1) hipLaunchKernelGGL((k_qgemm<FMT, 1, 2, SM, false>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k_qgemm<FMT, 2, 2, SM, false>), grid, block, 0, st, a);
+#define TB_QGO(MT_, NT_, PAIR_)                                                                  \
+    hipLaunchKernelGGL((k_qgemm<FMT, MT_, NT_, SM, PAIR_>), grid, block, 0, st, a)
+    if constexpr (SM != 2) {   // see plan()
+        if (pl.mt == 2 && pl.nt == 2) {
+            if (pair) TB_QGO(2, 2, true);
+            else TB_QGO(2, 2, false);
+            TB_LAUNCHED();
+            return TB_OK;
+        }
     }
+    if (pair) TB_QGO(1, 2, true);
+    else if (pl.mt == 2) TB_QGO(2, 1, false);
+    else if (pl.nt == 2) TB_QGO(1, 2, false);
+    else TB_QGO(1, 1, false);
+#undef TB_QGO
     TB_LAUNCHED();
     return TB_OK;
 }
@@ -589,21 +625,21 @@ bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt) {
     return k <= (int64_t)1 << 24 && m < (int64_t)1 << 24 && n < (int64_t)1 << 30;
 }
 
-size_t qgemm_scratch_bytes(int m, int n, int k, int fmt, bool pair) {
-    const Plan pl = plan(m, n, k, fmt, pair, SIZE_MAX);
+size_t qgemm_scratch_bytes(int m, int n, int k, int fmt, bool grouped, bool pair) {
+    const Plan pl = plan(m, n, k, fmt, grouped, pair, SIZE_MAX);
     return scratch_of(pl, pl.splits, m, n, pair);
 }
 
-bool qgemm_fits(int64_t m, int64_t n, int64_t k, int fmt, bool pair, size_t cap) {
+bool qgemm_fits(int64_t m, int64_t n, int64_t k, int fmt, bool grouped, bool pair, size_t cap) {
     return qgemm_shape_ok(m, n, k, fmt) &&
-           plan((int)m, (int)n, (int)k, fmt, pair, cap).splits > 0;
+           plan((int)m, (int)n, (int)k, fmt, grouped, pair, cap).splits > 0;
 }
 
 int qgemm(const QGemmParams &p, void *scratch, size_t cap, hipStream_t st) {
     const bool pair = p.w1 != nullptr;
     TB_REQUIRE(qgemm_shape_ok(p.m, p.n, p.k, p.fmt), TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: batched projection needs K % 32 == 0");
-    const Plan pl = plan(p.m, p.n, p.k, p.fmt, pair, cap);
+    const Plan pl = plan(p.m, p.n, p.k, p.fmt, p.grouped != 0, pair, cap);
     TB_REQUIRE(pl.splits > 0, TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: batched projection: scratch too small");
     uint8_t *rec = static_cast<uint8_t *>(scratch);

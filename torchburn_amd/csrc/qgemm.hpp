@@ -32,8 +32,8 @@ bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt);
 // Scratch of one call's fastest plan: the split activations and the split-K
 // partial sums.  A plan takes any `cap` that holds at least the activations
 // (qgemm_fits).
-size_t qgemm_scratch_bytes(int m, int n, int k, int fmt, bool pair);
-bool qgemm_fits(int64_t m, int64_t n, int64_t k, int fmt, bool pair, size_t cap);
+size_t qgemm_scratch_bytes(int m, int n, int k, int fmt, bool grouped, bool pair);
+bool qgemm_fits(int64_t m, int64_t n, int64_t k, int fmt, bool grouped, bool pair, size_t cap);
 
 // scratch: cap bytes, 256-byte aligned.
 int qgemm(const QGemmParams &p, void *scratch, size_t cap, hipStream_t st);

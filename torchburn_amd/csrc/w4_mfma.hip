@@ -237,14 +237,14 @@ size_t partials_only(int m, int n, int k, bool dual) {
 
 }  // namespace
 
-size_t w4_mfma_scratch_bytes(int m, int n, int k, bool dual, bool v2) {
+size_t w4_mfma_scratch_bytes(int m, int n, int k, bool dual, bool v2, bool grouped) {
     if (m >= kQGemmMinM && qgemm_shape_ok(m, n, k, qfmt(v2)))
-        return qgemm_scratch_bytes(m, n, k, qfmt(v2), dual);
+        return qgemm_scratch_bytes(m, n, k, qfmt(v2), grouped, dual);
     return partials_only(m, n, k, dual);
 }
 
 size_t w4_mfma_scratch_upto(int m, int n, int k, bool dual) {
-    return std::max(w4_mfma_scratch_bytes(m, n, k, dual, false),
+    return std::max(w4_mfma_scratch_bytes(m, n, k, dual),
                     partials_only(std::min(m, kQGemmMinM - 1), n, k, dual));
 }
 
@@ -259,14 +259,15 @@ int w4_mfma(const MfmaParams &p, int epi, float *part, size_t cap, hipStream_t s
                    TB_ERR_UNSUPPORTED,
                    "TB_UNSUPPORTED: v2 blocks need K % 64 == 0, a 4-byte aligned stream "
                    "under 4 GiB");
-    if (p.m >= kQGemmMinM && qgemm_fits(p.m, p.n, p.k, qfmt(p.v2), dual, cap)) {
+    const bool grouped = p.v2 || p.scale_mode == 0;
+    if (p.m >= kQGemmMinM && qgemm_fits(p.m, p.n, p.k, qfmt(p.v2), grouped, dual, cap)) {
         QGemmParams q{};
         q.x = p.x; q.w0 = p.w0; q.s0 = p.s0; q.b0 = p.b0;
         q.w1 = p.w1; q.s1 = p.s1; q.b1 = p.b1;
         q.res = epi == EPI_RESID ? p.res : nullptr;
         q.y = p.y; q.m = p.m; q.n = p.n; q.k = p.k;
         q.fmt = qfmt(p.v2);
-        q.grouped = p.v2 || p.scale_mode == 0;
+        q.grouped = grouped;
         q.gshift = p.gshift;
         q.s0_len = q.s1_len = p.scale_mode == 1 ? p.n : 1;
         return qgemm(q, part, cap, st);

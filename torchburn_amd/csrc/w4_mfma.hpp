@@ -26,7 +26,8 @@ struct MfmaParams {
 };
 
 // Scratch of the fastest form for this shape (dual = SwiGLU pair).
-size_t w4_mfma_scratch_bytes(int m, int n, int k, bool dual, bool v2 = false);
+size_t w4_mfma_scratch_bytes(int m, int n, int k, bool dual, bool v2 = false,
+                             bool grouped = true);
 
 // Scratch that serves every row count from 1 to m (v1 weights): below its own
 // fastest plan a call takes one that fits.
