@@ -44,11 +44,11 @@
 // nominal rate).  Measured on whole calls, against the kernel on fixed-point
 // limbs with an exponent per 64 elements and two more MFMAs per group for the
 // -8 of the weights that this one replaced:
-//   Llama-3-8B gate/up pair, 512 rows, group 32    271 us, 444 TFLOP/s (888 in
+//   Llama-3-8B gate/up pair, 512 rows, group 32    251 us, 479 TFLOP/s (958 in
 //                                                  MFMA work)
-//   Llama-3-8B MLP, 512 rows, group 64             949 -> 449 us
-//   64 rows, N = 14336, K = 4096, group 32         54.2 -> 38.8 us
-//   Llama-3-8B MLP in INT8, 128 rows               2562 -> 158 us, against GEMV
+//   Llama-3-8B MLP, 512 rows, group 64             939 -> 387 us
+//   64 rows, N = 14336, K = 4096, group 32         53.7 -> 32.0 us
+//   Llama-3-8B MLP in INT8, 128 rows               2561 -> 152 us, against GEMV
 //                                                  passes of 2 rows each
 // The error against 64 bits went from 6.2e-7 to 1.4e-7 for INT4 (activations
 // with large channels: the limbs follow each element's own size) and from
@@ -70,7 +70,6 @@ namespace {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kSlab = 32;            // activation rows of one MFMA tile
 constexpr int kGroupBytes = 4096;    // one slab x 32 K: 2 steps x 2 limbs x 1 KiB
@@ -85,10 +84,20 @@ __host__ __device__ constexpr int slot_elem(int e) { return (e >> 1) | ((e & 1) 
 // that large channels a power of two apart meet both signs).
 __host__ __device__ constexpr bool negated(int g) { return ((g ^ (g >> 2)) & 1) != 0; }
 
-__device__ __forceinline__ h8 expand_w4(uint32_t d) {
-    const uint32_t u = d >> 8, o = 0x64006400u;
-    const u32x4 v = {(d & 0x000F000Fu) | o, (d & 0x00F000F0u) | o, (u & 0x000F000Fu) | o,
-                     (u & 0x00F000F0u) | o};
+// The nibble masks, in registers: behind a literal the compiler takes an AND
+// and an OR instead of one v_and_or_b32.
+struct Masks {
+    uint32_t lo, hi;
+};
+__device__ __forceinline__ Masks nibble_masks() {
+    Masks k = {0x000F000Fu, 0x00F000F0u};
+    asm("" : "+v"(k.lo), "+v"(k.hi));
+    return k;
+}
+
+__device__ __forceinline__ h8 expand_w4(uint32_t d, const Masks &k, uint32_t o) {
+    const uint32_t u = d >> 8;
+    const u32x4 v = {(d & k.lo) | o, (d & k.hi) | o, (u & k.lo) | o, (u & k.hi) | o};
     const h8 c = {(_Float16)-1032.f, (_Float16)-1032.f, (_Float16)-1152.f, (_Float16)-1152.f,
                   (_Float16)-1032.f, (_Float16)-1032.f, (_Float16)-1152.f, (_Float16)-1152.f};
     return __builtin_bit_cast(h8, v) + c;
@@ -118,10 +127,10 @@ struct QArgs {
 // in the epilogue).
 template <int FMT, int MT, int NT, int SM, bool PAIR>
 struct QTile {
-    static constexpr int SG = FMT == Q_W8 ? 2 : 4;   // groups per stage
-    static constexpr int LD = 2;                     // 16-byte chunks per lane and column tile
+    static constexpr int SG = FMT == Q_W8 || MT == 4 ? 2 : 4;   // groups per stage
+    static constexpr int LD = FMT == Q_W8 ? SG : SG / 2;   // 16-byte chunks per lane and column tile
     static constexpr int NDW = FMT == Q_V2 ? 5 : 4;
-    static constexpr int NS = SM == 0 ? 4 : 2;       // scales per column tile and stage
+    static constexpr int NS = SM == 0 ? SG : SG / 2;       // scales per column tile and stage
 
     struct Stage {
         uint32_t q[NT][LD][NDW];
@@ -134,6 +143,8 @@ struct QTile {
     const float *sp[NT];
     uint32_t vrow[NT];       // byte offset of the lane's row (v2)
     int chunks;              // 32-element chunks of a row
+    Masks msk;
+    uint32_t magic;          // f16 1024 in both halves
 
     __device__ __forceinline__ QTile(const QArgs &aa) : a(aa) {
         lane = threadIdx.x & 63;
@@ -141,6 +152,9 @@ struct QTile {
         i = lane & 31;
         h = lane >> 5;
         chunks = a.k >> 5;
+        msk = nibble_masks();
+        magic = 0x64006400u;
+        asm("" : "+s"(magic));
     }
 
     __device__ __forceinline__ int col(int bx, int nt) const {
@@ -187,24 +201,25 @@ struct QTile {
             }
             if constexpr (FMT == Q_V2) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
+                for (int j = 0; j < NS; ++j) {
                     const int b = min((g0 >> 1) + j, (chunks >> 1) - 1);
                     st.s[nt][j] = __uint_as_float((uint32_t)*reinterpret_cast<const uint16_t *>(
                         wp[nt] + vrow[nt] + (uint32_t)b * kV2Block + 32u));
                 }
             } else if constexpr (SM == 0) {
-                if (g0 + 3 < chunks) {
-                    const f32x4u v = *reinterpret_cast<const f32x4u *>(sp[nt] + g0);
+                typedef float fvu __attribute__((ext_vector_type(NS), aligned(4)));
+                if (g0 + NS <= chunks) {
+                    const fvu v = *reinterpret_cast<const fvu *>(sp[nt] + g0);
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) st.s[nt][t] = v[t];
+                    for (int t = 0; t < NS; ++t) st.s[nt][t] = v[t];
                 } else {
 #pragma unroll
-                    for (int t = 0; t < 4; ++t)
+                    for (int t = 0; t < NS; ++t)
                         st.s[nt][t] = g0 + t < chunks ? sp[nt][g0 + t] : 0.f;
                 }
             } else if constexpr (SM == 1) {
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
+                for (int t = 0; t < NS; ++t)
                     st.s[nt][t] = g0 + 2 * t < chunks ? sp[nt][(32 * (g0 + 2 * t)) >> a.gshift] : 0.f;
             }
         }
@@ -232,13 +247,13 @@ struct QTile {
             }
             const auto s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
             const auto s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
-            B[0] = expand_w4((g & 1) ? s0[1] : s0[0]);
-            B[1] = expand_w4((g & 1) ? s1[1] : s1[0]);
+            B[0] = expand_w4((g & 1) ? s0[1] : s0[0], msk, magic);
+            B[1] = expand_w4((g & 1) ? s1[1] : s1[0], msk, magic);
         }
     }
 
     __device__ __forceinline__ float scale(const Stage &st, int nt, int g) const {
-        if (SM == 0) return st.s[nt][g & 3];
+        if (SM == 0) return st.s[nt][g];
         if (FMT == Q_V2) return f16_bits_to_f32(__float_as_uint(st.s[nt][g >> 1]));
         return SM == 1 ? st.s[nt][g >> 1] : 1.0f;
     }
@@ -557,41 +572,53 @@ size_t scratch_of(const Plan &pl, int splits, int m, int n, bool pair) {
            (splits > 1 ? (size_t)splits * (pair ? 2 : 1) * (size_t)m * n * sizeof(float) : 0);
 }
 
-// Tile and K split by a small cost model, in us, fitted to sweeps of (MT, NT,
-// splits) at M = 17..512 and N, K = 900..14336, which it meets within about 10%:
-//   * a CU finishes one 128-K stage of a block in 0.25 + 0.55 MT NT when other
-//     blocks hide its waits, and a block alone takes 0.9 + 0.45 MT NT (INT8 a
-//     third more: twice the weight bytes per stage); past one block per CU the
-//     last, partly filled round costs half a round at a time;
-//   * K splits cost the reduce kernel and the partials' way through memory.
-// splits == 0 in the result: no plan fits the scratch.
+// What a tile costs, in us per 128 K: `busy` of a CU's time when other blocks
+// hide its waits, `alone` by itself; `grain` is how finely a last, partly
+// filled round of blocks is paid for (blocks per CU).
+struct Tile {
+    int mt, nt;
+    double busy, alone, grain;
+};
+constexpr Tile kTiles[] = {{1, 1, 0.77, 1.35, 0.25}, {1, 2, 1.95, 1.0, 0.5}, {2, 1, 1.2, 1.95, 1.0},
+                           {2, 2, 2.15, 2.85, 1.0}, {4, 2, 3.9, 7.0, 1.0}};
+
+// Tile and K split by a cost model: K stages x the block rounds of the busiest
+// CU, each round's start, and for K splits the reduce kernel and the partials'
+// way through memory.  The constants are fitted to sweeps of every tile and
+// split at 45 shapes (5..1024 rows, N and K 900..14336, all formats): its
+// choice is the fastest at 40 of them and at most 8% from it at the others
+// (64 x 14336 x 4096: 38.8 us as first set, now 33.3).  Tiles of 64 x 64 and
+// more outputs per wave have no room for the second sum of row scales; the
+// 128-row tile is for v1 weights (5% ahead of 64 rows at 512 rows and N = 28672,
+// since a weight's expansion serves twice the rows; a v2 lane holds more of its
+// stage and would spill).  splits == 0 in the result: no plan fits the scratch.
 Plan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
     Plan pl{};
     pl.slabs = (m + kSlab - 1) / kSlab;
     pl.groups = (k + kPad - 1) / kPad * (kPad / 32);
     const int stages = pl.groups / 4;
+    const double f = fmt == Q_V2 ? 1.3 : fmt == Q_W8 ? 0.72 : 1.0;
+    const double fa = fmt == Q_V2 ? 1.3 : fmt == Q_W8 ? 0.95 : 1.0;
     double best = 1e30;
-    for (int mt = 1; mt <= (pl.slabs > 1 ? 2 : 1); ++mt)
-        for (int nt = pair ? 2 : 1; nt <= 2; ++nt) {
-            if (!grouped && mt * nt > 2) continue;   // two sums per result: registers
-            const int mz = (pl.slabs + mt - 1) / mt;
-            const int nbx = pair ? (n + 127) / 128 : (n + 128 * nt - 1) / (128 * nt);
-            const double busy = 0.25 + 0.55 * mt * nt;
-            const double alone = (0.9 + 0.45 * mt * nt) * (fmt == Q_W8 ? 1.35 : 1.0);
-            for (int s = 1; s <= stages && s <= kMaxSplits; ++s) {
-                const int len = (stages + s - 1) / s;
-                if ((stages + len - 1) / len != s) continue;
-                const double halves = (double)(((long)mz * nbx * s * 2 + kCUs - 1) / kCUs);
-                const double per_cu = std::max(1.0, halves * 0.5);
-                double t = len * std::max(per_cu * busy, alone);
-                if (s > 1) t += 3.0 + (double)(pair ? 2 : 1) * s * m * n * (8.0 / 5e6);
-                if (t < best && scratch_of(pl, s, m, n, pair) <= cap) {
-                    best = t;
-                    pl.mt = mt; pl.nt = nt; pl.mz = mz; pl.nbx = nbx;
-                    pl.splits = s; pl.slen = len * 4;
-                }
+    for (const Tile &t : kTiles) {
+        if (t.mt > pl.slabs || (pair && t.nt == 1)) continue;
+        if ((!grouped && t.mt * t.nt > 2) || (fmt == Q_V2 && t.mt * t.nt > 2)) continue;
+        const int mz = (pl.slabs + t.mt - 1) / t.mt;
+        const int nbx = pair ? (n + 127) / 128 : (n + 128 * t.nt - 1) / (128 * t.nt);
+        for (int s = 1; s <= stages && s <= kMaxSplits; ++s) {
+            const int len = (stages + s - 1) / s;
+            if ((stages + len - 1) / len != s) continue;
+            const double blocks = (double)mz * nbx * s / kCUs;
+            const double rounds = std::max(1.0, ceil(blocks / t.grain) * t.grain);
+            double us = len * std::max(rounds * t.busy * f, t.alone * fa) + 1.2 * ceil(blocks / 2);
+            if (s > 1) us += 3.0 + (double)(pair ? 2 : 1) * s * m * n * 1.57e-6;
+            if (us < best && scratch_of(pl, s, m, n, pair) <= cap) {
+                best = us;
+                pl.mt = t.mt; pl.nt = t.nt; pl.mz = mz; pl.nbx = nbx;
+                pl.splits = s; pl.slen = len * 4;
             }
         }
+    }
     return pl;
 }
 
@@ -601,10 +628,15 @@ int launch(const QArgs &a, const Plan &pl, bool pair, hipStream_t st) {
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
 #define TB_QGO(MT_, NT_, PAIR_)                                                                  \
     hipLaunchKernelGGL((k_qgemm<FMT, MT_, NT_, SM, PAIR_>), grid, block, 0, st, a)
-    if constexpr (SM != 2) {   // see plan()
-        if (pl.mt == 2 && pl.nt == 2) {
-            if (pair) TB_QGO(2, 2, true);
-            else TB_QGO(2, 2, false);
+    if constexpr (FMT == Q_W4 && SM != 2) {   // see plan()
+        if (pl.mt * pl.nt > 2) {
+            if (pl.mt == 4) {
+                if (pair) TB_QGO(4, 2, true);
+                else TB_QGO(4, 2, false);
+            } else {
+                if (pair) TB_QGO(2, 2, true);
+                else TB_QGO(2, 2, false);
+            }
             TB_LAUNCHED();
             return TB_OK;
         }
