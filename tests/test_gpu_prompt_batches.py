@@ -1,0 +1,71 @@
+"""Batched prompts against the CPU oracle's steps where the batch changes form:
+INT8 layers (GEMV passes and the batched kernel, by rows), prompts of 2 to 6
+tokens around the shortest batch, a second chunk after 1024 rows, buffers that
+grow with a longer prompt, and INT8 verify_tokens with every lm_head."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from torchburn_amd import synth
+from torchburn_amd.decoder import decoder_from_weights
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-4   # max|d| / max|ref|, as for the decoder's steps
+
+
+def pair(seed, wkind, lmkind, max_seq, **kw):
+    cfg = dict(num_layers=2, hidden=256, intermediate=512, num_heads=4, num_kv_heads=2,
+               head_dim=64, vocab=1000, eps=1e-6, rope_theta=1e6, qkv_bias=True)
+    cfg.update(kw)
+    w = synth.decoder_weights(cfg, seed, wkind, lmkind, 32)
+    ref = O.Decoder(w, dict(num_layers=cfg["num_layers"], hidden=cfg["hidden"],
+                            intermediate=cfg["intermediate"], num_heads=cfg["num_heads"],
+                            num_kv_heads=cfg["num_kv_heads"], head_dim=cfg["head_dim"],
+                            vocab=cfg["vocab"], group_size=32, max_seq=max_seq,
+                            rope_theta=cfg["rope_theta"], eps=cfg["eps"], wkind=wkind,
+                            lmkind=lmkind))
+    return ref, decoder_from_weights(w, cfg, group_size=32, max_seq_len=max_seq), cfg
+
+
+def rel(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return float(np.abs(a - b).max() / max(np.abs(b).max(), 1e-30))
+
+
+@pytest.mark.parametrize("wkind,lmkind,lengths", [
+    (8, 8, (2, 3, 6)), (8, 32, (40, 70)), (4, 4, (2, 3, 5)), (4, 4, (5, 300, 1030)), (8, 8, (520,))])
+def test_prompts_one_after_another(cuda, wkind, lmkind, lengths):
+    print(f"case prompts wkind={wkind} lmkind={lmkind} lengths={lengths}", flush=True)
+    ref, dec, cfg = pair(91, wkind, lmkind, sum(lengths) + 8)
+    g = np.random.default_rng(91)
+    pos = 0
+    for n in lengths:
+        toks = [int(t) for t in g.integers(0, cfg["vocab"], n)]
+        for i, t in enumerate(toks):
+            lo = ref.step(t, pos + i)
+        assert dec.prefill_tokens(toks, pos) == pos + n
+        assert rel(dec.get_logits(), lo) < TOL
+        pos += n
+    for i in range(3):   # steps over the cache that the batches wrote
+        t = O.argmax(lo)
+        lo = ref.step(t, pos + i)
+        lg, am = dec._step(t, pos + i, True)
+        assert rel(lg, lo) < TOL and am == O.argmax(lo)
+    ref.close()
+    dec.close()
+
+
+@pytest.mark.parametrize("lmkind,n", [(8, 2), (8, 7), (8, 70), (32, 5)])
+def test_int8_verify_rows(cuda, lmkind, n):
+    print(f"case int8 verify lmkind={lmkind} n={n}", flush=True)
+    ref, dec, cfg = pair(92, 8, lmkind, 128)
+    g = np.random.default_rng(92)
+    pre, toks = ([int(t) for t in g.integers(0, cfg["vocab"], k)] for k in (9, n))
+    for i, t in enumerate(pre):
+        ref.step(t, i)
+    dec.prefill_tokens(pre, 0)
+    want = np.stack([ref.step(t, 9 + i).copy() for i, t in enumerate(toks)])
+    assert rel(dec.verify_tokens(9, toks), want) < TOL
+    ref.close()
+    dec.close()

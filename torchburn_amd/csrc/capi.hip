@@ -389,14 +389,11 @@ static int generic(const float *x, const void *w0, const float *s0, int mode0, c
     return gemv_generic(g, st);
 }
 
-// One INT8 projection, or a SwiGLU pair (p.w1 set), over m rows.  GEMV passes
-// take 2 rows each and re-read the weights; from 5 rows, or 3 on weights of
-// 32 Mi elements, the batched kernel reads them once (us, passes against
-// batched: 4096 x 4096 at 3 rows 12.2 / 13.6 and at 5 17 / 14; 14336 x 4096 at
-// 2 rows 14.0 / 22.7 and at 3 25.4 / 23.5; 4864 x 896 at 4 rows 9.3 / 11.1).
+// One INT8 projection, or a SwiGLU pair (p.w1 set), over m rows: the batched
+// kernel where it wins, else GEMV passes or, for their other shapes, the
+// any-shape GEMV.
 static bool w8_batched(const DenseParams &p, int64_t m) {
-    const int64_t elems = (int64_t)p.n * p.k * (p.w1 ? 2 : 1);
-    return (m >= 5 || (m >= 3 && elems >= (int64_t)1 << 25)) && aligned(p.x, 16) &&
+    return qgemm_w8_wins(m, (int64_t)p.n * p.k * (p.w1 ? 2 : 1)) && aligned(p.x, 16) &&
            aligned(p.w0, 16) && aligned(p.w1, 16) && qgemm_shape_ok(m, p.n, p.k, Q_W8);
 }
 

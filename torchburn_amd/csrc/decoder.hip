@@ -30,6 +30,7 @@
 #include "gemv_dense.hpp"
 #include "tb_common.hpp"
 #include "w4_gemv.hpp"
+#include "qgemm.hpp"
 #include "w4_limb.hpp"
 #include "w4_mfma.hpp"
 #include "v2_layout.hpp"
@@ -559,30 +560,40 @@ struct Decoder {
         return TB_OK;
     }
 
-    // ---- Batched prefill (INT4 projections on the FP32-MFMA GEMM) ----------
+    // ---- Batched prefill ----------------------------------------------------
     // Chunks of up to kPrefillRows prompt positions go through each layer as
     // one batch: row RMSNorms, QKV GEMM (+bias), RoPE + KV append for every
     // row, causal prefill attention, O GEMM + residual, gate/up GEMM with
     // SwiGLU, down GEMM + residual; the last row then takes the final norm
-    // and lm_head as a step would.  Buffers are allocated on first use.
-    static constexpr int kPrefillRows = 256;
+    // and lm_head as a step would.  The buffers hold the longest chunk seen,
+    // rounded up to a power of two from 256 rows: 1024 rows fill the GEMMs' tiles
+    // (a 511-token Llama-3-8B prompt: 24.7 ms in chunks of 256, 21.4 ms in one).
+    static constexpr int kPrefillRows = 1024;
+    int pf_rows_cap = 0;
     float *pf_x = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr, *pf_q = nullptr,
           *pf_a = nullptr, *pf_h = nullptr, *pf_part = nullptr;
     size_t pf_part_bytes = 0;
     int *pf_tok = nullptr;
 
-    int prefill_alloc() {
-        if (pf_x) return TB_OK;
-        const int R = kPrefillRows;
+    // Scratch of a projection of up to m rows.
+    size_t gemm_scratch(int m, int n, int k, bool pair) const {
+        return wbits == 8 ? qgemm_scratch_bytes(m, n, k, Q_W8, false, pair)
+                          : w4_mfma_scratch_upto(m, n, k, pair);
+    }
+
+    int prefill_alloc(int64_t n) {
+        int R = 256;
+        while (R < kPrefillRows && R < n) R *= 2;
+        if (R <= pf_rows_cap) return TB_OK;
         const size_t nq = (size_t)(hq + 2 * hkv) * hd;
-        size_t part = w4_mfma_scratch_upto(R, (int)nq, H, false);
-        part = std::max(part, w4_mfma_scratch_upto(R, H, hq * hd, false));
-        part = std::max(part, w4_mfma_scratch_upto(R, I, H, true));
-        part = std::max(part, w4_mfma_scratch_upto(R, H, I, false));
+        size_t part = gemm_scratch(R, (int)nq, H, false);
+        part = std::max(part, gemm_scratch(R, H, hq * hd, false));
+        part = std::max(part, gemm_scratch(R, I, H, true));
+        part = std::max(part, gemm_scratch(R, H, I, false));
         // 3..16 rows (verify_tokens, short chunks) take the small-batch
         // projection: records + split partials of the largest of its shapes
         size_t lb = 0;
-        for (int m = 3; m <= kLimbMaxM; ++m) {
+        for (int m = 3; wbits == 4 && m <= kLimbMaxM; ++m) {
             auto need = [&](int n, int k, bool pair) -> size_t {
                 if (!limb_shape_ok(m, n, k, pair)) return 0;
                 return up256(limb_records_bytes(m, k)) + limb_partials_bytes(m, n, k, pair);
@@ -597,11 +608,12 @@ struct Decoder {
             (rc = alloc(&pf_q, (size_t)R * hq * hd * 4)) ||
             (rc = alloc(&pf_a, (size_t)R * hq * hd * 4)) || (rc = alloc(&pf_h, (size_t)R * I * 4)) ||
             (rc = alloc(&pf_part, part)) || (rc = alloc(&pf_tok, (size_t)R * 4)) ||
-            (lb && (rc = alloc(&pf_limb, lb))) ||
-            (lb && (rc = alloc(&pf_hrec, limb_records_bytes(kLimbMaxM, I)))))
+            (lb && !pf_limb && (rc = alloc(&pf_limb, lb))) ||
+            (lb && !pf_hrec && (rc = alloc(&pf_hrec, limb_records_bytes(kLimbMaxM, I)))))
             return rc;
         pf_limb_bytes = lb;
         pf_part_bytes = part;
+        pf_rows_cap = R;
         return TB_OK;
     }
 
@@ -652,9 +664,33 @@ struct Decoder {
                     EPI_RESID);
     }
 
+    // m rows through an INT8 projection: batched, or GEMV passes of 2 rows.
+    int rows_w8(const float *xin, const void *w, const float *s, const float *b, const void *w2,
+                const float *s2, const float *res, float *y, int m, int n, int k, int epi,
+                void *scratch, size_t cap) {
+        if (qgemm_w8_wins(m, (int64_t)n * k * (w2 ? 2 : 1)) || k > kMaxGemvElems) {
+            QGemmParams q{};
+            q.x = xin; q.w0 = w; q.s0 = s; q.b0 = b; q.w1 = w2; q.s1 = s2; q.res = res; q.y = y;
+            q.m = m; q.n = n; q.k = k; q.fmt = Q_W8; q.s0_len = q.s1_len = n;
+            return qgemm(q, scratch, cap, st);
+        }
+        for (int r0 = 0; r0 < m; r0 += kMaxRowsPerPass) {
+            DenseParams p{};
+            p.x = xin + (size_t)r0 * k; p.w0 = w; p.rs0 = s; p.rs0_len = n; p.b0 = b;
+            p.w1 = w2; p.rs1 = s2; p.rs1_len = w2 ? n : 0;
+            p.res = res ? res + (size_t)r0 * n : nullptr; p.y = y + (size_t)r0 * n;
+            p.m = std::min(kMaxRowsPerPass, m - r0); p.n = n; p.k = k;
+            int rc = dense_gemv(p, W_I8, epi, st);
+            if (rc) return rc;
+        }
+        return TB_OK;
+    }
+
     int gemm(const float *xin, const void *w, const float *s, const float *b, const void *w2,
              const float *s2, const float *res, float *y, int m, int n, int k, int epi) {
         int rc = TB_OK;
+        if (wbits == 8) return rows_w8(xin, w, s, b, w2, s2, res, y, m, n, k, epi, pf_part,
+                                       pf_part_bytes);
         if (limb_gemm(xin, w, s, b, w2, s2, res, y, m, n, k, rc)) return rc;
         MfmaParams p{};
         p.x = xin;
@@ -669,10 +705,16 @@ struct Decoder {
     // loop.
     bool under_cap(int64_t start, int64_t n) const { return start + n <= (int64_t)attn_cap; }
 
+    // Prompts from this length run as batches (us for 3 tokens, batched / step
+    // by step: eight Llama-3-8B layers in INT4 808 / 1496, in INT8 1129 / 1829,
+    // Qwen2.5-0.5B 1399 / 2546 and 1358 / 2530; for 2 tokens the INT4 layers
+    // 1193 / 1014).
+    static constexpr int kBatchPrompt = 3;
+    static constexpr int kMaxGemvElems = 16384;   // K of one streaming GEMV pass
     bool prefill_batchable(const int64_t *tokens, int64_t n, int64_t start) const {
         static const bool loop_only = getenv("TB_PREFILL_LOOP") != nullptr;
         // W4A8 rounds each token's projection inputs: the step loop does that
-        if (loop_only || wbits != 4 || n < 16 || !under_cap(start, n) || a8_wanted()) return false;
+        if (loop_only || n < kBatchPrompt || !under_cap(start, n) || a8_wanted()) return false;
         for (int64_t i = 0; i < n; ++i)
             if (tokens[i] < 0 || tokens[i] >= V) return false;   // the step's zero-logit rule
         return true;
@@ -704,6 +746,16 @@ struct Decoder {
             }
             return TB_OK;
         }
+        if (lmbits == 8 && qgemm_w8_wins(M, (int64_t)V * H)) {
+            const size_t lb = qgemm_scratch_bytes(64, V, H, Q_W8, false, false);
+            if (!pf_lmpart && (rc = alloc(&pf_lmpart, lb))) return rc;
+            for (int r0 = 0; r0 < M; r0 += 64)
+                if ((rc = rows_w8(xr + (size_t)r0 * H, lm_w, lm_s, nullptr, nullptr, nullptr,
+                                  nullptr, y + (size_t)r0 * V, std::min(64, M - r0), V, H,
+                                  EPI_PLAIN, pf_lmpart, lb)))
+                    return rc;
+            return TB_OK;
+        }
         for (int r0 = 0; r0 < M; r0 += 2) {
             DenseParams p{};
             p.x = xr + (size_t)r0 * H; p.w0 = lm_w; p.rs0 = lm_s; p.rs0_len = lm_s ? V : 0;
@@ -717,13 +769,13 @@ struct Decoder {
     // returns them (decoder.rs:565-581); otherwise only the last position's.
     int prefill_batched(const int64_t *tokens, int64_t n, int64_t start,
                         float *rows_out = nullptr) {
-        int rc = prefill_alloc();
+        int rc = prefill_alloc(n);
         if (rc) return rc;
         const int nq = (hq + 2 * hkv) * hd;
         // Host copy of the whole prompt, alive until the closing synchronize.
         std::vector<int> tok32(tokens, tokens + n);
-        for (int64_t c0 = 0; c0 < n; c0 += kPrefillRows) {
-            const int M = (int)std::min<int64_t>(kPrefillRows, n - c0);
+        for (int64_t c0 = 0; c0 < n; c0 += pf_rows_cap) {
+            const int M = (int)std::min<int64_t>(pf_rows_cap, n - c0);
             const int pos0 = (int)(start + c0);
             TB_HIP(hipMemcpyAsync(pf_tok, tok32.data() + c0, (size_t)M * 4, hipMemcpyHostToDevice,
                                   st));
@@ -1335,7 +1387,7 @@ int tb_decoder_verify(tb_decoder *d, int64_t start_offset, const int64_t *tokens
     TB_REQUIRE(start_offset >= 0 && start_offset + n <= d->max_seq, TB_ERR_VALUE,
                "verify exceeds max_seq_len");
     if (n == 0) return TB_OK;
-    bool batch = d->wbits == 4 && n >= 2 && d->under_cap(start_offset, n) && !d->a8_wanted();
+    bool batch = n >= 2 && d->under_cap(start_offset, n) && !d->a8_wanted();
     for (int64_t i = 0; i < n && batch; ++i) batch = tokens[i] >= 0 && tokens[i] < d->V;
     if (!batch) {
         for (int64_t i = 0; i < n; ++i) {

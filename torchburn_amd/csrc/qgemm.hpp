@@ -29,6 +29,15 @@ struct QGemmParams {
 // Shapes the kernel takes: m >= 1, k a multiple of 32 (v2: of 64) up to 2^24.
 bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt);
 
+// Whether INT8 rows go to this kernel rather than to GEMV passes of 2 rows that
+// re-read the weights (elems of them): from 5 rows, or 3 on weights of 32 Mi
+// elements (us, passes against batched: 4096 x 4096 at 3 rows 12.2 / 13.6 and
+// at 5 17 / 14; 14336 x 4096 at 2 rows 14.0 / 22.7 and at 3 25.4 / 23.5; 4864 x
+// 896 at 4 rows 9.3 / 11.1).
+inline bool qgemm_w8_wins(int64_t m, int64_t elems) {
+    return m >= 5 || (m >= 3 && elems >= (int64_t)1 << 25);
+}
+
 // Scratch of one call's fastest plan: the split activations and the split-K
 // partial sums.  A plan takes any `cap` that holds at least the activations
 // (qgemm_fits).
