@@ -76,8 +76,8 @@ TB_API const char *tb_version(void);
  * or NULL, out f32 [M, N].  Any K >= 1 and any even group_size (a short last
  * group, as gemv.rs:1650-1660; groups start on byte boundaries).  K a multiple of 32 with a power-of-two group_size >= 32
  * dividing K runs the streaming kernels: M <= 4 the GEMV (one pass of up to 4
- * rows, K <= 16384), M >= 5 the FP32-MFMA projection (weights dequantized in
- * registers into the MFMA operand); other shapes run the any-shape GEMV.
+ * rows, K <= 16384), M >= 5 the batched f16-MFMA projections; other shapes run
+ * the any-shape GEMV.
  */
 TB_API int tb_w4a32_grouped_linear(const float *x, const uint8_t *w_packed, const float *scales,
                             const float *bias, float *out, int64_t m, int64_t n, int64_t k,

@@ -21,7 +21,6 @@
 #include "tb_common.hpp"
 #include "w4_gemv.hpp"
 #include "w4_limb.hpp"
-#include "w4_mfma.hpp"
 #include "v2_layout.hpp"
 #include "qgemm.hpp"
 #include "quantize.hpp"
@@ -68,9 +67,9 @@ int rows_j_env() {
     static int v = env_int("TB_W4_J", 0);
     return v;
 }
-// Activation rows from which INT4 projections run on FP32 MFMA instead of the
-// GEMV (measured crossover: passes of 2 rows re-read the weights, the MFMA
-// tile pads to 16 rows; TB_MFMA_MIN_M overrides, for tuning sweeps only).
+// Activation rows from which INT4 projections run on the batched kernel
+// (qgemm.hip) instead of the GEMV, whose pass takes 4 rows (TB_MFMA_MIN_M
+// overrides, for tuning sweeps only).
 int64_t mfma_min_m() {
     static int v = env_int("TB_MFMA_MIN_M", 5);
     return v < 1 ? 1 : v;
@@ -164,32 +163,45 @@ static W4Params w4_params(const float *x, const uint8_t *w, const float *s, cons
     return p;
 }
 
-static MfmaParams mfma_params(const float *x, const uint8_t *w, const float *s, const float *b,
-                              float *y, int64_t m, int64_t n, int64_t k, int64_t gs) {
-    MfmaParams p{};
+static QGemmParams qgemm_params(const float *x, const uint8_t *w, const float *s, const float *b,
+                                float *y, int64_t m, int64_t n, int64_t k, int64_t gs) {
+    QGemmParams p{};
     p.x = x; p.w0 = w; p.s0 = s; p.b0 = b; p.y = y;
-    p.m = (int)m; p.n = (int)n; p.k = (int)k; p.gshift = std::max(gshift_of(gs), 5);
+    p.m = (int)m; p.n = (int)n; p.k = (int)k;
+    p.grouped = 1;
+    p.gshift = std::max(gshift_of(gs), 5);
     return p;
 }
 
-// The MFMA projection with its split-K partials in the library workspace.
-static int mfma_ws(const MfmaParams &p, int epi, hipStream_t st) {
-    WsLease lease;
-    const size_t bytes = w4_mfma_scratch_bytes(p.m, p.n, p.k, p.w1 != nullptr);
-    int rc = workspace(bytes, st, lease);
-    if (rc) return rc;
-    void *ws = lease.ptr;
-    return w4_mfma(p, epi, static_cast<float *>(ws), bytes, st);
+static QPlan mlp_plan(int64_t m, int64_t n, int64_t k, bool pair, size_t cap) {
+    return qgemm_plan((int)m, (int)n, (int)k, Q_W4, true, pair, cap);
 }
 
-// Shapes of the small-batch f16-MFMA projection: limb_min_m() <= m <= limb_max_m(),
-// K % 128 == 0 (a SwiGLU pair: N % 128 == 0), 16-byte aligned x and w, a power-of-two
-// group >= 32 dividing K (or per-row / scalar scales).
-static bool limb_fast(const float *x, const void *w, int64_t m, int64_t n, int64_t k,
-                      int64_t gs, bool per_row, bool pair) {
+// The batched projection with its scratch in the library workspace.
+static int qgemm_ws(const QGemmParams &p, hipStream_t st) {
+    WsLease lease;
+    const QPlan pl = qgemm_plan(p);
+    int rc = pl.bytes ? workspace(pl.bytes, st, lease) : TB_OK;
+    if (rc) return rc;
+    return qgemm(p, pl, lease.ptr, st);
+}
+
+// Shapes the small-batch f16-MFMA projection takes: limb_min_m() <= m <=
+// limb_max_m(), K % 128 == 0 (a SwiGLU pair: N % 128 == 0), 16-byte aligned x
+// and w, a power-of-two group >= 32 dividing K (or per-row / scalar scales).
+static bool limb_takes(const float *x, const void *w, int64_t m, int64_t n, int64_t k,
+                       int64_t gs, bool per_row, bool pair) {
     if (m < limb_min_m() || m > limb_max_m() || !limb_shape_ok(m, n, k, pair)) return false;
     if (!per_row && (gshift_of(gs) < 0 || k % gs != 0)) return false;
     return aligned(x, 16) && aligned(w, 16);
+}
+
+// ... and those it runs: weights large enough, or rows too few for the batched
+// kernel and K past one GEMV pass.
+static bool limb_fast(const float *x, const void *w, int64_t m, int64_t n, int64_t k,
+                      int64_t gs, bool per_row, bool pair) {
+    return limb_takes(x, w, m, n, k, gs, per_row, pair) &&
+           (limb_wins(n * k * (pair ? 2 : 1)) || (m < mfma_min_m() && k > kMaxGemvK));
 }
 
 // scale_mode 0: grouped scales [n, k / gs]; 1: one per row; 2: one scalar.
@@ -260,12 +272,7 @@ static int generic(const float *x, const void *w0, const float *s0, int mode0, c
 static int linear_w4(const float *x, const uint8_t *w, const float *s, bool v2,
                      const float *bias, const float *res, float *out, int64_t m, int64_t n,
                      int64_t k, int64_t gs, hipStream_t st, int scale_mode = 0) {
-    // M = 16 with N and K at most 4096 takes the FP32-MFMA projection: all 16
-    // rows share one LDS tile there, where the two-tile limb form needs five K
-    // splits (14.4 against 15.4 us at N = K = 4096; from N = 14336 the limb
-    // form is faster, 25.7 against 30.2 us)
-    const bool lb = !v2 && limb_fast(x, w, m, n, k, gs, scale_mode != 0, false) &&
-                    !(m == 16 && n <= 4096 && k <= 4096);
+    const bool lb = !v2 && limb_fast(x, w, m, n, k, gs, scale_mode != 0, false);
     const bool any_shape = !v2 && !lb && !w4_fast(x, w, m, k, gs, scale_mode != 0);
     // W4A8 applies to every group-64 projection, whichever kernel takes the
     // shape (gemv.rs:1559-1563).  With K % 64 != 0 the reference's VNNI row
@@ -275,11 +282,13 @@ static int linear_w4(const float *x, const uint8_t *w, const float *s, bool v2,
     const size_t xb = a8 ? up256((size_t)m * (size_t)k * sizeof(float)) : 0;
     const int epi = res ? EPI_RESID : EPI_PLAIN;
     const bool mf = !lb && !any_shape && m >= mfma_min_m();
+    const QPlan pl = mf ? qgemm_plan((int)m, (int)n, (int)k, v2 ? Q_V2 : Q_W4,
+                                     v2 || scale_mode == 0, false)
+                        : QPlan{};
     const size_t rest = any_shape ? 0
                         : lb ? up256(limb_records_bytes((int)m, (int)k)) +
                                    limb_partials_bytes((int)m, (int)n, (int)k, false)
-                        : mf ? w4_mfma_scratch_bytes((int)m, (int)n, (int)k, false, v2,
-                                                    v2 || scale_mode == 0)
+                        : mf ? pl.bytes
                              : xq_bytes(m, k);
     const float *xin = x;
     void *tail = nullptr;
@@ -307,11 +316,12 @@ static int linear_w4(const float *x, const uint8_t *w, const float *s, bool v2,
         return w4_limb(q, part, st);
     }
     if (mf) {
-        MfmaParams q = mfma_params(xin, w, s, bias, out, m, n, k, gs);
+        QGemmParams q = qgemm_params(xin, w, s, bias, out, m, n, k, gs);
         q.res = res;
-        q.v2 = v2 ? 1 : 0;
-        q.scale_mode = scale_mode;
-        return w4_mfma(q, epi, static_cast<float *>(tail), rest, st);
+        q.fmt = v2 ? Q_V2 : Q_W4;
+        q.grouped = v2 || scale_mode == 0;
+        q.s0_len = scale_mode == 1 ? (int)n : 1;
+        return qgemm(q, pl, tail, st);
     }
     W4Params p = w4_params(xin, w, s, bias, out, m, n, k, gs);
     p.res = res;
@@ -397,19 +407,20 @@ static bool w8_batched(const DenseParams &p, int64_t m) {
            aligned(p.w0, 16) && aligned(p.w1, 16) && qgemm_shape_ok(m, p.n, p.k, Q_W8);
 }
 
-static size_t w8_scratch_bytes(const DenseParams &p, int64_t m) {
-    return w8_batched(p, m) ? qgemm_scratch_bytes((int)m, p.n, p.k, Q_W8, false, p.w1 != nullptr) : 0;
+static QPlan w8_plan(const DenseParams &p, int64_t m) {
+    return w8_batched(p, m) ? qgemm_plan((int)m, p.n, p.k, Q_W8, false, p.w1 != nullptr) : QPlan{};
 }
 
-static int w8_rows(const DenseParams &p, int64_t m, void *scratch, size_t cap, hipStream_t st) {
-    if (w8_batched(p, m)) {
+static int w8_rows(const DenseParams &p, const QPlan &pl, int64_t m, void *scratch,
+                   hipStream_t st) {
+    if (pl.mt) {
         QGemmParams q{};
         q.x = p.x; q.w0 = p.w0; q.s0 = p.rs0; q.b0 = p.b0;
         q.w1 = p.w1; q.s1 = p.rs1; q.b1 = p.b1;
         q.res = p.res; q.y = p.y; q.m = (int)m; q.n = p.n; q.k = p.k;
         q.fmt = Q_W8;
         q.s0_len = p.rs0_len; q.s1_len = p.rs1_len;
-        return qgemm(q, scratch, cap, st);
+        return qgemm(q, pl, scratch, st);
     }
     if (w8_fast(p.x, p.w0, p.k) && aligned(p.w1, 16))
         return dense_rows(p, W_I8, p.w1 ? EPI_SWIGLU : (p.res ? EPI_RESID : EPI_PLAIN), m, st);
@@ -441,16 +452,26 @@ static int mlp_w4_check(const MlpW4 &a, const char *op) {
     return TB_OK;
 }
 
-// 0: any-shape GEMVs; 1: batched pair (w4_mfma); 2: GEMV passes; 3: small-batch f16 MFMA
-static int mlp_w4_path(const MlpW4 &a) {
-    if (limb_fast(a.x, a.gate_w, a.m, a.inter, a.k, a.gs, false, true) &&
-        aligned(a.up_w, 16) &&
-        limb_fast(a.x, a.down_w, a.m, a.n_out, a.inter, a.gs, false, false))
-        return 3;
+// 0: any-shape GEMVs; 1: batched pair (qgemm); 2: GEMV passes; 3: small-batch f16 MFMA
+static int mlp_w4_route(const MlpW4 &a, bool limbs) {
+    if (limbs) return 3;
     if (!w4_fast(a.x, a.gate_w, a.m, a.k, a.gs, false) || !aligned(a.up_w, 16) ||
         !w4_fast(a.x, a.down_w, a.m, a.inter, a.gs, false))
         return 0;
     return a.m >= mfma_min_m() ? 1 : 2;
+}
+
+// Whether both projections' shapes suit the small-batch kernel.
+static bool mlp_limb_takes(const MlpW4 &a) {
+    return limb_takes(a.x, a.gate_w, a.m, a.inter, a.k, a.gs, false, true) &&
+           aligned(a.up_w, 16) &&
+           limb_takes(a.x, a.down_w, a.m, a.n_out, a.inter, a.gs, false, false);
+}
+
+static int mlp_w4_path(const MlpW4 &a) {
+    const bool large = limb_wins(2 * a.inter * a.k) || limb_wins(a.n_out * a.inter) ||
+                       (a.m < mfma_min_m() && std::max(a.k, a.inter) > kMaxGemvK);
+    return mlp_w4_route(a, large && mlp_limb_takes(a));
 }
 
 // Scratch: h [m, inter] f32, then the batched projections' scratch (path 1), the
@@ -463,10 +484,8 @@ static bool mlp_a8(const MlpW4 &a) { return a.gs == 64 && vnni_semantics(); }
 static size_t mlp_w4_scratch_main(const MlpW4 &a);
 
 static size_t mlp_part_bytes(const MlpW4 &a) {
-    return std::min(
-        a.part_cap,
-        std::max(w4_mfma_scratch_bytes((int)a.m, (int)a.inter, (int)a.k, true),
-                 w4_mfma_scratch_bytes((int)a.m, (int)a.n_out, (int)a.inter, false)));
+    return std::max(mlp_plan(a.m, a.inter, a.k, true, a.part_cap).bytes,
+                    mlp_plan(a.m, a.n_out, a.inter, false, a.part_cap).bytes);
 }
 
 // [path scratch | x' (m x k) | h' (m x inter)], the last two under W4A8 only.
@@ -480,9 +499,9 @@ static size_t mlp_w4_scratch_bytes(const MlpW4 &a) {
     return mlp_w4_with_a8(a, mlp_w4_scratch_main(a));
 }
 
-static size_t mlp_w4_scratch_main(const MlpW4 &a) {
+static size_t mlp_w4_scratch_route(const MlpW4 &a, int route, size_t part) {
     const size_t hb = up256((size_t)a.m * (size_t)a.inter * sizeof(float));
-    switch (mlp_w4_path(a)) {
+    switch (route) {
         case 0: return hb;
         case 3: {
             return hb + up256(limb_records_bytes((int)a.m, (int)a.k)) +
@@ -490,9 +509,14 @@ static size_t mlp_w4_scratch_main(const MlpW4 &a) {
                    std::max(limb_partials_bytes((int)a.m, (int)a.inter, (int)a.k, true),
                             limb_partials_bytes((int)a.m, (int)a.n_out, (int)a.inter, false));
         }
-        case 1: return hb + mlp_part_bytes(a);
+        case 1: return hb + part;
         default: return hb + up256(xq_bytes(a.m, a.k)) + xq_bytes(a.m, a.inter);
     }
+}
+
+static size_t mlp_w4_scratch_main(const MlpW4 &a) {
+    const int route = mlp_w4_path(a);
+    return mlp_w4_scratch_route(a, route, route == 1 ? mlp_part_bytes(a) : 0);
 }
 
 // out = [residual +] down(silu(gate(x)) * up(x)) with `ws` of at least
@@ -547,15 +571,14 @@ static int mlp_w4_run(const MlpW4 &a, void *ws, hipStream_t st) {
         return w4_limb(d, part, st);
     }
     if (path == 1) {
-        float *part = reinterpret_cast<float *>(static_cast<char *>(ws) + hb);
-        const size_t pb = mlp_part_bytes(a);
-        MfmaParams g = mfma_params(x, a.gate_w, a.gate_s, a.gate_b, h, m, inter, k, gs);
+        void *part = static_cast<char *>(ws) + hb;
+        QGemmParams g = qgemm_params(x, a.gate_w, a.gate_s, a.gate_b, h, m, inter, k, gs);
         g.w1 = a.up_w; g.s1 = a.up_s; g.b1 = a.up_b;
-        if ((rc = w4_mfma(g, EPI_SWIGLU, part, pb, st))) return rc;
+        if ((rc = qgemm(g, qgemm_plan(g, a.part_cap), part, st))) return rc;
         if (a8 && (rc = act_u8(h, ha, m, inter, st))) return rc;
-        MfmaParams d = mfma_params(hin, a.down_w, a.down_s, a.down_b, a.out, m, n_out, inter, gs);
+        QGemmParams d = qgemm_params(hin, a.down_w, a.down_s, a.down_b, a.out, m, n_out, inter, gs);
         d.res = a.residual;
-        return w4_mfma(d, a.residual ? EPI_RESID : EPI_PLAIN, part, pb, st);
+        return qgemm(d, qgemm_plan(d, a.part_cap), part, st);
     }
     uint32_t *xq = reinterpret_cast<uint32_t *>(static_cast<char *>(ws) + hb);
     uint32_t *hq = reinterpret_cast<uint32_t *>(static_cast<char *>(ws) + hb +
@@ -590,10 +613,11 @@ static int mlp_w4_run(const MlpW4 &a, void *ws, hipStream_t st) {
 // hipGetSymbolAddress and is the only form passed to kernels.
 constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
 
-// Bytes that the entry point counts for a batched projection of m rows: split-K
-// partials of 64-row tiles in about 512 blocks and, from 17 rows at K % 128 ==
-// 0, 8224 bytes per 16 rows and 128 of K.  The sizes it takes are a promise of
-// its header, so this count stays what it was, whatever the kernels use of it.
+// Scratch that the entry point counts for a shape.  The shapes it takes are a
+// promise of its header, so the count stays what it was, whatever the kernels
+// use of it: limb records and partials for 3..16 rows, and for a batched
+// projection the split-K partials of 64-row tiles in about 512 blocks plus, from
+// 17 rows at K % 128 == 0, 8224 bytes per 16 rows and 128 of K.
 static size_t noalloc_part_bytes(int64_t m, int64_t n, int64_t k, bool dual) {
     const int64_t tiles = (m + 15) / 16, mz = (tiles + std::min<int64_t>(tiles, 4) - 1) /
                                               std::min<int64_t>(tiles, 4);
@@ -602,6 +626,12 @@ static size_t noalloc_part_bytes(int64_t m, int64_t n, int64_t k, bool dual) {
     const int64_t klen = (steps + want - 1) / want * 128, splits = (k + klen - 1) / klen;
     const size_t pb = up256((size_t)(dual ? 2 : 1) * splits * m * n * sizeof(float));
     return pb + (m >= 17 && k % 128 == 0 ? (size_t)tiles * (k / 128) * 8224 : 0);
+}
+
+static size_t noalloc_count(const MlpW4 &a) {
+    const size_t part = std::max(noalloc_part_bytes(a.m, a.inter, a.k, true),
+                                 noalloc_part_bytes(a.m, a.n_out, a.inter, false));
+    return mlp_w4_with_a8(a, mlp_w4_scratch_route(a, mlp_w4_route(a, mlp_limb_takes(a)), part));
 }
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -856,9 +886,9 @@ int tb_swiglu_w4a32(const float *x, const uint8_t *gate_w, const float *gate_s,
         return generic(x, gate_w, gate_s, 0, gate_b, up_w, up_s, 0, up_b, nullptr, h, m, inter, k,
                        group_size, 4, (hipStream_t)stream);
     if (m >= mfma_min_m()) {
-        MfmaParams q = mfma_params(x, gate_w, gate_s, gate_b, h, m, inter, k, group_size);
+        QGemmParams q = qgemm_params(x, gate_w, gate_s, gate_b, h, m, inter, k, group_size);
         q.w1 = up_w; q.s1 = up_s; q.b1 = up_b;
-        return mfma_ws(q, EPI_SWIGLU, (hipStream_t)stream);
+        return qgemm_ws(q, (hipStream_t)stream);
     }
     WsLease lease;
     rc = workspace(xq_bytes(m, k), (hipStream_t)stream, lease);
@@ -896,19 +926,16 @@ int tb_fused_swiglu_mlp_w4a32_noalloc(const float *x, const uint8_t *gate_w,
             residual, out, m, k, inter, n_out, group_size, SIZE_MAX};
     int rc = mlp_w4_check(a, "fused_swiglu_mlp_w4a32_noalloc");
     if (rc || m == 0 || n_out == 0) return rc;
-    size_t need = 0;
-    if (mlp_w4_path(a) == 1) {
-        a.part_cap = std::max(noalloc_part_bytes(m, inter, k, true),
-                              noalloc_part_bytes(m, n_out, inter, false));
-        need = mlp_w4_with_a8(a, up256((size_t)m * (size_t)inter * sizeof(float)) + a.part_cap);
-    } else {
-        need = mlp_w4_scratch_bytes(a);
-    }
+    const size_t need = noalloc_count(a);
     TB_REQUIRE(need <= kNoAllocScratchBytes, TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: fused_swiglu_mlp_w4a32_noalloc: this shape needs " +
                    std::to_string(need) + " bytes of scratch; the static scratch holds " +
                    std::to_string(kNoAllocScratchBytes) +
                    " (use tb_fused_swiglu_mlp_w4a32, which allocates)");
+    // the batched projections get what h (and the W4A8 rows) leave of the scratch
+    a.part_cap = 0;
+    const size_t fixed = mlp_w4_scratch_bytes(a);
+    a.part_cap = (kNoAllocScratchBytes - std::min(fixed, kNoAllocScratchBytes)) & ~(size_t)255;
     void *ws = nullptr;
     if ((rc = noalloc_scratch(&ws))) return rc;
     return mlp_w4_run(a, ws, (hipStream_t)stream);
@@ -939,9 +966,9 @@ int tb_w4a32_gemv_xq(const float *x, const uint32_t *xq, const uint8_t *w_packed
                ">= 32 and K <= " + std::to_string(kMaxGemvK));
     if (m == 0 || n == 0) return TB_OK;
     if (m >= mfma_min_m()) {
-        MfmaParams q = mfma_params(x, w_packed, scales, bias, out, m, n, k, group_size);
+        QGemmParams q = qgemm_params(x, w_packed, scales, bias, out, m, n, k, group_size);
         q.res = residual;
-        return mfma_ws(q, residual ? EPI_RESID : EPI_PLAIN, (hipStream_t)stream);
+        return qgemm_ws(q, (hipStream_t)stream);
     }
     W4Params p = w4_params(x, w_packed, scales, bias, out, m, n, k, group_size);
     p.res = residual;
@@ -965,9 +992,9 @@ int tb_swiglu_w4a32_xq(const float *x, const uint32_t *xq, const uint8_t *gate_w
                ">= 32 and K <= " + std::to_string(kMaxGemvK));
     if (m == 0 || inter == 0) return TB_OK;
     if (m >= mfma_min_m()) {
-        MfmaParams q = mfma_params(x, gate_w, gate_s, gate_b, h, m, inter, k, group_size);
+        QGemmParams q = qgemm_params(x, gate_w, gate_s, gate_b, h, m, inter, k, group_size);
         q.w1 = up_w; q.s1 = up_s; q.b1 = up_b;
-        return mfma_ws(q, EPI_SWIGLU, (hipStream_t)stream);
+        return qgemm_ws(q, (hipStream_t)stream);
     }
     W4Params p = w4_params(x, gate_w, gate_s, gate_b, h, m, inter, k, group_size);
     p.w1 = up_w; p.s1 = up_s; p.b1 = up_b;
@@ -1008,10 +1035,10 @@ int tb_w8a32_linear(const float *x, const int8_t *w, const float *scales, int64_
     DenseParams p{};
     p.x = x; p.w0 = w; p.rs0 = scales; p.rs0_len = (int)s_len; p.b0 = bias; p.y = out;
     p.m = (int)m; p.n = (int)n; p.k = (int)k;
-    const size_t bytes = w8_scratch_bytes(p, m);
+    const QPlan pl = w8_plan(p, m);
     WsLease lease;
-    if (bytes && (rc = workspace(bytes, (hipStream_t)stream, lease))) return rc;
-    return w8_rows(p, m, lease.ptr, bytes, (hipStream_t)stream);
+    if (pl.bytes && (rc = workspace(pl.bytes, (hipStream_t)stream, lease))) return rc;
+    return w8_rows(p, pl, m, lease.ptr, (hipStream_t)stream);
 }
 
 int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float *gate_s,
@@ -1042,16 +1069,16 @@ int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float 
     // workspace: h, 16-byte aligned as x must be, then the batched projections'
     // scratch (d.x is null here: aligned like the h it will be)
     const size_t hb = up256((size_t)m * (size_t)inter * sizeof(float));
-    const size_t sb = std::max(w8_scratch_bytes(p, m), w8_scratch_bytes(d, m));
+    const QPlan pp = w8_plan(p, m), pd = w8_plan(d, m);
     hipStream_t st = (hipStream_t)stream;
     WsLease lease;
-    if ((rc = workspace(hb + sb, st, lease))) return rc;
+    if ((rc = workspace(hb + std::max(pp.bytes, pd.bytes), st, lease))) return rc;
     float *h = static_cast<float *>(lease.ptr);
     void *scratch = static_cast<char *>(lease.ptr) + hb;
     p.y = h;
     d.x = h;
-    if ((rc = w8_rows(p, m, scratch, sb, st))) return rc;
-    return w8_rows(d, m, scratch, sb, st);
+    if ((rc = w8_rows(p, pp, m, scratch, st))) return rc;
+    return w8_rows(d, pd, m, scratch, st);
 }
 
 }  // extern "C"

@@ -32,7 +32,6 @@
 #include "w4_gemv.hpp"
 #include "qgemm.hpp"
 #include "w4_limb.hpp"
-#include "w4_mfma.hpp"
 #include "v2_layout.hpp"
 #include "sample.hpp"
 
@@ -577,8 +576,7 @@ struct Decoder {
 
     // Scratch of a projection of up to m rows.
     size_t gemm_scratch(int m, int n, int k, bool pair) const {
-        return wbits == 8 ? qgemm_scratch_bytes(m, n, k, Q_W8, false, pair)
-                          : w4_mfma_scratch_upto(m, n, k, pair);
+        return qgemm_plan(m, n, k, wbits == 8 ? Q_W8 : Q_W4, wbits != 8, pair).bytes;
     }
 
     int prefill_alloc(int64_t n) {
@@ -628,7 +626,9 @@ struct Decoder {
                    const void *w2, const float *s2, const float *res, float *y, int m, int n,
                    int k, int &rc, uint8_t *rec_out = nullptr, const uint8_t *rec_in = nullptr) {
         const bool pair = w2 != nullptr;
-        if (!pf_limb || m < 3 || m > kLimbMaxM || !limb_shape_ok(m, n, k, pair)) return false;
+        if (!pf_limb || m < 3 || m > kLimbMaxM || !limb_shape_ok(m, n, k, pair) ||
+            !limb_wins((int64_t)n * k * (pair ? 2 : 1)))
+            return false;
         const size_t rb = up256(limb_records_bytes(m, k));
         if (rb + limb_partials_bytes(m, n, k, pair) > pf_limb_bytes) return false;
         LimbParams p{};
@@ -672,7 +672,7 @@ struct Decoder {
             QGemmParams q{};
             q.x = xin; q.w0 = w; q.s0 = s; q.b0 = b; q.w1 = w2; q.s1 = s2; q.res = res; q.y = y;
             q.m = m; q.n = n; q.k = k; q.fmt = Q_W8; q.s0_len = q.s1_len = n;
-            return qgemm(q, scratch, cap, st);
+            return qgemm(q, qgemm_plan(q, cap), scratch, st);
         }
         for (int r0 = 0; r0 < m; r0 += kMaxRowsPerPass) {
             DenseParams p{};
@@ -692,12 +692,17 @@ struct Decoder {
         if (wbits == 8) return rows_w8(xin, w, s, b, w2, s2, res, y, m, n, k, epi, pf_part,
                                        pf_part_bytes);
         if (limb_gemm(xin, w, s, b, w2, s2, res, y, m, n, k, rc)) return rc;
-        MfmaParams p{};
-        p.x = xin;
-        p.w0 = static_cast<const uint8_t *>(w); p.s0 = s; p.b0 = b;
-        p.w1 = static_cast<const uint8_t *>(w2); p.s1 = s2;
-        p.res = res; p.y = y; p.m = m; p.n = n; p.k = k; p.gshift = gshift(gs);
-        return w4_mfma(p, epi, pf_part, pf_part_bytes, st);
+        const QGemmParams q = w4_params(xin, w, s, b, w2, s2, res, y, m, n, k);
+        return qgemm(q, qgemm_plan(q, pf_part_bytes), pf_part, st);
+    }
+
+    QGemmParams w4_params(const float *xin, const void *w, const float *s, const float *b,
+                          const void *w2, const float *s2, const float *res, float *y, int m,
+                          int n, int k) const {
+        QGemmParams q{};
+        q.x = xin; q.w0 = w; q.s0 = s; q.b0 = b; q.w1 = w2; q.s1 = s2; q.res = res; q.y = y;
+        q.m = m; q.n = n; q.k = k; q.fmt = Q_W4; q.grouped = 1; q.gshift = gshift(gs);
+        return q;
     }
 
     // Positions start .. start + n - 1 attend every earlier position (the
@@ -734,20 +739,18 @@ struct Decoder {
             if (M <= 8 && limb_gemm(xr, lm_w, lm_s, nullptr, nullptr, nullptr, nullptr, y, M, V, H,
                                     rc))
                 return rc;
-            const size_t lb = w4_mfma_scratch_upto(64, V, H, false);
+            const size_t lb = qgemm_plan(64, V, H, Q_W4, true, false).bytes;
             if (!pf_lmpart && (rc = alloc(&pf_lmpart, lb))) return rc;
             for (int r0 = 0; r0 < M; r0 += 64) {
-                MfmaParams p{};
-                p.x = xr + (size_t)r0 * H;
-                p.w0 = static_cast<const uint8_t *>(lm_w); p.s0 = lm_s;
-                p.y = y + (size_t)r0 * V; p.m = std::min(64, M - r0); p.n = V; p.k = H;
-                p.gshift = gshift(gs);
-                if ((rc = w4_mfma(p, EPI_PLAIN, pf_lmpart, lb, st))) return rc;
+                const QGemmParams q =
+                    w4_params(xr + (size_t)r0 * H, lm_w, lm_s, nullptr, nullptr, nullptr, nullptr,
+                              y + (size_t)r0 * V, std::min(64, M - r0), V, H);
+                if ((rc = qgemm(q, qgemm_plan(q, lb), pf_lmpart, st))) return rc;
             }
             return TB_OK;
         }
         if (lmbits == 8 && qgemm_w8_wins(M, (int64_t)V * H)) {
-            const size_t lb = qgemm_scratch_bytes(64, V, H, Q_W8, false, false);
+            const size_t lb = qgemm_plan(64, V, H, Q_W8, false, false).bytes;
             if (!pf_lmpart && (rc = alloc(&pf_lmpart, lb))) return rc;
             for (int r0 = 0; r0 < M; r0 += 64)
                 if ((rc = rows_w8(xr + (size_t)r0 * H, lm_w, lm_s, nullptr, nullptr, nullptr,

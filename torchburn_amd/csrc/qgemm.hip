@@ -74,6 +74,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kSlab = 32;            // activation rows of one MFMA tile
 constexpr int kGroupBytes = 4096;    // one slab x 32 K: 2 steps x 2 limbs x 1 KiB
 constexpr int kRun = 512;            // K per level of the row-scale sums
+constexpr int kDirectGroups = 12;    // k_qdirect: K range of a block, 48 KiB of limbs
 constexpr int kPad = 128;            // K is padded to whole stages in the records
 
 // K slot e of a step's 8 holds element slot_elem(e): the order in which a dword
@@ -112,6 +113,7 @@ __device__ __forceinline__ h8 expand_w8(uint32_t d0, uint32_t d1) {
 }
 
 struct QArgs {
+    const float *x;        // activations (k_qdirect)
     const uint8_t *rec;    // split activations
     const float *inv;      // [splits][slabs * 32] 2^-e
     const uint8_t *w0, *w1;
@@ -315,6 +317,104 @@ struct QTile {
     }
 };
 
+// Consecutive tiles (row blocks of the same columns first) on one XCD: blocks
+// go to the 8 XCDs round robin, the grid is a multiple of 8.
+__device__ __forceinline__ int block_tile() {
+    const int per = gridDim.x >> 3;
+    return (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+}
+
+// The limbs of 8 consecutive elements a, b of a row, scaled by sc (2^e, negated
+// for the groups negated() names).  W4: slots in nibble order, those that meet
+// 16 x weights divided by 16.
+template <bool W4>
+__device__ __forceinline__ void limbs8(const f32x4 &a, const f32x4 &b, float sc, h8 &l1, h8 &l2) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int el = W4 ? slot_elem(j) : j;
+        const float v = el < 4 ? a[el & 3] : b[el & 3];
+        const float s = v * ((W4 && (j & 2)) ? sc * 0.0625f : sc);
+        const _Float16 u = (_Float16)s;
+        l1[j] = u;
+        l2[j] = fabsf(s) < INFINITY ? (_Float16)(s - (float)u) : (_Float16)0.f;
+    }
+}
+
+// The largest finite magnitude of a, b and mx.
+__device__ __forceinline__ float max_finite(float mx, const f32x4 &a, const f32x4 &b) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float u = fabsf(a[e]), v = fabsf(b[e]);
+        mx = fmaxf(mx, u < INFINITY ? u : 0.f);
+        mx = fmaxf(mx, v < INFINITY ? v : 0.f);
+    }
+    return mx;
+}
+
+// e of a row whose largest finite magnitude is mx: mx 2^e in [2^14, 2^15).
+__device__ __forceinline__ int row_exp(float mx) {
+    int E = 0;
+    (void)frexpf(mx, &E);   // mx = f 2^E, f in [0.5, 1)
+    return mx > 0.f ? min(15 - E, 126) : 0;
+}
+
+// The block's results, scaled by their rows' 2^-e (inv: of slab0's first row
+// on), to y or the split's partials.  Register r of lane (i, h) is row
+// 8 (r / 4) + 4 h + r % 4 of weight row i.
+template <int FMT, int MT, int NT, int SM, bool PAIR>
+__device__ __forceinline__ void store_tile(const QArgs &a, const QTile<FMT, MT, NT, SM, PAIR> &t,
+                                           const f32x16 (&acc)[MT][NT], int bx, int split,
+                                           int slab0, const float *inv) {
+    const bool split_k = a.splits > 1;
+    const size_t plane = (size_t)a.m * a.n;
+    float *y = a.y + (split_k ? (size_t)split * (PAIR ? 2 : 1) * plane : 0);
+    auto row_scale = [&](const float *s, int len, int c) {
+        return SM == 2 ? s[len > 1 ? c : 0] : 1.0f;
+    };
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int slab = slab0 + mt;
+        if (slab >= a.slabs) break;
+        f32x4 f[4];
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+            f[r4] = *reinterpret_cast<const f32x4 *>(inv + mt * kSlab + 8 * r4 + 4 * t.h);
+#pragma unroll
+        for (int nt = 0; nt < (PAIR ? 1 : NT); ++nt) {
+            const int c = t.col(bx, nt);
+            if (c >= a.n) continue;
+            const float rs0 = row_scale(a.s0, a.s0_len, c);
+            const float rs1 = PAIR ? row_scale(a.s1, a.s1_len, c) : 1.0f;
+            const float b0 = !split_k && a.b0 ? a.b0[c] : 0.f;
+            const float b1 = PAIR && !split_k && a.b1 ? a.b1[c] : 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = slab * kSlab + 8 * (r >> 2) + 4 * t.h + (r & 3);
+                if (row >= a.m) continue;
+                const size_t o = (size_t)row * a.n + c;
+                const float fr = f[r >> 2][r & 3];
+                const float g = acc[mt][nt][r] * fr * rs0;
+                if constexpr (PAIR) {
+                    const float u = acc[mt][NT - 1][r] * fr * rs1;
+                    if (split_k) {
+                        y[o] = g;
+                        y[plane + o] = u;
+                    } else {
+                        y[o] = silu(g + b0) * (u + b1);
+                    }
+                } else {
+                    float v = g;
+                    if (!split_k) {
+                        if (a.b0) v += b0;
+                        if (a.res) v += a.res[o];
+                    }
+                    y[o] = v;
+                }
+            }
+        }
+    }
+}
+
 template <int FMT, int MT, int NT, int SM, bool PAIR>
 __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
     using T = QTile<FMT, MT, NT, SM, PAIR>;
@@ -323,10 +423,7 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
     static_assert(!PAIR || NT == 2, "a pair's column tiles are gate and up");
     __shared__ __align__(16) uint8_t lds0[kStage];
     __shared__ __align__(16) uint8_t lds1[kStage];
-    // Consecutive tiles (row blocks of the same columns first) on one XCD:
-    // blocks go to the 8 XCDs round robin.
-    const int per = gridDim.x >> 3;
-    const int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+    const int tile = block_tile();
     if (tile >= a.mz * a.nbx * a.splits) return;
     const int mz = tile % a.mz, rest = tile / a.mz;
     const int bx = rest % a.nbx, split = rest / a.nbx;
@@ -376,62 +473,101 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
     }
     T::flush(acc, run);
 
-    // Register r of lane (i, h) is row 8 (r / 4) + 4 h + r % 4 of weight row i.
-    const bool split_k = a.splits > 1;
-    const size_t plane = (size_t)a.m * a.n;
-    float *y = a.y + (split_k ? (size_t)split * (PAIR ? 2 : 1) * plane : 0);
-    const float *inv = a.inv + (size_t)split * a.slabs * kSlab;
-    auto row_scale = [&](const float *s, int len, int c) {
-        return SM == 2 ? s[len > 1 ? c : 0] : 1.0f;
-    };
+    store_tile<FMT, MT, NT, SM, PAIR>(a, t, acc, bx, split, slab0,
+                                      a.inv + ((size_t)split * a.slabs + slab0) * kSlab);
+}
+
+// The same projection for few rows: the block builds the limbs of its 32 rows
+// itself, straight into LDS and while its first weights are on their way, 12
+// groups at a time, and needs no record kernel before it.  Up to 12 groups per
+// split x is read once and the loop has no barrier; a longer range (LONG, for
+// calls with little scratch) reads x once more before, for the rows' maxima.
+// Wave w converts rows 8 w .. 8 w + 7, eight lanes each.  Small calls are bound
+// by their launches: 41 x 904 x 1088 takes 8.9 us here, 12.4 with the record
+// kernel (FP32 MFMA with split K, which this replaced: 9.8), 16 x 4096 x 4096
+// 13.9 / 14.8 (14.7), 37 x 4805 x 1600 in v2 15.2 / 16.6 (19.3), 13 x 4605 x 1984
+// in INT8 12.5 / 13.8 (35 as GEMV passes).
+template <int FMT, int NT, int SM, bool PAIR, bool LONG>
+__global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
+    using T = QTile<FMT, 1, NT, SM, PAIR>;
+    constexpr int SG = T::SG, PC = kDirectGroups * 32 / 64;   // pieces of 8 per lane
+    extern __shared__ __align__(16) uint8_t lds[];             // min(slen, 12) groups
+    __shared__ float inv[kSlab];
+    const int tile = block_tile();
+    if (tile >= a.mz * a.nbx * a.splits) return;
+    const int mz = tile % a.mz, rest = tile / a.mz;
+    const int bx = rest % a.nbx, split = rest / a.nbx;
+    const int gb = split * a.slen, ge = min(gb + a.slen, a.groups);
+
+    T t(a);
+    t.rows(bx);
+    const int r = 8 * t.wave + (t.lane >> 3), row = mz * kSlab + r, c0 = t.lane & 7;
+    const float *xr = a.x + (size_t)min(row, a.m - 1) * a.k;
+    f32x4 xa[PC], xb[PC];
+    auto fetch = [&](int g0) {   // the lane's pieces of groups g0 .. g0 + 11
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-        const int slab = slab0 + mt;
-        if (slab >= a.slabs) break;
-        f32x4 f[4];
-#pragma unroll
-        for (int r4 = 0; r4 < 4; ++r4)
-            f[r4] = *reinterpret_cast<const f32x4 *>(inv + slab * kSlab + 8 * r4 + 4 * t.h);
-#pragma unroll
-        for (int nt = 0; nt < (PAIR ? 1 : NT); ++nt) {
-            const int c = t.col(bx, nt);
-            if (c >= a.n) continue;
-            const float rs0 = row_scale(a.s0, a.s0_len, c);
-            const float rs1 = PAIR ? row_scale(a.s1, a.s1_len, c) : 1.0f;
-            const float b0 = !split_k && a.b0 ? a.b0[c] : 0.f;
-            const float b1 = PAIR && !split_k && a.b1 ? a.b1[c] : 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = slab * kSlab + 8 * (r >> 2) + 4 * t.h + (r & 3);
-                if (row >= a.m) continue;
-                const size_t o = (size_t)row * a.n + c;
-                const float fr = f[r >> 2][r & 3];
-                const float g = acc[mt][nt][r] * fr * rs0;
-                if constexpr (PAIR) {
-                    const float u = acc[mt][NT - 1][r] * fr * rs1;
-                    if (split_k) {
-                        y[o] = g;
-                        y[plane + o] = u;
-                    } else {
-                        y[o] = silu(g + b0) * (u + b1);
-                    }
-                } else {
-                    float v = g;
-                    if (!split_k) {
-                        if (a.b0) v += b0;
-                        if (a.res) v += a.res[o];
-                    }
-                    y[o] = v;
-                }
+        for (int c = 0; c < PC; ++c) {
+            const int kk = g0 * 32 + 8 * (c0 + 8 * c);
+            xa[c] = xb[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (row < a.m && kk < min(ge * 32, a.k)) {
+                xa[c] = *reinterpret_cast<const f32x4 *>(xr + kk);
+                xb[c] = *reinterpret_cast<const f32x4 *>(xr + kk + 4);
             }
         }
+    };
+    float mx = 0.f;
+    for (int g = gb + kDirectGroups; LONG && g < ge; g += kDirectGroups) {
+        fetch(g);
+#pragma unroll
+        for (int c = 0; c < PC; ++c) mx = max_finite(mx, xa[c], xb[c]);
     }
+    fetch(gb);
+    typename T::Stage sa, sb;
+    t.load(gb, sa);
+#pragma unroll
+    for (int c = 0; c < PC; ++c) mx = max_finite(mx, xa[c], xb[c]);
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    const int e = row_exp(mx);
+    const float up = ldexpf(1.f, e);
+    if (c0 == 0) inv[r] = ldexpf(1.f, -e);
+    f32x16 acc[1][NT] = {}, run[1][NT] = {};
+    for (int g0 = gb; g0 < (LONG ? ge : gb + 1); g0 += kDirectGroups) {
+        const int g1 = LONG ? min(g0 + kDirectGroups, ge) : ge;
+        if (LONG && g0 > gb) {
+            fetch(g0);
+            __syncthreads();   // the last chunk's readers are done
+        }
+#pragma unroll
+        for (int c = 0; c < PC; ++c) {
+            const int p = c0 + 8 * c, g = p >> 2, q = p & 3;
+            if (g0 + g < g1) {
+                h8 l1, l2;
+                limbs8<FMT != Q_W8>(xa[c], xb[c], negated(g0 + g) ? -up : up, l1, l2);
+                uint8_t *d = lds + g * kGroupBytes + (q & 1) * 2048 + ((q >> 1) * 32 + r) * 16;
+                *reinterpret_cast<h8 *>(d) = l1;
+                *reinterpret_cast<h8 *>(d + 1024) = l2;
+            }
+        }
+        __syncthreads();
+        for (int g = g0; g < g1; g += 2 * SG) {
+            if (g + SG < ge) t.load(g + SG, sb);
+            t.compute(lds + (g - g0) * kGroupBytes, g, sa, acc, run);
+            if (g + SG >= g1) {   // an odd number of stages: the next chunk's first is in sb
+                if (LONG) sa = sb;
+                break;
+            }
+            if (g + 2 * SG < ge) t.load(g + 2 * SG, sa);
+            t.compute(lds + (g + SG - g0) * kGroupBytes, g + SG, sb, acc, run);
+        }
+        T::flush(acc, run);
+    }
+    store_tile<FMT, 1, NT, SM, PAIR>(a, t, acc, bx, split, mz, inv);
 }
 
 // The limbs of x [m, k] for one K split of 8 rows: slab s, group g at
 // rec + (s groups + g) 4096, then [step][limb][lane (i, h)][8 slots].  A thread
 // takes pieces of 8 elements of row t % 8; rows past m and K past k are 0.
-// W4: slots in nibble order, the ones that meet 16 x weights divided by 16.
 template <bool W4>
 __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
                                                  uint8_t *__restrict__ rec,
@@ -453,14 +589,6 @@ __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
         }
     };
     float mx = 0.f;
-    auto see = [&](const f32x4 &a, const f32x4 &b) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float u = fabsf(a[e]), v = fabsf(b[e]);
-            mx = fmaxf(mx, u < INFINITY ? u : 0.f);
-            mx = fmaxf(mx, v < INFINITY ? v : 0.f);
-        }
-    };
     f32x4 ra[PC], rb[PC];
 #pragma unroll
     for (int c = 0; c < PC; ++c) {
@@ -469,36 +597,24 @@ __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
         if (p < pieces) fetch(p, ra[c], rb[c]);
     }
 #pragma unroll
-    for (int c = 0; c < PC; ++c) see(ra[c], rb[c]);
+    for (int c = 0; c < PC; ++c) mx = max_finite(mx, ra[c], rb[c]);
     for (int p = (t >> 3) + PC * tpr; p < pieces; p += tpr) {
         f32x4 a, b;
         fetch(p, a, b);
-        see(a, b);
+        mx = max_finite(mx, a, b);
     }
 #pragma unroll
     for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
     if ((t & 63) < 8) red[t >> 6][t & 7] = mx;
     __syncthreads();
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t & 7]);
-    int E = 0;
-    (void)frexpf(mx, &E);   // mx = f 2^E, f in [0.5, 1)
-    const int e = mx > 0.f ? min(15 - E, 126) : 0;
+    const int e = row_exp(mx);
     const float up = ldexpf(1.f, e);
     if (t < 8) inv[(size_t)split * slabs * kSlab + row] = ldexpf(1.f, -e);
     auto put = [&](int p, const f32x4 &a, const f32x4 &b) {
         const int kk = k0 + 8 * p, g = kk >> 5, q = (kk >> 3) & 3;
-        const float sup = negated(g) ? -up : up;
         h8 l1, l2;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int el = W4 ? slot_elem(j) : j;
-            const float v = el < 4 ? a[el & 3] : b[el & 3];
-            const float s = v * ((W4 && (j & 2)) ? sup * 0.0625f : sup);
-            const _Float16 u = (_Float16)s;
-            const float r = s - (float)u;
-            l1[j] = u;
-            l2[j] = fabsf(s) < INFINITY ? (_Float16)r : (_Float16)0.f;
-        }
+        limbs8<W4>(a, b, negated(g) ? -up : up, l1, l2);
         uint8_t *d = rec + ((size_t)(row >> 5) * groups + g) * kGroupBytes +
                      (size_t)(q & 1) * 2048 + (size_t)((q >> 1) * 32 + (row & 31)) * 16;
         *reinterpret_cast<h8 *>(d) = l1;
@@ -557,18 +673,14 @@ __global__ __launch_bounds__(256) void k_qreduce(const float *__restrict__ part,
 constexpr int kCUs = 256;
 constexpr int kMaxSplits = 16;
 
-struct Plan {
-    int mt, nt, mz, nbx, splits, slen, slabs, groups;
-};
-
 size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-size_t rec_bytes(const Plan &pl) { return (size_t)pl.slabs * pl.groups * kGroupBytes; }
-size_t inv_bytes(const Plan &pl, int splits) {
+size_t rec_bytes(const QPlan &pl) { return (size_t)pl.slabs * pl.groups * kGroupBytes; }
+size_t inv_bytes(const QPlan &pl, int splits) {
     return up256((size_t)splits * pl.slabs * kSlab * sizeof(float));
 }
-size_t scratch_of(const Plan &pl, int splits, int m, int n, bool pair) {
-    return rec_bytes(pl) + inv_bytes(pl, splits) +
+size_t scratch_of(const QPlan &pl, int splits, bool direct, int m, int n, bool pair) {
+    return (direct ? 0 : rec_bytes(pl) + inv_bytes(pl, splits)) +
            (splits > 1 ? (size_t)splits * (pair ? 2 : 1) * (size_t)m * n * sizeof(float) : 0);
 }
 
@@ -591,9 +703,9 @@ constexpr Tile kTiles[] = {{1, 1, 0.77, 1.35, 0.25}, {1, 2, 1.95, 1.0, 0.5}, {2,
 // more outputs per wave have no room for the second sum of row scales; the
 // 128-row tile is for v1 weights (5% ahead of 64 rows at 512 rows and N = 28672,
 // since a weight's expansion serves twice the rows; a v2 lane holds more of its
-// stage and would spill).  splits == 0 in the result: no plan fits the scratch.
-Plan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
-    Plan pl{};
+// stage and would spill).  One K split on k_qdirect needs no scratch: some plan fits.
+QPlan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
+    QPlan pl{};
     pl.slabs = (m + kSlab - 1) / kSlab;
     pl.groups = (k + kPad - 1) / kPad * (kPad / 32);
     const int stages = pl.groups / 4;
@@ -612,10 +724,18 @@ Plan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
             const double rounds = std::max(1.0, ceil(blocks / t.grain) * t.grain);
             double us = len * std::max(rounds * t.busy * f, t.alone * fa) + 1.2 * ceil(blocks / 2);
             if (s > 1) us += 3.0 + (double)(pair ? 2 : 1) * s * m * n * 1.57e-6;
-            if (us < best && scratch_of(pl, s, m, n, pair) <= cap) {
-                best = us;
-                pl.mt = t.mt; pl.nt = t.nt; pl.mz = mz; pl.nbx = nbx;
-                pl.splits = s; pl.slen = len * 4;
+            for (int d = 0; d < 2; ++d) {
+                if (d && (t.mt > 1 || (t.nt == 2 && !pair))) continue;
+                // the record kernel, or every block's own conversion
+                const double ud =
+                    us + (d ? 1.0 + (len * 4 > kDirectGroups ? 0.7 : 0.25) * len * rounds : 5.0);
+                const size_t bytes = scratch_of(pl, s, d != 0, m, n, pair);
+                if (ud < best && bytes <= cap) {
+                    best = ud;
+                    pl.bytes = bytes;
+                    pl.mt = t.mt; pl.nt = t.nt; pl.mz = mz; pl.nbx = nbx;
+                    pl.splits = s; pl.slen = len * 4; pl.direct = d != 0;
+                }
             }
         }
     }
@@ -623,9 +743,24 @@ Plan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
 }
 
 template <int FMT, int SM>
-int launch(const QArgs &a, const Plan &pl, bool pair, hipStream_t st) {
+int launch(const QArgs &a, const QPlan &pl, bool pair, hipStream_t st) {
     const long tiles = (long)pl.mz * pl.nbx * pl.splits;
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
+    if (pl.direct) {
+        const size_t lds = (size_t)std::min(pl.slen, kDirectGroups) * kGroupBytes;
+#define TB_QDIRECT(LONG_)                                                                        \
+    do {                                                                                         \
+        if (pair)                                                                                \
+            hipLaunchKernelGGL((k_qdirect<FMT, 2, SM, true, LONG_>), grid, block, lds, st, a);   \
+        else                                                                                     \
+            hipLaunchKernelGGL((k_qdirect<FMT, 1, SM, false, LONG_>), grid, block, lds, st, a);  \
+    } while (0)
+        if (pl.slen > kDirectGroups) TB_QDIRECT(true);
+        else TB_QDIRECT(false);
+#undef TB_QDIRECT
+        TB_LAUNCHED();
+        return TB_OK;
+    }
 #define TB_QGO(MT_, NT_, PAIR_)                                                                  \
     hipLaunchKernelGGL((k_qgemm<FMT, MT_, NT_, SM, PAIR_>), grid, block, 0, st, a)
     if constexpr (FMT == Q_W4 && SM != 2) {   // see plan()
@@ -654,40 +789,36 @@ int launch(const QArgs &a, const Plan &pl, bool pair, hipStream_t st) {
 
 bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt) {
     if (m < 1 || n < 1 || k < 32 || k % (fmt == Q_V2 ? 64 : 32) != 0) return false;
-    return k <= (int64_t)1 << 24 && m < (int64_t)1 << 24 && n < (int64_t)1 << 30;
+    return k <= (int64_t)1 << 30 && m < (int64_t)1 << 24 && n < ((int64_t)1 << 31) - 512;
 }
 
-size_t qgemm_scratch_bytes(int m, int n, int k, int fmt, bool grouped, bool pair) {
-    const Plan pl = plan(m, n, k, fmt, grouped, pair, SIZE_MAX);
-    return scratch_of(pl, pl.splits, m, n, pair);
+QPlan qgemm_plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
+    return plan(m, n, k, fmt, grouped, pair, cap);
 }
 
-bool qgemm_fits(int64_t m, int64_t n, int64_t k, int fmt, bool grouped, bool pair, size_t cap) {
-    return qgemm_shape_ok(m, n, k, fmt) &&
-           plan((int)m, (int)n, (int)k, fmt, grouped, pair, cap).splits > 0;
-}
-
-int qgemm(const QGemmParams &p, void *scratch, size_t cap, hipStream_t st) {
+int qgemm(const QGemmParams &p, const QPlan &pl, void *scratch, hipStream_t st) {
     const bool pair = p.w1 != nullptr;
     TB_REQUIRE(qgemm_shape_ok(p.m, p.n, p.k, p.fmt), TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: batched projection needs K % 32 == 0");
-    const Plan pl = plan(p.m, p.n, p.k, p.fmt, p.grouped != 0, pair, cap);
-    TB_REQUIRE(pl.splits > 0, TB_ERR_UNSUPPORTED,
-               "TB_UNSUPPORTED: batched projection: scratch too small");
     uint8_t *rec = static_cast<uint8_t *>(scratch);
-    float *inv = reinterpret_cast<float *>(rec + rec_bytes(pl));
-    float *part = reinterpret_cast<float *>(rec + rec_bytes(pl) + inv_bytes(pl, pl.splits));
-    const dim3 pg((unsigned)(pl.slabs * 4), (unsigned)pl.splits);
-    const unsigned threads = pl.slen * 32 <= 1024 ? 256 : pl.slen * 32 <= 2048 ? 512 : 1024;
-    if (p.fmt == Q_W8)
-        hipLaunchKernelGGL((k_qsplit<false>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m, p.k,
-                           pl.slabs, pl.groups, pl.slen);
-    else
-        hipLaunchKernelGGL((k_qsplit<true>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m, p.k,
-                           pl.slabs, pl.groups, pl.slen);
-    TB_LAUNCHED();
+    float *inv = nullptr, *part = reinterpret_cast<float *>(rec);
+    if (!pl.direct) {
+        inv = reinterpret_cast<float *>(rec + rec_bytes(pl));
+        part = reinterpret_cast<float *>(rec + rec_bytes(pl) + inv_bytes(pl, pl.splits));
+    }
+    if (!pl.direct) {
+        const dim3 pg((unsigned)(pl.slabs * 4), (unsigned)pl.splits);
+        const unsigned threads = pl.slen * 32 <= 1024 ? 256 : pl.slen * 32 <= 2048 ? 512 : 1024;
+        if (p.fmt == Q_W8)
+            hipLaunchKernelGGL((k_qsplit<false>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m,
+                               p.k, pl.slabs, pl.groups, pl.slen);
+        else
+            hipLaunchKernelGGL((k_qsplit<true>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m,
+                               p.k, pl.slabs, pl.groups, pl.slen);
+        TB_LAUNCHED();
+    }
     QArgs a{};
-    a.rec = rec; a.inv = inv;
+    a.x = p.x; a.rec = rec; a.inv = inv;
     a.w0 = static_cast<const uint8_t *>(p.w0);
     a.w1 = static_cast<const uint8_t *>(p.w1);
     a.s0 = p.s0; a.s1 = p.s1; a.b0 = p.b0; a.b1 = p.b1; a.res = p.res;

@@ -30,21 +30,37 @@ struct QGemmParams {
 bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt);
 
 // Whether INT8 rows go to this kernel rather than to GEMV passes of 2 rows that
-// re-read the weights (elems of them): from 5 rows, or 3 on weights of 32 Mi
-// elements (us, passes against batched: 4096 x 4096 at 3 rows 12.2 / 13.6 and
-// at 5 17 / 14; 14336 x 4096 at 2 rows 14.0 / 22.7 and at 3 25.4 / 23.5; 4864 x
-// 896 at 4 rows 9.3 / 11.1).
+// re-read the weights (elems of them): from 4 rows, or 3 on weights of 32 Mi
+// elements (us, passes / batched: 4096 x 4096 at 3 rows 12.3 / 12.5, 14336 x 4096
+// at 2 rows 14.0 / 22.7 and at 3 25.4 / 23.5, 4864 x 896 at 4 rows 9.4 / 9.2).
 inline bool qgemm_w8_wins(int64_t m, int64_t elems) {
-    return m >= 5 || (m >= 3 && elems >= (int64_t)1 << 25);
+    return m >= 4 || (m >= 3 && elems >= (int64_t)1 << 25);
 }
 
-// Scratch of one call's fastest plan: the split activations and the split-K
-// partial sums.  A plan takes any `cap` that holds at least the activations
-// (qgemm_fits).
-size_t qgemm_scratch_bytes(int m, int n, int k, int fmt, bool grouped, bool pair);
-bool qgemm_fits(int64_t m, int64_t n, int64_t k, int fmt, bool grouped, bool pair, size_t cap);
+// Whether 3..16 INT4 rows with K % 128 == 0 stay on the small-batch kernel of
+// w4_limb.hip, which reads large weights faster (us, it / this one: 8 rows,
+// 14336 x 4096 17.9 / 20.3 and 4096 x 14336 16.8 / 21.5; at 4096 x 4096 12.7 / 13.0;
+// with its record and reduce kernels it is behind on smaller ones: 4 rows, 4864 x
+// 896 11.5 / 9.2, and 16 rows, 4096 x 4096 15.4 / 13.9).
+inline bool limb_wins(int64_t elems) { return elems > (int64_t)1 << 24; }
 
-// scratch: cap bytes, 256-byte aligned.
-int qgemm(const QGemmParams &p, void *scratch, size_t cap, hipStream_t st);
+// How a call runs: the block's tile, the K split and whether the blocks build
+// the activations' limbs themselves.
+struct QPlan {
+    int mt, nt, mz, nbx, splits, slen, slabs, groups;
+    bool direct;
+    size_t bytes;   // scratch: the activations' limbs and the split-K partial sums
+};
+
+// The fastest plan whose scratch is at most cap bytes (one with none exists).
+QPlan qgemm_plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap = SIZE_MAX);
+
+inline QPlan qgemm_plan(const QGemmParams &p, size_t cap = SIZE_MAX) {
+    return qgemm_plan(p.m, p.n, p.k, p.fmt, p.grouped != 0, p.w1 != nullptr, cap);
+}
+
+// y = epilogue(x . deq(w)^T): + bias (+ residual), or silu(x w0^T + b0) *
+// (x w1^T + b1) for a pair.  scratch: pl.bytes, 256-byte aligned.
+int qgemm(const QGemmParams &p, const QPlan &pl, void *scratch, hipStream_t st);
 
 }  // namespace tb

@@ -6,7 +6,7 @@
 // (packed_v2.rs:114-143) with f32_to_f16's round-to-nearest-even
 // (packed_v2.rs:66-105); k_dequant_v2 replaces dequantize_int4_grouped_v2
 // (python/torchburn/quantization.py:155-169).  The GEMV over the blocks is the
-// V2 form of k_w4_gemv / k_w4_mfma.
+// V2 form of k_w4_gemv / k_qgemm.
 //
 // W4A8 (gemv.rs:1353-1389): on hosts with AVX-512 VNNI the reference's group-64
 // GEMVs first quantize each activation row to bytes, s_x = max(max|x|, 1e-10) /
