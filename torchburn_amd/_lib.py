@@ -115,4 +115,6 @@ def check(rc: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(lib(), name)(*args))
+    rc = getattr(_lib or lib(), name)(*args)
+    if rc != TB_OK:
+        check(rc)

