@@ -38,6 +38,7 @@
 //     A chunk is one half of a block: its 16 nibble bytes come from five
 //     dword-aligned loads and a funnel shift, its scale from the block's two
 //     trailing bytes; the arithmetic is unchanged.
+#include "decode.hpp"
 #include "gemv_common.hpp"
 #include "tb_common.hpp"
 
@@ -306,9 +307,12 @@ __global__ __launch_bounds__(NW * 64) void k_w4_gemv(W4Params p, Layout L, Epi e
     reduce_and_store<G::V, J, M, DUAL, EPI>(v, red, sh, L, g.lane, g.wave, row0, e, in);
 }
 
-// Chunk records of x [m, k]: eight lanes per (row, 32-element chunk).
+// Chunk records of x [m, k]: eight lanes per (row, 32-element chunk).  st (a
+// layer step's state, or null) is set to position pos.
 __global__ __launch_bounds__(256) void k_xquant(const float *__restrict__ x,
-                                               uint32_t *__restrict__ xq, int m, int k) {
+                                               uint32_t *__restrict__ xq, int m, int k,
+                                               DecState *st, int pos) {
+    if (st && blockIdx.x == 0 && threadIdx.x == 0) *st = DecState{0, pos, 0, 0};
     const int c = k / 32;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int rec = t >> 3, sub = t & 7;
@@ -420,10 +424,11 @@ int dispatch_m(const W4Params &p, hipStream_t st) {
 
 }  // namespace
 
-int xquant(const float *x, uint32_t *xq, int m, int k, hipStream_t st) {
+int xquant(const float *x, uint32_t *xq, int m, int k, hipStream_t st, DecState *state, int pos) {
     const int n = m * (k / 32) * 8;   // 8 lanes per chunk record
     if (n == 0) return TB_OK;
-    hipLaunchKernelGGL(k_xquant, dim3((n + 255) / 256), dim3(256), 0, st, x, xq, m, k);
+    hipLaunchKernelGGL(k_xquant, dim3((n + 255) / 256), dim3(256), 0, st, x, xq, m, k,
+                       state, pos);
     TB_LAUNCHED();
     return TB_OK;
 }

@@ -73,6 +73,7 @@ struct W4Params {
 int w4_gemv(W4Params p, int epi, hipStream_t st);
 
 // Chunk records of x [m, k] (k % 32 == 0) into xq [m, 7, k/32, 4] (by quad).
-int xquant(const float *x, uint32_t *xq, int m, int k, hipStream_t st);
+int xquant(const float *x, uint32_t *xq, int m, int k, hipStream_t st,
+           struct DecState *state = nullptr, int pos = 0);   // state: also set to pos
 
 }  // namespace tb
