@@ -821,6 +821,7 @@ __global__ __launch_bounds__(256) void k_prefill_attn_mfma(const float *__restri
     const int last = start + (min(i0 + QT, NR) - 1) / G;   // last position any row sees
     const int ntiles = last / KT + 1;
     const int kt0 = blockIdx.z * tps, kt1 = min(ntiles, kt0 + tps);
+    if (kt0 >= ntiles) return;   // past every row's keys: the merge skips this split
     const float *kb = kc + (size_t)kvh * max_seq * HD, *vb = vc + (size_t)kvh * max_seq * HD;
     // A tile's K and V rows go global -> registers -> LDS; the next tile's
     // loads are in flight while the current one is multiplied (rows past
@@ -1044,21 +1045,76 @@ __global__ __launch_bounds__(256) void k_prefill_attn_mfma(const float *__restri
     }
 }
 
+// Key splits of the attention and the query rows per tile: which splits wrote a
+// partial for a row (those that start before its tile's last key).
+struct SplitShape {
+    int start, G, hq, M, tile, tps, rows, nsplit;   // keys per tile, tiles per split, rows per tile
+    __device__ __forceinline__ int used(int m, int h) const {
+        const int i0 = (m * G + h % G) / rows * rows;
+        const int last = start + (min(i0 + rows, M * G) - 1) / G;
+        return min(nsplit, (last / tile + tps) / tps);
+    }
+};
+
+// Combines up to kFewSplits key-range splits, one thread per float4 column of a
+// (row, head), every load in flight (two splits of 511 positions x 32 heads of
+// 128: 8.2 us; k_prefill_merge's block per (row, head) took 12.8 for 256).
+constexpr int kFewSplits = 8;
+template <int HD>
+__global__ __launch_bounds__(256) void k_prefill_merge_few(const float *__restrict__ part,
+                                                           const float *__restrict__ pml,
+                                                           float *__restrict__ out,
+                                                           SplitShape sh) {
+    constexpr int C4 = HD / 4, PB = 256 / C4;
+    const int c = threadIdx.x % C4;
+    const int64_t id = (int64_t)blockIdx.x * PB + threadIdx.x / C4;   // (row, head)
+    if (id >= (int64_t)sh.M * sh.hq) return;
+    const int m = (int)(id / sh.hq), h = (int)(id - (int64_t)m * sh.hq);
+    const int nv = sh.used(m, h);
+    const size_t plane = (size_t)sh.M * sh.hq;
+    float ms[kFewSplits], ls[kFewSplits];
+    float4 ov[kFewSplits];
+#pragma unroll
+    for (int s = 0; s < kFewSplits; ++s) {
+        const bool ok = s < nv;
+        const size_t row = (ok ? s : 0) * plane + (size_t)id;
+        ms[s] = ok ? pml[row * 2] : -INFINITY;
+        ls[s] = ok ? pml[row * 2 + 1] : 0.f;
+        ov[s] = ok ? reinterpret_cast<const float4 *>(part + row * HD)[c]
+                   : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float mx = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int s = 0; s < kFewSplits; ++s) mx = fmaxf(mx, ms[s]);
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int s = 0; s < kFewSplits; ++s) {
+        const float a = ms[s] == -INFINITY ? 0.f : expf(ms[s] - mx);
+        l = fmaf(ls[s], a, l);
+        o.x = fmaf(ov[s].x, a, o.x); o.y = fmaf(ov[s].y, a, o.y);
+        o.z = fmaf(ov[s].z, a, o.z); o.w = fmaf(ov[s].w, a, o.w);
+    }
+    const float inv = 1.0f / fmaxf(l, 1e-30f);
+    reinterpret_cast<float4 *>(out + (size_t)id * HD)[c] =
+        make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+}
+
 // Combines the key-range splits of one (row, head): M = max m_s,
 // l = sum l_s e^(m_s - M), o = sum o_s e^(m_s - M) / max(l, 1e-30).  Splits
-// past a row's last tile hold m = -inf and contribute nothing.  256 threads =
+// past the row tile's last key wrote nothing and are skipped.  256 threads =
 // SG split groups x HD / 4 float4 columns; each thread folds splits sg, sg +
 // SG, ... NB at a time (all NB loads in flight) with its own running max, and
 // the split groups combine through LDS.
 template <int HD>
 __global__ __launch_bounds__(256) void k_prefill_merge(const float *__restrict__ part,
                                                       const float *__restrict__ pml,
-                                                      float *__restrict__ out, int M, int hq,
-                                                      int nsplit) {
+                                                      float *__restrict__ out, SplitShape sh) {
+    const int M = sh.M, hq = sh.hq;
     constexpr int C4 = HD / 4, SG = 256 / C4, NB = 8;
     __shared__ float4 so[SG][C4];
     __shared__ float smx[SG], sl[SG];
     const int m = blockIdx.x, h = blockIdx.y, c = threadIdx.x % C4, sg = threadIdx.x / C4;
+    const int nsplit = sh.used(m, h);
     float mx = -INFINITY, l = 0.f;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int s0 = sg; s0 < nsplit; s0 += SG * NB) {
@@ -1273,19 +1329,25 @@ void launch_attn_mfma(int kg, dim3 grid, hipStream_t s, const float *q, const fl
 }  // namespace
 
 int prefill_attention_splits(int start, int M, int hq, int hkv) {
-    // 64 / kg-row tiles; about 256 blocks (one or two per CU at their LDS;
-    // TB_PREFILL_ATTN_BLOCKS overrides, measurement only), every split with at
-    // least one key tile
+    // 64 / kg-row tiles; about 768 blocks (up to three per CU at their LDS, so
+    // that the causal rows' uneven key counts even out), but two splits at most
+    // from 256 blocks on (Qwen2.5-0.5B prompt of 511 tokens, 112 blocks: one split
+    // per 256 blocks 3253 us, 768 3158; of 1024 tokens 5465 and 5101; eight
+    // Llama-3-8B layers, 1024 tokens 9581 and 9373; 511 tokens, 256 blocks, 4918,
+    // with two splits 4928, with three 4940).  Every split
+    // takes at least one key tile.  TB_PREFILL_ATTN_BLOCKS overrides (measurement
+    // only).
     static const int target = [] {
         const char *e = getenv("TB_PREFILL_ATTN_BLOCKS");
         const int v = e ? atoi(e) : 0;
-        return v > 0 ? v : 256;
+        return v > 0 ? v : 768;
     }();
     const int kg = mfma_attn_kg(M, hq / hkv);
     const int rows = 64 / kg, tile = mfma_attn_tile(kg);
     const int rtiles = (M * (hq / hkv) + rows - 1) / rows;
     const int tiles = (start + M - 1) / tile + 1;
-    const int want = (target + rtiles * hkv - 1) / (rtiles * hkv);
+    const int blocks = rtiles * hkv;
+    const int want = std::min((target + blocks - 1) / blocks, blocks >= 256 ? 2 : target);
     const int ns = std::max(1, std::min(want, tiles));
     const int tps = (tiles + ns - 1) / ns;
     return (tiles + tps - 1) / tps;
@@ -1321,12 +1383,19 @@ int launch_prefill_attention(const float *q, const float *kc, const float *vc, f
                              tps, part, pml);
     TB_LAUNCHED();
     if (nsplit > 1) {
-        if (hd == 128)
-            hipLaunchKernelGGL(k_prefill_merge<128>, dim3(M, hq), dim3(256), 0, s, part, pml, out,
-                               M, hq, nsplit);
-        else
-            hipLaunchKernelGGL(k_prefill_merge<64>, dim3(M, hq), dim3(256), 0, s, part, pml, out,
-                               M, hq, nsplit);
+        const SplitShape sh{start, hq / hkv, hq, M, kt, tps, rows, nsplit};
+        if (nsplit <= kFewSplits) {
+            const int pb = 256 / (hd / 4);
+            const dim3 mg((unsigned)(((int64_t)M * hq + pb - 1) / pb));
+            if (hd == 128)
+                hipLaunchKernelGGL(k_prefill_merge_few<128>, mg, dim3(256), 0, s, part, pml, out, sh);
+            else
+                hipLaunchKernelGGL(k_prefill_merge_few<64>, mg, dim3(256), 0, s, part, pml, out, sh);
+        } else if (hd == 128) {
+            hipLaunchKernelGGL(k_prefill_merge<128>, dim3(M, hq), dim3(256), 0, s, part, pml, out, sh);
+        } else {
+            hipLaunchKernelGGL(k_prefill_merge<64>, dim3(M, hq), dim3(256), 0, s, part, pml, out, sh);
+        }
         TB_LAUNCHED();
     }
     return TB_OK;
