@@ -175,12 +175,21 @@ struct Decoder {
         return TB_OK;
     }
 
-    // Device copy of a caller buffer (host or device memory).
+    // Device copy of a caller buffer (host or device memory), queued on the null
+    // stream: behind the caller's work there, which may still be producing it.
+    // The decoder's own stream does not wait for that stream: settle() first.
     template <class T>
     int upload(T **dst, const void *src, size_t bytes) {
         int rc = alloc(dst, bytes);
         if (rc) return rc;
         TB_HIP(hipMemcpy(*dst, src, bytes, hipMemcpyDefault));
+        return TB_OK;
+    }
+
+    // Copies between device buffers and fills on the null stream return before
+    // they are done; after this they are.
+    int settle() {
+        TB_HIP(hipStreamSynchronize(nullptr));
         return TB_OK;
     }
 
@@ -190,7 +199,8 @@ struct Decoder {
     int upload_f16_scaled(void **w_dst, float **s_dst, const void *w, const float *s, int64_t n,
                           int64_t k) {
         int rc;
-        if ((rc = upload(w_dst, w, wbytes(4, n, k))) || (rc = upload(s_dst, s, sbytes(4, n, k))))
+        if ((rc = upload(w_dst, w, wbytes(4, n, k))) ||
+            (rc = upload(s_dst, s, sbytes(4, n, k))) || (rc = settle()))
             return rc;
         if ((rc = round_scales_f16(*s_dst, n * (k / gs), st))) return rc;
         TB_HIP(hipStreamSynchronize(st));
@@ -1017,7 +1027,7 @@ int tb_decoder_create(const tb_decoder_config *cfg, const float *embed, const fl
         return bail(fail(TB_ERR_HIP, "stream/event creation failed"));
     if (hipHostMalloc((void **)&d->host_logits, (size_t)d->V * sizeof(float)) != hipSuccess) {
         d->host_logits = nullptr;
-        return fail(TB_ERR_MEMORY, "Out of memory allocating the decoder's host logits");
+        return bail(fail(TB_ERR_MEMORY, "Out of memory allocating the decoder's host logits"));
     }
     std::fill(d->host_logits, d->host_logits + d->V, 0.f);
     if (hipHostMalloc((void **)&d->hstate, sizeof(DecState)) != hipSuccess)
@@ -1064,6 +1074,7 @@ int tb_decoder_create(const tb_decoder_config *cfg, const float *embed, const fl
     if (hipMemset(d->kc, 0, kv) != hipSuccess || hipMemset(d->vc, 0, kv) != hipSuccess ||
         hipMemset(d->x, 0, d->H * 4) != hipSuccess)
         return bail(fail(TB_ERR_HIP, "initial clear failed"));
+    if ((rc = d->settle())) return bail(rc);
     *out = d;
     return TB_OK;
 }
@@ -1105,6 +1116,7 @@ int tb_decoder_set_layer(tb_decoder *d, int64_t layer, const float *in_norm, con
         return rc;
     }
     if (qkv_b && (rc = d->upload(&y.qkv_b, qkv_b, (size_t)d->tq * 4))) return rc;
+    if ((rc = d->settle())) return rc;
     y.set = true;
     return TB_OK;
 }
@@ -1486,6 +1498,8 @@ int tb_decoder_copy_kv(tb_decoder *d, int64_t layer, const float *k, const float
     TB_REQUIRE(seq_len >= 0 && seq_len <= src_max && seq_len <= d->max_seq, TB_ERR_VALUE,
                "KV cache copy out of bounds");
     // Source [hkv, src_max, hd] per layer (decoder.rs:479-523).
+    int rc = d->settle();   // device sources that the null stream is still writing
+    if (rc) return rc;
     const size_t row = (size_t)d->hd * 4;
     for (int hh = 0; hh < d->hkv; ++hh) {
         const size_t so = (size_t)hh * src_max * d->hd;
@@ -1540,7 +1554,7 @@ int tb_decoder_set_rope_tables(tb_decoder *d, const float *cos_t, const float *s
     TB_HIP(hipStreamSynchronize(d->st));
     TB_HIP(hipMemcpy(d->cos_t, cos_t, bytes, hipMemcpyDefault));
     TB_HIP(hipMemcpy(d->sin_t, sin_t, bytes, hipMemcpyDefault));
-    return TB_OK;
+    return d->settle();
 }
 
 int tb_decoder_time_greedy(tb_decoder *d, int64_t first_token, int64_t offset, int64_t n_steps,
