@@ -121,7 +121,7 @@ def test_w4_extreme_and_nonfinite_rows(cuda):
 
 @pytest.mark.parametrize("m,k,inter,gs", [
     (40, 2048, 4096, 32),    # limbs and partials within the scratch the entry point counts
-    (20, 4128, 64, 32)])     # limbs larger than that count: the FP32-MFMA form
+    (20, 4128, 64, 32)])     # limbs larger than that count: a plan that fits the rest
 def test_noalloc_mlp_at_17_rows_or_more(cuda, m, k, inter, gs):
     print(f"case qgemm noalloc m={m} k={k} inter={inter}", flush=True)
     g = synth.rng(73, m, k)
@@ -143,3 +143,35 @@ def test_noalloc_mlp_at_17_rows_or_more(cuda, m, k, inter, gs):
     ref = (a / (1 + np.exp(-a)) * u) @ dw.T + r
     for o in outs:
         assert np.abs(o - ref).max() / np.abs(ref).max() < 2e-6
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 300, 4096), (70, 515, 2080)])
+def test_w8_graphs_of_one_stream_run_side_by_side(cuda, m, n, k):
+    """A captured INT8 projection uses no workspace: two graphs captured on one
+    stream replay on two others at a time, beside eager calls on the first."""
+    print(f"case qgemm w8 graphs m={m} n={n} k={k}", flush=True)
+    g = synth.rng(79, m, n, k)
+    x = [synth.activations(g, m, k) for _ in range(3)]
+    w = g.integers(-127, 128, (n, k)).astype(np.int8)
+    s = (0.001 + 0.01 * g.random(n)).astype(np.float32)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    dx, dw, ds = [T(a) for a in x], T(w), T(s)
+    torch.cuda.synchronize()
+    cap, graphs, ys = torch.cuda.Stream(), [], []
+    for i in range(2):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[i], stream=cap):
+            ys.append(tb.w8a32_linear(dx[i], dw, ds))
+    st = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for rep in range(3):
+        for y in ys:
+            y.zero_()
+        torch.cuda.synchronize()
+        for i in range(2):
+            with torch.cuda.stream(st[i]):
+                graphs[i].replay()
+        with torch.cuda.stream(cap):
+            ye = tb.w8a32_linear(dx[2], dw, ds)
+        torch.cuda.synchronize()
+        for i, y in enumerate(ys + [ye]):
+            check(y.cpu().numpy(), x[i], w * s.astype(np.float64)[:, None])

@@ -407,8 +407,16 @@ static bool w8_batched(const DenseParams &p, int64_t m) {
            aligned(p.w0, 16) && aligned(p.w1, 16) && qgemm_shape_ok(m, p.n, p.k, Q_W8);
 }
 
-static QPlan w8_plan(const DenseParams &p, int64_t m) {
-    return w8_batched(p, m) ? qgemm_plan((int)m, p.n, p.k, Q_W8, false, p.w1 != nullptr) : QPlan{};
+static QPlan w8_plan(const DenseParams &p, int64_t m, size_t cap = SIZE_MAX) {
+    return w8_batched(p, m) ? qgemm_plan((int)m, p.n, p.k, Q_W8, false, p.w1 != nullptr, cap)
+                            : QPlan{};
+}
+
+static bool capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
 }
 
 static int w8_rows(const DenseParams &p, const QPlan &pl, int64_t m, void *scratch,
@@ -1035,10 +1043,19 @@ int tb_w8a32_linear(const float *x, const int8_t *w, const float *scales, int64_
     DenseParams p{};
     p.x = x; p.w0 = w; p.rs0 = scales; p.rs0_len = (int)s_len; p.b0 = bias; p.y = out;
     p.m = (int)m; p.n = (int)n; p.k = (int)k;
-    const QPlan pl = w8_plan(p, m);
+    // An INT8 projection runs without the workspace where a caller can tell: in a
+    // captured graph (replayed on any stream, beside others captured on this one)
+    // and where the device has no room for more.
+    QPlan pl = w8_plan(p, m);
     WsLease lease;
-    if (pl.bytes && (rc = workspace(pl.bytes, (hipStream_t)stream, lease))) return rc;
-    return w8_rows(p, pl, m, lease.ptr, (hipStream_t)stream);
+    hipStream_t st = (hipStream_t)stream;
+    if (pl.bytes && capturing(st)) pl = w8_plan(p, m, 0);
+    if (pl.bytes && (rc = workspace(pl.bytes, st, lease))) {
+        if (rc != TB_ERR_MEMORY) return rc;
+        (void)hipGetLastError();
+        pl = w8_plan(p, m, 0);
+    }
+    return w8_rows(p, pl, m, lease.ptr, st);
 }
 
 int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float *gate_s,
@@ -1069,10 +1086,18 @@ int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float 
     // workspace: h, 16-byte aligned as x must be, then the batched projections'
     // scratch (d.x is null here: aligned like the h it will be)
     const size_t hb = up256((size_t)m * (size_t)inter * sizeof(float));
-    const QPlan pp = w8_plan(p, m), pd = w8_plan(d, m);
+    QPlan pp = w8_plan(p, m), pd = w8_plan(d, m);
     hipStream_t st = (hipStream_t)stream;
     WsLease lease;
-    if ((rc = workspace(hb + std::max(pp.bytes, pd.bytes), st, lease))) return rc;
+    rc = workspace(hb + std::max(pp.bytes, pd.bytes), st, lease);
+    if (rc == TB_ERR_MEMORY && (pp.bytes || pd.bytes)) {   // h alone, as the GEMV passes need it
+        (void)hipGetLastError();
+        lease = WsLease();
+        pp = w8_plan(p, m, 0);
+        pd = w8_plan(d, m, 0);
+        rc = workspace(hb, st, lease);
+    }
+    if (rc) return rc;
     float *h = static_cast<float *>(lease.ptr);
     void *scratch = static_cast<char *>(lease.ptr) + hb;
     p.y = h;
