@@ -1,6 +1,7 @@
 // Small-batch grouped-INT4 projection Y[M, N] = X[M, K] . deq(W)^T for up to
 // 16 activation rows on f16 MFMA (v_mfma_f32_16x16x32_f16), reading every
-// weight byte once (the C ABI routes 3..16 rows here).
+// weight byte once.  3..16 rows come here on weights of more than 16 Mi elements,
+// and 3 and 4 rows whose K is past one GEMV pass; the rest takes qgemm.hip.
 //
 // Replaces the M > 1 path of the reference's w4a32_grouped_linear
 // (src/quantization/packed_v2.rs:557-624 -> gemm_w4a32_grouped,
