@@ -43,7 +43,8 @@ def check(y, x, w, bias=None, res=None):
 @pytest.mark.parametrize("m,n,k,gs,v2", [
     (17, 33, 160, 32, False), (32, 128, 128, 64, False), (33, 257, 2080, 32, False),
     (64, 300, 4096, 128, False), (65, 130, 96, 32, False), (130, 515, 1600, 64, False),
-    (19, 70, 224, 0, False), (48, 129, 64, 64, True), (200, 65, 1600, 64, True)])
+    (19, 70, 224, 0, False), (48, 129, 64, 64, True), (200, 65, 1600, 64, True),
+    (500, 2050, 4128, 32, False)])   # 128 record blocks: 4 rows each
 def test_w4_projection_edges(cuda, m, n, k, gs, v2):
     print(f"case qgemm w4 m={m} n={n} k={k} gs={gs} v2={v2}", flush=True)
     g = synth.rng(71, m, n, k)
@@ -66,6 +67,7 @@ def test_w4_projection_edges(cuda, m, n, k, gs, v2):
 @pytest.mark.parametrize("m,n,k,per_row", [
     (3, 8200, 4096, True),   # 32 Mi weights: from 3 rows
     (5, 33, 160, True), (32, 129, 992, False), (33, 300, 2080, True), (130, 260, 4160, True),
+    (497, 2050, 2080, True),   # 128 record blocks: 4 rows each
     (6, 40, 16416, True)])   # K past the streaming GEMV's range
 def test_w8_projection_edges(cuda, m, n, k, per_row):
     print(f"case qgemm w8 m={m} n={n} k={k}", flush=True)

@@ -46,9 +46,9 @@
 // -8 of the weights that this one replaced:
 //   Llama-3-8B gate/up pair, 512 rows, group 32    251 us, 479 TFLOP/s (958 in
 //                                                  MFMA work)
-//   Llama-3-8B MLP, 512 rows, group 64             939 -> 387 us
-//   64 rows, N = 14336, K = 4096, group 32         53.7 -> 32.0 us
-//   Llama-3-8B MLP in INT8, 128 rows               2561 -> 152 us, against GEMV
+//   Llama-3-8B MLP, 512 rows, group 64             942 -> 382 us
+//   64 rows, N = 14336, K = 4096, group 32         54.0 -> 31.0 us
+//   Llama-3-8B MLP in INT8, 128 rows               2559 -> 154 us, against GEMV
 //                                                  passes of 2 rows each
 // The error against 64 bits went from 6.2e-7 to 1.4e-7 for INT4 (activations
 // with large channels: the limbs follow each element's own size) and from
@@ -565,18 +565,22 @@ __global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
     store_tile<FMT, 1, NT, SM, PAIR>(a, t, acc, bx, split, mz, inv);
 }
 
-// The limbs of x [m, k] for one K split of 8 rows: slab s, group g at
+// The limbs of x [m, k] for one K split of R rows: slab s, group g at
 // rec + (s groups + g) 4096, then [step][limb][lane (i, h)][8 slots].  A thread
-// takes pieces of 8 elements of row t % 8; rows past m and K past k are 0.
-template <bool W4>
+// takes pieces of 8 elements of row t % R; rows past m and K past k are 0.
+// Bound by how many CUs take part (a row's largest magnitude ties its K range to
+// one block) against the length of the stores (16 R bytes).  us at 8 / 4 / 2 rows:
+// 64 x 4096 5.7 / 4.9 / 4.1, 128 rows of 4096 and 14336 8.2 / 6.4 / 6.4 on average,
+// 512 rows 11.6 / 9.6 / 12.4.
+template <bool W4, int R>
 __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
                                                  uint8_t *__restrict__ rec,
                                                  float *__restrict__ inv, int m, int k, int slabs,
                                                  int groups, int slen) {
     constexpr int PC = 4;   // pieces kept in registers
-    __shared__ float red[16][8];
-    const int t = threadIdx.x, tpr = blockDim.x >> 3;
-    const int row = blockIdx.x * 8 + (t & 7), split = blockIdx.y;
+    __shared__ float red[16][R];
+    const int t = threadIdx.x, tpr = blockDim.x / R, p0 = t / R;
+    const int row = blockIdx.x * R + t % R, split = blockIdx.y;
     const int k0 = split * slen * 32, k1 = min(k0 + slen * 32, groups * 32);
     const int pieces = (k1 - k0) >> 3;
     const float *xr = x + (size_t)row * k;
@@ -592,25 +596,25 @@ __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
     f32x4 ra[PC], rb[PC];
 #pragma unroll
     for (int c = 0; c < PC; ++c) {
-        const int p = (t >> 3) + c * tpr;
+        const int p = p0 + c * tpr;
         ra[c] = rb[c] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (p < pieces) fetch(p, ra[c], rb[c]);
     }
 #pragma unroll
     for (int c = 0; c < PC; ++c) mx = max_finite(mx, ra[c], rb[c]);
-    for (int p = (t >> 3) + PC * tpr; p < pieces; p += tpr) {
+    for (int p = p0 + PC * tpr; p < pieces; p += tpr) {
         f32x4 a, b;
         fetch(p, a, b);
         mx = max_finite(mx, a, b);
     }
 #pragma unroll
-    for (int o = 8; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if ((t & 63) < 8) red[t >> 6][t & 7] = mx;
+    for (int o = R; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((t & 63) < R) red[t >> 6][t % R] = mx;
     __syncthreads();
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t & 7]);
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t % R]);
     const int e = row_exp(mx);
     const float up = ldexpf(1.f, e);
-    if (t < 8) inv[(size_t)split * slabs * kSlab + row] = ldexpf(1.f, -e);
+    if (t < R) inv[(size_t)split * slabs * kSlab + row] = ldexpf(1.f, -e);
     auto put = [&](int p, const f32x4 &a, const f32x4 &b) {
         const int kk = k0 + 8 * p, g = kk >> 5, q = (kk >> 3) & 3;
         h8 l1, l2;
@@ -622,10 +626,10 @@ __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
     };
 #pragma unroll
     for (int c = 0; c < PC; ++c) {
-        const int p = (t >> 3) + c * tpr;
+        const int p = p0 + c * tpr;
         if (p < pieces) put(p, ra[c], rb[c]);
     }
-    for (int p = (t >> 3) + PC * tpr; p < pieces; p += tpr) {
+    for (int p = p0 + PC * tpr; p < pieces; p += tpr) {
         f32x4 a, b;
         fetch(p, a, b);
         put(p, a, b);
@@ -785,6 +789,9 @@ int launch(const QArgs &a, const QPlan &pl, bool pair, hipStream_t st) {
     return TB_OK;
 }
 
+// Rows of a k_qsplit block: 4, or 2 where that leaves fewer than 128 blocks.
+static int split_rows(const QPlan &pl) { return pl.slabs * 8 * pl.splits < 128 ? 2 : 4; }
+
 }  // namespace
 
 bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt) {
@@ -807,14 +814,21 @@ int qgemm(const QGemmParams &p, const QPlan &pl, void *scratch, hipStream_t st) 
         part = reinterpret_cast<float *>(rec + rec_bytes(pl) + inv_bytes(pl, pl.splits));
     }
     if (!pl.direct) {
-        const dim3 pg((unsigned)(pl.slabs * 4), (unsigned)pl.splits);
-        const unsigned threads = pl.slen * 32 <= 1024 ? 256 : pl.slen * 32 <= 2048 ? 512 : 1024;
-        if (p.fmt == Q_W8)
-            hipLaunchKernelGGL((k_qsplit<false>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m,
-                               p.k, pl.slabs, pl.groups, pl.slen);
-        else
-            hipLaunchKernelGGL((k_qsplit<true>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m,
-                               p.k, pl.slabs, pl.groups, pl.slen);
+        const int r = split_rows(pl);
+        const dim3 pg((unsigned)(pl.slabs * (kSlab / r)), (unsigned)pl.splits);
+        const int want = r * pl.slen;   // 4 pieces of 8 a thread
+        const unsigned threads = want <= 256 ? 256 : want <= 512 ? 512 : 1024;
+#define TB_QS(W4, R)                                                                      \
+    hipLaunchKernelGGL((k_qsplit<W4, R>), pg, dim3(threads), 0, st, p.x, rec, inv, p.m, p.k, \
+                       pl.slabs, pl.groups, pl.slen)
+        if (p.fmt == Q_W8) {
+            if (r == 2) TB_QS(false, 2);
+            else TB_QS(false, 4);
+        } else {
+            if (r == 2) TB_QS(true, 2);
+            else TB_QS(true, 4);
+        }
+#undef TB_QS
         TB_LAUNCHED();
     }
     QArgs a{};
