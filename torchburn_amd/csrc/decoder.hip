@@ -434,10 +434,16 @@ struct Decoder {
         return enqueue_tail(sampled);
     }
 
-    int capture(bool sampled, hipGraph_t *gr, hipGraphExec_t *ex) {
+    // A step or a batch reads every layer's weights.
+    int layers_set() const {
         for (int l = 0; l < L; ++l)
             TB_REQUIRE(layers[l].set, TB_ERR_VALUE,
                        "decoder layer " + std::to_string(l) + " was never set");
+        return TB_OK;
+    }
+
+    int capture(bool sampled, hipGraph_t *gr, hipGraphExec_t *ex) {
+        if (int unset = layers_set()) return unset;
         TB_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         int rc = enqueue_step(sampled);
         hipGraph_t g = nullptr;
@@ -785,8 +791,8 @@ struct Decoder {
     // returns them (decoder.rs:565-581); otherwise only the last position's.
     int prefill_batched(const int64_t *tokens, int64_t n, int64_t start,
                         float *rows_out = nullptr) {
-        int rc = prefill_alloc(n);
-        if (rc) return rc;
+        int rc = layers_set();
+        if (rc || (rc = prefill_alloc(n))) return rc;
         const int nq = (hq + 2 * hkv) * hd;
         // Host copy of the whole prompt, alive until the closing synchronize.
         std::vector<int> tok32(tokens, tokens + n);
