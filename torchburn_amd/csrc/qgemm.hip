@@ -9,15 +9,25 @@
 // row; here a weight byte is read once per block of activation rows.
 //
 // Arithmetic.  A stored weight is a small integer, exact in f16: the nibble q
-// becomes (1024 + q) - 1032 (one AND-OR and half a packed subtraction; a nibble
-// at bits 4-7 becomes 16 (q - 8), and its activation is divided by 16), an INT8
-// code b becomes (1024 + b + 128) - 1152.  An activation is scaled by a power
-// of two 2^e (the largest magnitude of its row in the block's K range lands in
-// [2^14, 2^15)) and split into two f16 limbs, x 2^e = h1 + h2 + r with
-// |r| <= 2^-22 |x 2^e| (or 2^-25 absolute, 2^-39 of the row's largest).  Both
-// limbs accumulate in one f32 MFMA chain over 32 elements, smaller limb first;
-// the chain's result takes the group scale and is added in f32, and the row's
-// 2^-e is applied once at the end.
+// becomes (1024 + q) - 1032, at bits 4-7 of its byte (64 + q) - 72 (one AND-OR
+// and half a packed subtraction), an INT8 code b becomes (1024 + b + 128) - 1152.
+// An activation is scaled by a power of two 2^e (the largest magnitude of its
+// row in the block's K range lands in [2^14, 2^15)) and split into two f16 limbs,
+// x 2^e = h1 + h2 + r with |r| <= 2^-22 |x 2^e| (or 2^-25 absolute, 2^-39 of the
+// row's largest).  Both limbs accumulate in one f32 MFMA chain over 32 elements,
+// smaller limb first; the chain's result takes the group scale and is added in
+// f32, and the row's 2^-e is applied once at the end.
+//
+// Rows of wide range.  Elements below 2^-17 of the row's largest keep fewer than
+// 22 bits, and where the large ones meet zero codes nothing else is left of the
+// sum.  A row in whose K range more than one in 16 nonzero elements is that small,
+// or whose largest is past 2^100, is marked by a negative 2^-e, and its slab of
+// 32 rows is multiplied from the f32 activations on f32 MFMA instead (wide_slab).
+// Under that share the small elements' error, 2^-39 of the largest each, stays
+// below the f32 rounding of the sum of the others, 15 times as many and each at
+// least 2^-17 of the largest.  N(0, 1) rows are marked from a channel of 5100 to
+// 10300 on.  Counting takes 0 to 0.3 us of a call (37 x 4805 x 1600 in v2 14.6 ->
+// 14.9 us, 64 x 14336 x 4096 31.2 -> 31.3).
 // Inf and NaN travel through the first limb, as in the reference's
 // unpack-and-fma.  An MFMA step rounds its sum down, which over a long row adds
 // up (a mean error of 1.3e-7 of the results' size at K = 14336): the records
@@ -78,7 +88,7 @@ constexpr int kDirectGroups = 12;    // k_qdirect: K range of a block, 48 KiB of
 constexpr int kPad = 128;            // K is padded to whole stages in the records
 
 // K slot e of a step's 8 holds element slot_elem(e): the order in which a dword
-// of nibbles expands; slots with (e & 2) hold 16 x weights.
+// of nibbles expands.
 __host__ __device__ constexpr int slot_elem(int e) { return (e >> 1) | ((e & 1) << 2); }
 
 // The groups held negated: every other one, starting anew each 4 groups (so
@@ -86,22 +96,24 @@ __host__ __device__ constexpr int slot_elem(int e) { return (e >> 1) | ((e & 1) 
 __host__ __device__ constexpr bool negated(int g) { return ((g ^ (g >> 2)) & 1) != 0; }
 
 // The nibble masks, in registers: behind a literal the compiler takes an AND
-// and an OR instead of one v_and_or_b32.
+// and an OR instead of one v_and_or_b32.  The f16 numbers that the nibbles are
+// put into, in both halves: 1024 (a unit in the last place of 1) for bits 0-3,
+// 64 (of 1/16) for bits 4-7.
 struct Masks {
-    uint32_t lo, hi;
+    uint32_t lo, hi, f_lo, f_hi;
 };
 __device__ __forceinline__ Masks nibble_masks() {
-    Masks k = {0x000F000Fu, 0x00F000F0u};
-    asm("" : "+v"(k.lo), "+v"(k.hi));
+    Masks k = {0x000F000Fu, 0x00F000F0u, 0x64006400u, 0x54005400u};
+    asm("" : "+v"(k.lo), "+v"(k.hi), "+s"(k.f_lo), "+s"(k.f_hi));
     return k;
 }
 
-__device__ __forceinline__ h8 expand_w4(uint32_t d, const Masks &k, uint32_t o) {
+__device__ __forceinline__ h8 expand_w4(uint32_t d, const Masks &k) {
     const uint32_t u = d >> 8;
-    const u32x4 v = {(d & k.lo) | o, (d & k.hi) | o, (u & k.lo) | o, (u & k.hi) | o};
-    const h8 c = {(_Float16)-1032.f, (_Float16)-1032.f, (_Float16)-1152.f, (_Float16)-1152.f,
-                  (_Float16)-1032.f, (_Float16)-1032.f, (_Float16)-1152.f, (_Float16)-1152.f};
-    return __builtin_bit_cast(h8, v) + c;
+    const u32x4 v = {(d & k.lo) | k.f_lo, (d & k.hi) | k.f_hi, (u & k.lo) | k.f_lo,
+                     (u & k.hi) | k.f_hi};
+    const _Float16 a = (_Float16)-1032.f, b = (_Float16)-72.f;
+    return __builtin_bit_cast(h8, v) + h8{a, a, b, b, a, a, b, b};
 }
 
 __device__ __forceinline__ h8 expand_w8(uint32_t d0, uint32_t d1) {
@@ -113,9 +125,9 @@ __device__ __forceinline__ h8 expand_w8(uint32_t d0, uint32_t d1) {
 }
 
 struct QArgs {
-    const float *x;        // activations (k_qdirect)
+    const float *x;        // activations (k_qdirect, wide_slab)
     const uint8_t *rec;    // split activations
-    const float *inv;      // [splits][slabs * 32] 2^-e
+    const float *inv;      // [splits][slabs * 32] 2^-e, negative for rows of wide range
     const uint8_t *w0, *w1;
     const float *s0, *s1, *b0, *b1, *res;
     float *y;              // [m, n], or the partials [splits][pair ? 2 : 1][m][n]
@@ -146,7 +158,6 @@ struct QTile {
     uint32_t vrow[NT];       // byte offset of the lane's row (v2)
     int chunks;              // 32-element chunks of a row
     Masks msk;
-    uint32_t magic;          // f16 1024 in both halves
 
     __device__ __forceinline__ QTile(const QArgs &aa) : a(aa) {
         lane = threadIdx.x & 63;
@@ -155,8 +166,6 @@ struct QTile {
         h = lane >> 5;
         chunks = a.k >> 5;
         msk = nibble_masks();
-        magic = 0x64006400u;
-        asm("" : "+s"(magic));
     }
 
     __device__ __forceinline__ int col(int bx, int nt) const {
@@ -249,8 +258,8 @@ struct QTile {
             }
             const auto s0 = __builtin_amdgcn_permlane32_swap(d[0], d[2], false, false);
             const auto s1 = __builtin_amdgcn_permlane32_swap(d[1], d[3], false, false);
-            B[0] = expand_w4((g & 1) ? s0[1] : s0[0], msk, magic);
-            B[1] = expand_w4((g & 1) ? s1[1] : s1[0], msk, magic);
+            B[0] = expand_w4((g & 1) ? s0[1] : s0[0], msk);
+            B[1] = expand_w4((g & 1) ? s1[1] : s1[0], msk);
         }
     }
 
@@ -304,6 +313,35 @@ struct QTile {
         }
     }
 
+    // Group g of the stage at g0 for one slab (MT 1) in f32: xg is element 16 h of
+    // the group in the lane's row, scaled by up.
+    __device__ __forceinline__ void compute_wide(const float *xg, float up, int g, int g0,
+                                                 const Stage &st, f32x16 (&acc)[1][NT],
+                                                 f32x16 (&run)[1][NT]) const {
+        f32x4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = reinterpret_cast<const f32x4 *>(xg)[j] * up;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            h8 B[2];
+            expand(st, nt, g, g0, B);
+            f32x16 D = {};
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const int el = 8 * u + (FMT == Q_W8 ? e : slot_elem(e));
+                    D = __builtin_amdgcn_mfma_f32_32x32x2f32(v[el >> 2][el & 3], (float)B[u][e], D,
+                                                             0, 0, 0);
+                }
+            const float s = scale(st, nt, g);
+            f32x16 &to = SM == 2 ? run[0][nt] : acc[0][nt];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) to[r] = fmaf(D[r], s, to[r]);
+            __builtin_amdgcn_sched_barrier(0);   // few registers rather than overlap
+        }
+    }
+
     __device__ __forceinline__ static void flush(f32x16 (&acc)[MT][NT], f32x16 (&run)[MT][NT]) {
         if constexpr (SM == 2) {
 #pragma unroll
@@ -325,19 +363,33 @@ __device__ __forceinline__ int block_tile() {
 }
 
 // The limbs of 8 consecutive elements a, b of a row, scaled by sc (2^e, negated
-// for the groups negated() names).  W4: slots in nibble order, those that meet
-// 16 x weights divided by 16.
+// for the groups negated() names), W4: slots in nibble order.  A row is of wide
+// range when the sum of `lack`, 15 for an element that keeps fewer than 22 bits
+// and -1 for another, is positive over its nonzero elements; here zeros count as
+// short too, an upper bound that ordinary rows keep negative in every wave, so
+// that only others pay for counting their zeros (zeros8).
 template <bool W4>
-__device__ __forceinline__ void limbs8(const f32x4 &a, const f32x4 &b, float sc, h8 &l1, h8 &l2) {
+__device__ __forceinline__ void limbs8(const f32x4 &a, const f32x4 &b, float sc, h8 &l1, h8 &l2,
+                                       int &lack) {
+    int full = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int el = W4 ? slot_elem(j) : j;
-        const float v = el < 4 ? a[el & 3] : b[el & 3];
-        const float s = v * ((W4 && (j & 2)) ? sc * 0.0625f : sc);
+        const float s = (el < 4 ? a[el & 3] : b[el & 3]) * sc;
         const _Float16 u = (_Float16)s;
         l1[j] = u;
         l2[j] = fabsf(s) < INFINITY ? (_Float16)(s - (float)u) : (_Float16)0.f;
+        full += fabsf(s) >= 0.25f;   // h2's last place is 2^-24 or more
     }
+    lack += 15 * 8 - 16 * full;
+    asm("" : "+v"(lack));   // summed here, not kept as 8 flags for later
+}
+
+__device__ __forceinline__ int zeros8(const f32x4 &a, const f32x4 &b) {
+    int z = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) z += (a[e] == 0.f) + (b[e] == 0.f);
+    return z;
 }
 
 // The largest finite magnitude of a, b and mx.
@@ -351,20 +403,30 @@ __device__ __forceinline__ float max_finite(float mx, const f32x4 &a, const f32x
     return mx;
 }
 
-// e of a row whose largest finite magnitude is mx: mx 2^e in [2^14, 2^15).
+// e of a row whose largest finite magnitude is mx: mx 2^e in [2^14, 2^15), past
+// 2^100 (a row of wide range) in [2^99, 2^100).
+constexpr float kLargest = 0x1p100f;
 __device__ __forceinline__ int row_exp(float mx) {
     int E = 0;
     (void)frexpf(mx, &E);   // mx = f 2^E, f in [0.5, 1)
-    return mx > 0.f ? min(15 - E, 126) : 0;
+    return mx > kLargest ? 100 - E : mx > 0.f ? min(15 - E, 126) : 0;
+}
+
+// 2^-e as stored: negative for a row of wide range.
+__device__ __forceinline__ float row_inv(int e, float mx, float score) {
+    const float v = ldexpf(1.f, -e);
+    return mx > kLargest || score > 0.f ? -v : v;
 }
 
 // The block's results, scaled by their rows' 2^-e (inv: of slab0's first row
 // on), to y or the split's partials.  Register r of lane (i, h) is row
-// 8 (r / 4) + 4 h + r % 4 of weight row i.
-template <int FMT, int MT, int NT, int SM, bool PAIR>
-__device__ __forceinline__ void store_tile(const QArgs &a, const QTile<FMT, MT, NT, SM, PAIR> &t,
-                                           const f32x16 (&acc)[MT][NT], int bx, int split,
-                                           int slab0, const float *inv) {
+// 8 (r / 4) + 4 h + r % 4 of weight row i.  Slabs with a row of wide range are
+// left out (unless WIDE) and returned, a bit each.
+template <bool WIDE, int FMT, int MT, int NT, int SM, bool PAIR>
+__device__ __forceinline__ int store_tile(const QArgs &a, const QTile<FMT, MT, NT, SM, PAIR> &t,
+                                          const f32x16 (&acc)[MT][NT], int bx, int split,
+                                          int slab0, const float *inv) {
+    int left = 0;
     const bool split_k = a.splits > 1;
     const size_t plane = (size_t)a.m * a.n;
     float *y = a.y + (split_k ? (size_t)split * (PAIR ? 2 : 1) * plane : 0);
@@ -379,6 +441,13 @@ __device__ __forceinline__ void store_tile(const QArgs &a, const QTile<FMT, MT, 
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4)
             f[r4] = *reinterpret_cast<const f32x4 *>(inv + mt * kSlab + 8 * r4 + 4 * t.h);
+        float least = f[0][0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) least = fminf(least, f[r >> 2][r & 3]);
+        if (!WIDE && __any(least < 0.f)) {
+            left |= 1 << mt;
+            continue;
+        }
 #pragma unroll
         for (int nt = 0; nt < (PAIR ? 1 : NT); ++nt) {
             const int c = t.col(bx, nt);
@@ -392,7 +461,7 @@ __device__ __forceinline__ void store_tile(const QArgs &a, const QTile<FMT, MT, 
                 const int row = slab * kSlab + 8 * (r >> 2) + 4 * t.h + (r & 3);
                 if (row >= a.m) continue;
                 const size_t o = (size_t)row * a.n + c;
-                const float fr = f[r >> 2][r & 3];
+                const float fr = fabsf(f[r >> 2][r & 3]);
                 const float g = acc[mt][nt][r] * fr * rs0;
                 if constexpr (PAIR) {
                     const float u = acc[mt][NT - 1][r] * fr * rs1;
@@ -413,6 +482,35 @@ __device__ __forceinline__ void store_tile(const QArgs &a, const QTile<FMT, MT, 
             }
         }
     }
+    return left;
+}
+
+// The results of one slab with rows of wide range, from the f32 activations: K
+// range and columns as the block's, 16 f32 MFMAs per group in place of 4 in f16 (8
+// times the matrix time; only such slabs pay it, after the block's other work).
+template <int FMT, int NT, int SM, bool PAIR>
+__device__ __forceinline__ void wide_slab(const QArgs &a, int bx, int split, int slab,
+                                          const float *inv) {
+    using T = QTile<FMT, 1, NT, SM, PAIR>;
+    constexpr int SG = T::SG;
+    const int gb = split * a.slen, ge = min(gb + a.slen, a.groups);
+    T t(a);
+    t.rows(bx);
+    // rows past m repeat the last one and are not stored
+    const float *xr = a.x + (size_t)min(slab * kSlab + t.i, a.m - 1) * a.k + 16 * t.h;
+    const float up = 1.0f / fabsf(inv[t.i]);   // a power of two
+    f32x16 acc[1][NT] = {}, run[1][NT] = {};
+#pragma unroll 1
+    for (int g = gb; g < ge; g += SG) {
+        typename T::Stage st;
+        t.load(g, st);
+#pragma unroll
+        for (int j = 0; j < SG; ++j)
+            if (g + j < t.chunks) t.compute_wide(xr + 32 * (size_t)(g + j), up, j, g, st, acc, run);
+        if (((g - gb) & (kRun / 32 - 1)) == kRun / 32 - SG) T::flush(acc, run);
+    }
+    T::flush(acc, run);
+    store_tile<true>(a, t, acc, bx, split, slab, inv);
 }
 
 template <int FMT, int MT, int NT, int SM, bool PAIR>
@@ -473,8 +571,12 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
     }
     T::flush(acc, run);
 
-    store_tile<FMT, MT, NT, SM, PAIR>(a, t, acc, bx, split, slab0,
-                                      a.inv + ((size_t)split * a.slabs + slab0) * kSlab);
+    const float *inv = a.inv + ((size_t)split * a.slabs + slab0) * kSlab;
+    const int left = store_tile<false>(a, t, acc, bx, split, slab0, inv);
+#pragma unroll 1
+    for (int mt = 0; left >> mt; ++mt)
+        if ((left >> mt) & 1)
+            wide_slab<FMT, NT, SM, PAIR>(a, bx, split, slab0 + mt, inv + mt * kSlab);
 }
 
 // The same projection for few rows: the block builds the limbs of its 32 rows
@@ -487,8 +589,10 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
 // kernel (FP32 MFMA with split K, which this replaced: 9.8), 16 x 4096 x 4096
 // 13.9 / 14.8 (14.7), 37 x 4805 x 1600 in v2 15.2 / 16.6 (19.3), 13 x 4605 x 1984
 // in INT8 12.5 / 13.8 (35 as GEMV passes).
+// (Three blocks a CU where the registers allow it, by the LDS they take.)
 template <int FMT, int NT, int SM, bool PAIR, bool LONG>
-__global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
+__global__ __launch_bounds__(256, NT == 1 && (FMT == Q_W8 || (FMT == Q_W4 && SM != 2)) ? 3 : 2)
+    void k_qdirect(QArgs a) {
     using T = QTile<FMT, 1, NT, SM, PAIR>;
     constexpr int SG = T::SG, PC = kDirectGroups * 32 / 64;   // pieces of 8 per lane
     extern __shared__ __align__(16) uint8_t lds[];             // min(slen, 12) groups
@@ -504,16 +608,16 @@ __global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
     const int r = 8 * t.wave + (t.lane >> 3), row = mz * kSlab + r, c0 = t.lane & 7;
     const float *xr = a.x + (size_t)min(row, a.m - 1) * a.k;
     f32x4 xa[PC], xb[PC];
+    auto piece = [&](int kk, f32x4 &va, f32x4 &vb) {
+        va = vb = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (row < a.m && kk < min(ge * 32, a.k)) {
+            va = *reinterpret_cast<const f32x4 *>(xr + kk);
+            vb = *reinterpret_cast<const f32x4 *>(xr + kk + 4);
+        }
+    };
     auto fetch = [&](int g0) {   // the lane's pieces of groups g0 .. g0 + 11
 #pragma unroll
-        for (int c = 0; c < PC; ++c) {
-            const int kk = g0 * 32 + 8 * (c0 + 8 * c);
-            xa[c] = xb[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (row < a.m && kk < min(ge * 32, a.k)) {
-                xa[c] = *reinterpret_cast<const f32x4 *>(xr + kk);
-                xb[c] = *reinterpret_cast<const f32x4 *>(xr + kk + 4);
-            }
-        }
+        for (int c = 0; c < PC; ++c) piece(g0 * 32 + 8 * (c0 + 8 * c), xa[c], xb[c]);
     };
     float mx = 0.f;
     for (int g = gb + kDirectGroups; LONG && g < ge; g += kDirectGroups) {
@@ -527,10 +631,9 @@ __global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
 #pragma unroll
     for (int c = 0; c < PC; ++c) mx = max_finite(mx, xa[c], xb[c]);
 #pragma unroll
-    for (int o = 1; o < 8; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    const int e = row_exp(mx);
-    const float up = ldexpf(1.f, e);
-    if (c0 == 0) inv[r] = ldexpf(1.f, -e);
+    for (int o = 1; o < 8; o <<= 1) mx = fmaxf(mx, shfl_xor_u(mx, o));
+    const float up = ldexpf(1.f, row_exp(mx));
+    int lack = 0;
     f32x16 acc[1][NT] = {}, run[1][NT] = {};
     for (int g0 = gb; g0 < (LONG ? ge : gb + 1); g0 += kDirectGroups) {
         const int g1 = LONG ? min(g0 + kDirectGroups, ge) : ge;
@@ -543,7 +646,8 @@ __global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
             const int p = c0 + 8 * c, g = p >> 2, q = p & 3;
             if (g0 + g < g1) {
                 h8 l1, l2;
-                limbs8<FMT != Q_W8>(xa[c], xb[c], negated(g0 + g) ? -up : up, l1, l2);
+                limbs8<FMT != Q_W8>(xa[c], xb[c], negated(g0 + g) ? -up : up, l1, l2, lack);
+                if (32 * g0 + 8 * p >= a.k) lack -= 15 * 8;   // padding
                 uint8_t *d = lds + g * kGroupBytes + (q & 1) * 2048 + ((q >> 1) * 32 + r) * 16;
                 *reinterpret_cast<h8 *>(d) = l1;
                 *reinterpret_cast<h8 *>(d + 1024) = l2;
@@ -562,7 +666,26 @@ __global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
         }
         T::flush(acc, run);
     }
-    store_tile<FMT, 1, NT, SM, PAIR>(a, t, acc, bx, split, mz, inv);
+    float sc = row < a.m ? (float)lack : 0.f;
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) sc += shfl_xor_u(sc, o);
+    if (__any(sc > 0.f)) {
+        int z = 0;
+#pragma unroll 1
+        for (int kk = gb * 32 + 8 * c0; kk < min(ge * 32, a.k); kk += 64) {
+            f32x4 va, vb;
+            piece(kk, va, vb);
+            z += zeros8(va, vb);
+        }
+        float zc = (float)(15 * z);
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) zc += shfl_xor_u(zc, o);
+        sc -= zc;
+    }
+    if (c0 == 0) inv[r] = row_inv(row_exp(mx), mx, sc);
+    __syncthreads();
+    if (store_tile<false>(a, t, acc, bx, split, mz, inv))
+        wide_slab<FMT, NT, SM, PAIR>(a, bx, split, mz, inv);
 }
 
 // The limbs of x [m, k] for one K split of R rows: slab s, group g at
@@ -573,12 +696,13 @@ __global__ __launch_bounds__(256, 2) void k_qdirect(QArgs a) {
 // 64 x 4096 5.7 / 4.9 / 4.1, 128 rows of 4096 and 14336 8.2 / 6.4 / 6.4 on average,
 // 512 rows 11.6 / 9.6 / 12.4.
 template <bool W4, int R>
-__global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
+__global__ __launch_bounds__(1024, 8) void k_qsplit(const float *__restrict__ x,
                                                  uint8_t *__restrict__ rec,
                                                  float *__restrict__ inv, int m, int k, int slabs,
                                                  int groups, int slen) {
     constexpr int PC = 4;   // pieces kept in registers
     __shared__ float red[16][R];
+    __shared__ int any_short;
     const int t = threadIdx.x, tpr = blockDim.x / R, p0 = t / R;
     const int row = blockIdx.x * R + t % R, split = blockIdx.y;
     const int k0 = split * slen * 32, k1 = min(k0 + slen * 32, groups * 32);
@@ -608,17 +732,20 @@ __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
         mx = max_finite(mx, a, b);
     }
 #pragma unroll
-    for (int o = R; o < 64; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    for (int o = R; o < 64; o <<= 1) mx = fmaxf(mx, shfl_xor_u(mx, o));
     if ((t & 63) < R) red[t >> 6][t % R] = mx;
+    if (t == 0) any_short = 0;
     __syncthreads();
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t % R]);
     const int e = row_exp(mx);
     const float up = ldexpf(1.f, e);
-    if (t < R) inv[(size_t)split * slabs * kSlab + row] = ldexpf(1.f, -e);
+    if (t < R) inv[(size_t)split * slabs * kSlab + row] = row_inv(e, mx, 0.f);
+    int lack = 0;
     auto put = [&](int p, const f32x4 &a, const f32x4 &b) {
         const int kk = k0 + 8 * p, g = kk >> 5, q = (kk >> 3) & 3;
         h8 l1, l2;
-        limbs8<W4>(a, b, negated(g) ? -up : up, l1, l2);
+        limbs8<W4>(a, b, negated(g) ? -up : up, l1, l2, lack);
+        if (kk >= k) lack -= 15 * 8;   // padding
         uint8_t *d = rec + ((size_t)(row >> 5) * groups + g) * kGroupBytes +
                      (size_t)(q & 1) * 2048 + (size_t)((q >> 1) * 32 + (row & 31)) * 16;
         *reinterpret_cast<h8 *>(d) = l1;
@@ -634,6 +761,31 @@ __global__ __launch_bounds__(1024) void k_qsplit(const float *__restrict__ x,
         fetch(p, a, b);
         put(p, a, b);
     }
+    float sc = row < m ? (float)lack : 0.f;
+#pragma unroll
+    for (int o = R; o < 64; o <<= 1) sc += shfl_xor_u(sc, o);
+    if (sc > 0.f) any_short = 1;
+    __syncthreads();
+    if (!any_short) return;
+    mx = 0.f;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t % R]);
+    __syncthreads();
+    int z = 0;
+#pragma unroll 1
+    for (int p = p0; p < pieces; p += tpr) {
+        f32x4 a, b;
+        fetch(p, a, b);
+        if (k0 + 8 * p < k) z += zeros8(a, b);
+    }
+    float zc = (float)(15 * z);
+#pragma unroll
+    for (int o = R; o < 64; o <<= 1) zc += shfl_xor_u(zc, o);
+    if ((t & 63) < R) red[t >> 6][t % R] = sc - zc;
+    __syncthreads();
+    if (t >= R) return;
+    sc = 0.f;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) sc += red[w][t];
+    inv[(size_t)split * slabs * kSlab + row] = row_inv(row_exp(mx), mx, sc);
 }
 
 // Sum of the split-K partials in split order, then the epilogue.  res may be y
