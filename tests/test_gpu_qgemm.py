@@ -177,3 +177,52 @@ def test_w8_graphs_of_one_stream_run_side_by_side(cuda, m, n, k):
         torch.cuda.synchronize()
         for i, y in enumerate(ys + [ye]):
             check(y.cpu().numpy(), x[i], w * s.astype(np.float64)[:, None])
+
+
+def graph_us(f, n=20):
+    """Microseconds of one call of f inside a captured graph of n."""
+    f()
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=torch.cuda.Stream()):
+        for _ in range(n):
+            f()
+    best = float("inf")
+    for _ in range(5):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        g.replay()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best
+
+
+@pytest.mark.parametrize("n,k", [(4096, 4096), (4096, 14336), (896, 4864), (1024, 512)])
+def test_captured_w8_is_no_slower_than_passes_of_two_rows(cuda, n, k):
+    """Without scratch the batched kernel and GEMV passes of 2 rows (4 us at the
+    least, and the weights read again) are both there: the faster one runs, within a
+    third (the batched kernel alone was 1.3 to 13 times the passes at these rows)."""
+    g = synth.rng(105, n, k)
+    w, s = synth.int8_weight(g, n, k)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(cuda)
+    dw, ds = T(w), T(s)
+    xs = {m: synth.activations(g, m, k) for m in (2, 4, 8, 32)}
+    two = graph_us(lambda x=T(xs[2]): tb.w8a32_linear(x, dw, ds))
+    for m in (4, 8, 32):
+        x = T(xs[m])
+        us = graph_us(lambda: tb.w8a32_linear(x, dw, ds))
+        print(f"case w8 captured m={m} n={n} k={k}: {us:.1f} us, a pass {two:.1f}", flush=True)
+        assert us < 4 / 3 * two * m / 2
+    out = {}
+    gr = torch.cuda.CUDAGraph()
+    dx = {m: T(x) for m, x in xs.items()}
+    with torch.cuda.graph(gr, stream=torch.cuda.Stream()):
+        for m, x in dx.items():
+            out[m] = tb.w8a32_linear(x, dw, ds)
+    for _ in range(3):
+        gr.replay()
+        torch.cuda.synchronize()
+        for m, y in out.items():
+            check(y.cpu().numpy(), xs[m], w.astype(np.float64) * s.astype(np.float64)[:, None])
+            y.zero_()

@@ -412,6 +412,18 @@ static QPlan w8_plan(const DenseParams &p, int64_t m, size_t cap = SIZE_MAX) {
                             : QPlan{};
 }
 
+// Without scratch the batched kernel has one K split, whose blocks are few where N
+// is small and long where K is: GEMV passes of 2 rows, 4 us each and 170 ns per Mi
+// weights, are taken where they are faster by the plan's model (captured calls in
+// us, batched / passes: 4096 x 4096 at 8 rows 57 / 26, at 32 rows 60 / 103; N 4096,
+// K 14336 at 8 rows 220 / 58, at 32 rows 229 / 231; 896 x 4864 at 8 rows 68 / 18).
+static QPlan w8_plan_bare(const DenseParams &p, int64_t m) {
+    const QPlan pl = w8_plan(p, m, 0);
+    const double passes = (double)((m + kMaxRowsPerPass - 1) / kMaxRowsPerPass) *
+                          (4.0 + 1.7e-7 * (double)p.n * p.k * (p.w1 ? 2 : 1));
+    return pl.mt && w8_fast(p.x, p.w0, p.k) && passes < pl.us ? QPlan{} : pl;
+}
+
 static bool capturing(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
@@ -1049,11 +1061,11 @@ int tb_w8a32_linear(const float *x, const int8_t *w, const float *scales, int64_
     QPlan pl = w8_plan(p, m);
     WsLease lease;
     hipStream_t st = (hipStream_t)stream;
-    if (pl.bytes && capturing(st)) pl = w8_plan(p, m, 0);
+    if (pl.bytes && capturing(st)) pl = w8_plan_bare(p, m);
     if (pl.bytes && (rc = workspace(pl.bytes, st, lease))) {
         if (rc != TB_ERR_MEMORY) return rc;
         (void)hipGetLastError();
-        pl = w8_plan(p, m, 0);
+        pl = w8_plan_bare(p, m);
     }
     return w8_rows(p, pl, m, lease.ptr, st);
 }
@@ -1093,8 +1105,8 @@ int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float 
     if (rc == TB_ERR_MEMORY && (pp.bytes || pd.bytes)) {   // h alone, as the GEMV passes need it
         (void)hipGetLastError();
         lease = WsLease();
-        pp = w8_plan(p, m, 0);
-        pd = w8_plan(d, m, 0);
+        pp = w8_plan_bare(p, m);
+        pd = w8_plan_bare(d, m);
         rc = workspace(hb, st, lease);
     }
     if (rc) return rc;

@@ -887,7 +887,7 @@ QPlan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
                     us + (d ? 1.0 + (len * 4 > kDirectGroups ? 0.7 : 0.25) * len * rounds : 5.0);
                 const size_t bytes = scratch_of(pl, s, d != 0, m, n, pair);
                 if (ud < best && bytes <= cap) {
-                    best = ud;
+                    best = pl.us = ud;
                     pl.bytes = bytes;
                     pl.mt = t.mt; pl.nt = t.nt; pl.mz = mz; pl.nbx = nbx;
                     pl.splits = s; pl.slen = len * 4; pl.direct = d != 0;

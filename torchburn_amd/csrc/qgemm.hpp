@@ -50,6 +50,7 @@ struct QPlan {
     int mt, nt, mz, nbx, splits, slen, slabs, groups;
     bool direct;
     size_t bytes;   // scratch: the activations' limbs and the split-K partial sums
+    double us;      // the cost model's time
 };
 
 // The fastest plan whose scratch is at most cap bytes (one with none exists).
