@@ -114,6 +114,7 @@ int workspace(size_t bytes, hipStream_t st, WsLease &out) {
         TB_HIP(hipThreadExchangeStreamCaptureMode(&mode));
         const hipError_t e = hipMalloc(&p, sz);
         TB_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+        if (e != hipSuccess) (void)hipGetLastError();   // ours: not the caller's next call's
         TB_HIP(e);
         if (sc->ptr) sc->retired.push_back(sc->ptr);
         sc->ptr = p;
@@ -177,11 +178,46 @@ static QPlan mlp_plan(int64_t m, int64_t n, int64_t k, bool pair, size_t cap) {
     return qgemm_plan((int)m, (int)n, (int)k, Q_W4, true, pair, cap);
 }
 
+static size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Scratch that a batched projection always gets along with: the split-K partials of
+// 64-row tiles in about 512 blocks plus, from 17 rows at K % 128 == 0, 8224 bytes
+// per 16 rows and 128 of K.
+static size_t part_bytes(int64_t m, int64_t n, int64_t k, bool dual) {
+    if (m < 1 || n < 1 || k < 1) return 0;
+    const int64_t tiles = (m + 15) / 16, mz = (tiles + std::min<int64_t>(tiles, 4) - 1) /
+                                              std::min<int64_t>(tiles, 4);
+    const int64_t blocks = (n + 63) / 64 * (dual ? 2 : 1) * mz, steps = (k + 127) / 128;
+    const int64_t want = std::max<int64_t>(1, std::min((512 + blocks - 1) / blocks, steps));
+    const int64_t klen = (steps + want - 1) / want * 128, splits = (k + klen - 1) / klen;
+    const size_t pb = up256((size_t)(dual ? 2 : 1) * splits * m * n * sizeof(float));
+    return pb + (m >= 17 && k % 128 == 0 ? (size_t)tiles * (k / 128) * 8224 : 0);
+}
+
+// A lease of need(cap) bytes, the batched projections' scratch at most cap: as much
+// as the fastest plan takes where the device has room, else `least`, else none.
+template <class Need>
+static int workspace_capped(Need need, size_t least, hipStream_t st, WsLease &lease) {
+    int rc = TB_OK;
+    for (const size_t cap : {SIZE_MAX, least, (size_t)0}) {
+        const size_t bytes = need(cap);
+        rc = bytes ? workspace(bytes, st, lease) : TB_OK;
+        if (rc != TB_ERR_MEMORY) return rc;
+        lease = WsLease();
+    }
+    return rc;
+}
+
 // The batched projection with its scratch in the library workspace.
 static int qgemm_ws(const QGemmParams &p, hipStream_t st) {
     WsLease lease;
-    const QPlan pl = qgemm_plan(p);
-    int rc = pl.bytes ? workspace(pl.bytes, st, lease) : TB_OK;
+    QPlan pl{};
+    int rc = workspace_capped(
+        [&](size_t cap) {
+            pl = qgemm_plan(p, cap);
+            return pl.bytes;
+        },
+        part_bytes(p.m, p.n, p.k, p.w1 != nullptr), st, lease);
     if (rc) return rc;
     return qgemm(p, pl, lease.ptr, st);
 }
@@ -258,8 +294,6 @@ std::atomic<int> g_vnni{0};
 
 bool vnni_semantics() { return g_vnni.load(std::memory_order_relaxed) != 0; }
 
-static size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
-
 // One INT4 projection y = x . deq(W)^T (+ bias) (+ residual) over m rows, with
 // the weights as v1 nibbles + f32 scales or as v2 blocks.  Under W4A8
 // semantics (group 64) each row of x is first replaced by its byte
@@ -282,21 +316,23 @@ static int linear_w4(const float *x, const uint8_t *w, const float *s, bool v2,
     const size_t xb = a8 ? up256((size_t)m * (size_t)k * sizeof(float)) : 0;
     const int epi = res ? EPI_RESID : EPI_PLAIN;
     const bool mf = !lb && !any_shape && m >= mfma_min_m();
-    const QPlan pl = mf ? qgemm_plan((int)m, (int)n, (int)k, v2 ? Q_V2 : Q_W4,
-                                     v2 || scale_mode == 0, false)
-                        : QPlan{};
-    const size_t rest = any_shape ? 0
-                        : lb ? up256(limb_records_bytes((int)m, (int)k)) +
-                                   limb_partials_bytes((int)m, (int)n, (int)k, false)
-                        : mf ? pl.bytes
-                             : xq_bytes(m, k);
+    QPlan pl{};
+    const auto need = [&](size_t cap) -> size_t {
+        if (mf)
+            pl = qgemm_plan((int)m, (int)n, (int)k, v2 ? Q_V2 : Q_W4, v2 || scale_mode == 0, false,
+                            cap);
+        return xb + (any_shape ? 0
+                     : lb ? up256(limb_records_bytes((int)m, (int)k)) +
+                                limb_partials_bytes((int)m, (int)n, (int)k, false)
+                     : mf ? pl.bytes
+                          : xq_bytes(m, k));
+    };
     const float *xin = x;
     void *tail = nullptr;
-    int rc;
     WsLease lease;
-    if (xb + rest) {
-        if ((rc = workspace(xb + rest, st, lease))) return rc;
-        void *ws = lease.ptr;
+    int rc = workspace_capped(need, part_bytes(m, n, k, false), st, lease);
+    if (rc) return rc;
+    if (void *ws = lease.ptr) {
         if (a8) {
             if ((rc = act_u8(x, static_cast<float *>(ws), m, k, st))) return rc;
             xin = static_cast<const float *>(ws);
@@ -635,22 +671,11 @@ constexpr size_t kNoAllocScratchBytes = (size_t)16 << 20;
 
 // Scratch that the entry point counts for a shape.  The shapes it takes are a
 // promise of its header, so the count stays what it was, whatever the kernels
-// use of it: limb records and partials for 3..16 rows, and for a batched
-// projection the split-K partials of 64-row tiles in about 512 blocks plus, from
-// 17 rows at K % 128 == 0, 8224 bytes per 16 rows and 128 of K.
-static size_t noalloc_part_bytes(int64_t m, int64_t n, int64_t k, bool dual) {
-    const int64_t tiles = (m + 15) / 16, mz = (tiles + std::min<int64_t>(tiles, 4) - 1) /
-                                              std::min<int64_t>(tiles, 4);
-    const int64_t blocks = (n + 63) / 64 * (dual ? 2 : 1) * mz, steps = (k + 127) / 128;
-    const int64_t want = std::max<int64_t>(1, std::min((512 + blocks - 1) / blocks, steps));
-    const int64_t klen = (steps + want - 1) / want * 128, splits = (k + klen - 1) / klen;
-    const size_t pb = up256((size_t)(dual ? 2 : 1) * splits * m * n * sizeof(float));
-    return pb + (m >= 17 && k % 128 == 0 ? (size_t)tiles * (k / 128) * 8224 : 0);
-}
-
+// use of it: limb records and partials for 3..16 rows, part_bytes() for a batched
+// projection.
 static size_t noalloc_count(const MlpW4 &a) {
-    const size_t part = std::max(noalloc_part_bytes(a.m, a.inter, a.k, true),
-                                 noalloc_part_bytes(a.m, a.n_out, a.inter, false));
+    const size_t part = std::max(part_bytes(a.m, a.inter, a.k, true),
+                                 part_bytes(a.m, a.n_out, a.inter, false));
     return mlp_w4_with_a8(a, mlp_w4_scratch_route(a, mlp_w4_route(a, mlp_limb_takes(a)), part));
 }
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
@@ -925,13 +950,19 @@ int tb_fused_swiglu_mlp_w4a32(const float *x, const uint8_t *gate_w, const float
                               const float *down_b, const float *residual, float *out,
                               int64_t m, int64_t k, int64_t inter, int64_t n_out,
                               int64_t group_size, void *stream) {
-    const MlpW4 a{x, gate_w, gate_s, gate_b, up_w, up_s, up_b, down_w, down_s, down_b,
-                  residual, out, m, k, inter, n_out, group_size, SIZE_MAX};
+    MlpW4 a{x, gate_w, gate_s, gate_b, up_w, up_s, up_b, down_w, down_s, down_b,
+            residual, out, m, k, inter, n_out, group_size, SIZE_MAX};
     int rc = mlp_w4_check(a, "fused_swiglu_mlp_w4a32");
     if (rc || m == 0 || n_out == 0) return rc;
     hipStream_t st = (hipStream_t)stream;
     WsLease lease;
-    if ((rc = workspace(mlp_w4_scratch_bytes(a), st, lease))) return rc;
+    rc = workspace_capped(
+        [&](size_t cap) {
+            a.part_cap = cap;
+            return mlp_w4_scratch_bytes(a);
+        },
+        std::max(part_bytes(m, inter, k, true), part_bytes(m, n_out, inter, false)), st, lease);
+    if (rc) return rc;
     return mlp_w4_run(a, lease.ptr, st);
 }
 
@@ -1064,7 +1095,6 @@ int tb_w8a32_linear(const float *x, const int8_t *w, const float *scales, int64_
     if (pl.bytes && capturing(st)) pl = w8_plan_bare(p, m);
     if (pl.bytes && (rc = workspace(pl.bytes, st, lease))) {
         if (rc != TB_ERR_MEMORY) return rc;
-        (void)hipGetLastError();
         pl = w8_plan_bare(p, m);
     }
     return w8_rows(p, pl, m, lease.ptr, st);
@@ -1103,7 +1133,6 @@ int tb_fused_swiglu_mlp_w8a32(const float *x, const int8_t *gate_w, const float 
     WsLease lease;
     rc = workspace(hb + std::max(pp.bytes, pd.bytes), st, lease);
     if (rc == TB_ERR_MEMORY && (pp.bytes || pd.bytes)) {   // h alone, as the GEMV passes need it
-        (void)hipGetLastError();
         lease = WsLease();
         pp = w8_plan_bare(p, m);
         pd = w8_plan_bare(d, m);
