@@ -56,6 +56,29 @@ def test_prompts_one_after_another(cuda, wkind, lmkind, lengths):
     dec.close()
 
 
+@pytest.mark.parametrize("wkind", [4, 8])
+def test_same_prompt_same_bits(cuda, wkind):
+    """A prompt's logits do not depend on the prompts before it: 70 rows, whose
+    gate/up plan takes more scratch than any of 256 rows, before and after 700."""
+    print(f"case same prompt wkind={wkind}", flush=True)
+    cfg = dict(num_layers=2, hidden=512, intermediate=2048, num_heads=8, num_kv_heads=2,
+               head_dim=64, vocab=1000, eps=1e-6, rope_theta=1e6, qkv_bias=True)
+    dec = decoder_from_weights(synth.decoder_weights(cfg, 93, wkind, wkind, 32), cfg,
+                               group_size=32, max_seq_len=800)
+    g = np.random.default_rng(93)
+    short, long = ([int(t) for t in g.integers(0, cfg["vocab"], k)] for k in (70, 700))
+
+    def logits(toks):
+        dec.reset_kv_cache()
+        dec.prefill_tokens(toks, 0)
+        return np.array(dec.get_logits())
+
+    first = logits(short)
+    logits(long)
+    assert np.array_equal(logits(short), first)
+    dec.close()
+
+
 @pytest.mark.parametrize("lmkind,n", [(8, 2), (8, 7), (8, 70), (32, 5)])
 def test_int8_verify_rows(cuda, lmkind, n):
     print(f"case int8 verify lmkind={lmkind} n={n}", flush=True)

@@ -593,9 +593,21 @@ struct Decoder {
     size_t pf_part_bytes = 0;
     int *pf_tok = nullptr;
 
-    // Scratch of a projection of up to m rows.
-    size_t gemm_scratch(int m, int n, int k, bool pair) const {
-        return qgemm_plan(m, n, k, wbits == 8 ? Q_W8 : Q_W4, wbits != 8, pair).bytes;
+    // Scratch of the batched projections: what the fastest plans take at any row
+    // count, so that a prompt's plans, and with them its logits' bits, are the same
+    // whatever prompts came before.
+    size_t gemm_scratch() const {
+        size_t b = 0;
+        auto add = [&](int m, int n, int k, bool pair) {
+            b = std::max(b, qgemm_plan(m, n, k, wbits == 8 ? Q_W8 : Q_W4, wbits != 8, pair).bytes);
+        };
+        for (int m = 32; m <= kPrefillRows; m += 32) {
+            add(m, tq, H, false);
+            add(m, H, hq * hd, false);
+            add(m, I, H, true);
+            add(m, H, I, false);
+        }
+        return b;
     }
 
     int prefill_alloc(int64_t n) {
@@ -603,10 +615,7 @@ struct Decoder {
         while (R < kPrefillRows && R < n) R *= 2;
         if (R <= pf_rows_cap) return TB_OK;
         const size_t nq = (size_t)(hq + 2 * hkv) * hd;
-        size_t part = gemm_scratch(R, (int)nq, H, false);
-        part = std::max(part, gemm_scratch(R, H, hq * hd, false));
-        part = std::max(part, gemm_scratch(R, I, H, true));
-        part = std::max(part, gemm_scratch(R, H, I, false));
+        if (!pf_part) pf_part_bytes = gemm_scratch();
         // 3..16 rows (verify_tokens, short chunks) take the small-batch
         // projection: records + split partials of the largest of its shapes
         size_t lb = 0;
@@ -624,12 +633,12 @@ struct Decoder {
             (rc = alloc(&pf_qkv, (size_t)R * nq * 4)) ||
             (rc = alloc(&pf_q, (size_t)R * hq * hd * 4)) ||
             (rc = alloc(&pf_a, (size_t)R * hq * hd * 4)) || (rc = alloc(&pf_h, (size_t)R * I * 4)) ||
-            (rc = alloc(&pf_part, part)) || (rc = alloc(&pf_tok, (size_t)R * 4)) ||
+            (!pf_part && (rc = alloc(&pf_part, pf_part_bytes))) ||
+            (rc = alloc(&pf_tok, (size_t)R * 4)) ||
             (lb && !pf_limb && (rc = alloc(&pf_limb, lb))) ||
             (lb && !pf_hrec && (rc = alloc(&pf_hrec, limb_records_bytes(kLimbMaxM, I)))))
             return rc;
         pf_limb_bytes = lb;
-        pf_part_bytes = part;
         pf_rows_cap = R;
         return TB_OK;
     }
