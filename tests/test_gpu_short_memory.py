@@ -3,10 +3,13 @@ scratch of their fastest plan only where it is there, and run with less, or with
 none, where it is not."""
 import contextlib
 
+import numpy as np
 import pytest
 import torch
 
 import torchburn_amd as tb
+from torchburn_amd import synth
+from torchburn_amd.decoder import decoder_from_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +90,30 @@ def test_int8_mlp(cuda):
     s = [torch.rand(n, device="cuda", generator=g) * 1e-3 for n in (inter, inter, k)]
     same(lambda: tb.fused_swiglu_mlp_w8a32(x, w[0], s[0], None, w[1], s[1], None, w[2], s[2],
                                            None), cuda, 110)
+
+
+@pytest.mark.parametrize("wkind,mb,n", [
+    (4, 300, 700),   # an arena and the buffers of 256 rows would fit, not those of 1024
+    (4, 190, 700), (8, 60, 40)])   # ... 256 rows, or fewer than a chunk: step by step
+def test_prompt_and_verify(cuda, wkind, mb, n):
+    print(f"case short memory prompt wkind={wkind} left={mb} n={n}", flush=True)
+    cfg = dict(num_layers=1, hidden=4096, intermediate=14336, num_heads=32, num_kv_heads=8,
+               head_dim=128, vocab=1000, eps=1e-6, rope_theta=1e6, qkv_bias=True)
+    w = synth.decoder_weights(cfg, 95, wkind, wkind, 32)
+    g = np.random.default_rng(95)
+    warm, toks = ([int(t) for t in g.integers(0, cfg["vocab"], k)] for k in (2, n))
+
+    def run(dec):
+        dec.prefill_tokens(toks, 0)
+        return np.array(dec.get_logits()), np.array(dec.verify_tokens(n, toks[:5]))
+
+    out = []
+    for mem in (None, mb):
+        dec = decoder_from_weights(w, cfg, group_size=32, max_seq_len=n + 8)
+        for i, t in enumerate(warm):
+            dec._step(t, i, True)
+        with left(cuda, mem) if mem else contextlib.nullcontext():
+            out.append(run(dec))
+        dec.close()
+    for want, got in zip(*out):
+        assert np.abs(got - want).max() / np.abs(want).max() < 2e-4

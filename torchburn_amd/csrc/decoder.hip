@@ -127,6 +127,9 @@ struct Decoder {
         }
         if (st) (void)hipStreamSynchronize(st);
         for (void *p : allocs) (void)hipFree(p);
+        if (pf_slab) (void)hipFree(pf_slab);
+        if (pf_attn) (void)hipFree(pf_attn);
+        if (pf_rows) (void)hipFree(pf_rows);
         if (hstate) (void)hipHostFree(hstate);
         if (host_logits) (void)hipHostFree(host_logits);
         if (ev0) (void)hipEventDestroy(ev0);
@@ -142,13 +145,31 @@ struct Decoder {
     char *arena = nullptr;
     size_t arena_left = 0;
 
-    int raw_alloc(void **q, size_t bytes) {
+    static int device_alloc(void **q, size_t bytes) {
         hipError_t e = hipMalloc(q, bytes);
-        if (e != hipSuccess)
-            return fail(e == hipErrorOutOfMemory ? TB_ERR_MEMORY : TB_ERR_HIP,
-                        "Out of memory allocating " + std::to_string(bytes >> 20) +
-                            " MB for the decoder on the GPU: " + hipGetErrorString(e));
-        allocs.push_back(*q);
+        if (e == hipSuccess) return TB_OK;
+        (void)hipGetLastError();   // ours: not the caller's next call's
+        return fail(e == hipErrorOutOfMemory ? TB_ERR_MEMORY : TB_ERR_HIP,
+                    "Out of memory allocating " + std::to_string(bytes >> 20) +
+                        " MB for the decoder on the GPU: " + hipGetErrorString(e));
+    }
+
+    int raw_alloc(void **q, size_t bytes) {
+        int rc = device_alloc(q, bytes);
+        if (!rc) allocs.push_back(*q);
+        return rc;
+    }
+
+    // A buffer of at least `bytes` in place of *p, which idle work may have used.
+    template <class T>
+    int regrow(T **p, size_t *have, size_t bytes) {
+        if (bytes <= *have) return TB_OK;
+        void *q = nullptr;
+        int rc = device_alloc(&q, bytes);
+        if (rc) return rc;
+        if (*p) (void)hipFree(*p);   // waits for the device
+        *p = static_cast<T *>(q);
+        *have = bytes;
         return TB_OK;
     }
 
@@ -163,7 +184,13 @@ struct Decoder {
         } else {
             if (bytes > arena_left) {
                 void *a = nullptr;
-                if ((rc = raw_alloc(&a, kArena))) return rc;
+                rc = raw_alloc(&a, kArena);
+                if (rc == TB_ERR_MEMORY) {   // no room for an arena: the buffer alone
+                    if ((rc = raw_alloc(&q, bytes))) return rc;
+                    *p = static_cast<T *>(q);
+                    return TB_OK;
+                }
+                if (rc) return rc;
                 arena = static_cast<char *>(a);
                 arena_left = kArena;
             }
@@ -586,8 +613,13 @@ struct Decoder {
     // and lm_head as a step would.  The buffers hold the longest chunk seen,
     // rounded up to a power of two from 256 rows: 1024 rows fill the GEMMs' tiles
     // (a 511-token Llama-3-8B prompt: 24.7 ms in chunks of 256, 21.4 ms in one).
+    // Where the device has no room for them the chunks are smaller, down to 256
+    // rows, and where it has none for those the prompt goes step by step.
     static constexpr int kPrefillRows = 1024;
+    static constexpr int kPrefillLeast = 256;
     int pf_rows_cap = 0;
+    char *pf_slab = nullptr;   // pf_x .. pf_h and pf_tok, one allocation
+    size_t pf_slab_bytes = 0;
     float *pf_x = nullptr, *pf_xn = nullptr, *pf_qkv = nullptr, *pf_q = nullptr,
           *pf_a = nullptr, *pf_h = nullptr, *pf_part = nullptr;
     size_t pf_part_bytes = 0;
@@ -610,37 +642,72 @@ struct Decoder {
         return b;
     }
 
-    int prefill_alloc(int64_t n) {
-        int R = 256;
-        while (R < kPrefillRows && R < n) R *= 2;
+    // The row buffers of chunks of R rows.
+    int prefill_rows(int R) {
         if (R <= pf_rows_cap) return TB_OK;
-        const size_t nq = (size_t)(hq + 2 * hkv) * hd;
-        if (!pf_part) pf_part_bytes = gemm_scratch();
-        // 3..16 rows (verify_tokens, short chunks) take the small-batch
-        // projection: records + split partials of the largest of its shapes
-        size_t lb = 0;
-        for (int m = 3; wbits == 4 && m <= kLimbMaxM; ++m) {
-            auto need = [&](int n, int k, bool pair) -> size_t {
-                if (!limb_shape_ok(m, n, k, pair)) return 0;
-                return up256(limb_records_bytes(m, k)) + limb_partials_bytes(m, n, k, pair);
-            };
-            lb = std::max({lb, need((int)nq, H, false), need(H, hq * hd, false), need(I, H, true),
-                           need(H, I, false)});
-            if (m <= 8 && lmbits == 4) lb = std::max(lb, need(V, H, false));
+        const size_t nq = (size_t)(hq + 2 * hkv) * hd, qd = (size_t)hq * hd;
+        const size_t cols[7] = {(size_t)H, (size_t)H, nq, qd, qd, (size_t)I, 1};
+        size_t total = 0;
+        for (size_t c : cols) total += up256(c * R * 4);
+        int rc = regrow(&pf_slab, &pf_slab_bytes, total);
+        if (rc) return rc;
+        float **const at[6] = {&pf_x, &pf_xn, &pf_qkv, &pf_q, &pf_a, &pf_h};
+        char *p = pf_slab;
+        for (int i = 0; i < 6; ++i) {
+            *at[i] = reinterpret_cast<float *>(p);
+            p += up256(cols[i] * R * 4);
         }
-        int rc;
-        if ((rc = alloc(&pf_x, (size_t)R * H * 4)) || (rc = alloc(&pf_xn, (size_t)R * H * 4)) ||
-            (rc = alloc(&pf_qkv, (size_t)R * nq * 4)) ||
-            (rc = alloc(&pf_q, (size_t)R * hq * hd * 4)) ||
-            (rc = alloc(&pf_a, (size_t)R * hq * hd * 4)) || (rc = alloc(&pf_h, (size_t)R * I * 4)) ||
-            (!pf_part && (rc = alloc(&pf_part, pf_part_bytes))) ||
-            (rc = alloc(&pf_tok, (size_t)R * 4)) ||
-            (lb && !pf_limb && (rc = alloc(&pf_limb, lb))) ||
-            (lb && !pf_hrec && (rc = alloc(&pf_hrec, limb_records_bytes(kLimbMaxM, I)))))
-            return rc;
-        pf_limb_bytes = lb;
+        pf_tok = reinterpret_cast<int *>(p);
         pf_rows_cap = R;
         return TB_OK;
+    }
+
+    // The key-split partials of the attention over n positions from start, in
+    // chunks of R.
+    int prefill_partials(int64_t n, int64_t start, int R) {
+        size_t b = 0;
+        for (int64_t c0 = 0; c0 < n; c0 += R) {
+            const int M = (int)std::min<int64_t>(R, n - c0);
+            b = std::max(b, prefill_attention_scratch(
+                                M, hq, hd,
+                                prefill_attention_splits((int)(start + c0), M, hq, hkv)));
+        }
+        return regrow(&pf_attn, &pf_attn_bytes, b);
+    }
+
+    // Everything that a prompt of n positions from start needs, in chunks of *rows.
+    int prefill_alloc(int64_t n, int64_t start, int *rows) {
+        int rc;
+        if (!pf_part) {
+            pf_part_bytes = gemm_scratch();
+            if ((rc = alloc(&pf_part, pf_part_bytes))) return rc;
+        }
+        if (wbits == 4 && !pf_limb_bytes) {
+            // 3..16 rows (verify_tokens, short chunks) take the small-batch
+            // projection: records + split partials of the largest of its shapes
+            size_t lb = 0;
+            for (int m = 3; m <= kLimbMaxM; ++m) {
+                auto need = [&](int n, int k, bool pair) -> size_t {
+                    if (!limb_shape_ok(m, n, k, pair)) return 0;
+                    return up256(limb_records_bytes(m, k)) + limb_partials_bytes(m, n, k, pair);
+                };
+                lb = std::max({lb, need(tq, H, false), need(H, hq * hd, false), need(I, H, true),
+                               need(H, I, false)});
+                if (m <= 8 && lmbits == 4) lb = std::max(lb, need(V, H, false));
+            }
+            if (lb && !pf_hrec && (rc = alloc(&pf_hrec, limb_records_bytes(kLimbMaxM, I)))) return rc;
+            if (lb && (rc = alloc(&pf_limb, lb))) return rc;
+            pf_limb_bytes = lb;
+        }
+        int R = kPrefillLeast;
+        while (R < kPrefillRows && R < n) R *= 2;
+        for (;; R /= 2) {
+            rc = prefill_rows(R);
+            if (!rc) rc = prefill_partials(n, start, R);
+            if (rc != TB_ERR_MEMORY || R == kPrefillLeast) break;
+        }
+        *rows = R;
+        return rc;
     }
 
     // The small-batch projection (records of x, then w4_limb) when it takes
@@ -760,7 +827,7 @@ struct Decoder {
     float *pf_attn = nullptr;    // key-range split partials of the prefill attention
     size_t pf_attn_bytes = 0;
     float *pf_rows = nullptr;    // verify_tokens: logits of every position
-    int64_t pf_rows_n = 0;
+    size_t pf_rows_bytes = 0;
     int lm_rows(const float *xr, float *y, int M) {
         int rc;
         if (lmbits == 4) {
@@ -800,22 +867,16 @@ struct Decoder {
     // returns them (decoder.rs:565-581); otherwise only the last position's.
     int prefill_batched(const int64_t *tokens, int64_t n, int64_t start,
                         float *rows_out = nullptr) {
-        int rc = layers_set();
-        if (rc || (rc = prefill_alloc(n))) return rc;
+        int rc = layers_set(), rows = 0;
+        if (rc || (rc = prefill_alloc(n, start, &rows))) return rc;
         const int nq = (hq + 2 * hkv) * hd;
         // Host copy of the whole prompt, alive until the closing synchronize.
         std::vector<int> tok32(tokens, tokens + n);
-        for (int64_t c0 = 0; c0 < n; c0 += pf_rows_cap) {
-            const int M = (int)std::min<int64_t>(pf_rows_cap, n - c0);
+        for (int64_t c0 = 0; c0 < n; c0 += rows) {
+            const int M = (int)std::min<int64_t>(rows, n - c0);
             const int pos0 = (int)(start + c0);
             TB_HIP(hipMemcpyAsync(pf_tok, tok32.data() + c0, (size_t)M * 4, hipMemcpyHostToDevice,
                                   st));
-            const size_t ab = prefill_attention_scratch(
-                M, hq, hd, prefill_attention_splits(pos0, M, hq, hkv));
-            if (ab > pf_attn_bytes) {
-                if ((rc = alloc(&pf_attn, ab))) return rc;
-                pf_attn_bytes = ab;
-            }
             if ((rc = launch_embed_rows(pf_tok, embed, pf_x, M, H, st))) return rc;
             for (int l = 0; l < L; ++l) {
                 const Layer &y = layers[l];
@@ -1425,23 +1486,20 @@ int tb_decoder_verify(tb_decoder *d, int64_t start_offset, const int64_t *tokens
     if (n == 0) return TB_OK;
     bool batch = n >= 2 && d->under_cap(start_offset, n) && !d->a8_wanted();
     for (int64_t i = 0; i < n && batch; ++i) batch = tokens[i] >= 0 && tokens[i] < d->V;
-    if (!batch) {
-        for (int64_t i = 0; i < n; ++i) {
-            int rc = d->step(tokens[i], start_offset + i, true, nullptr);
-            if (rc) return rc;
-            memcpy(logits_out + (size_t)i * d->V, d->host_logits, (size_t)d->V * 4);
-        }
-        return TB_OK;
+    if (batch) {
+        // verify_tokens (decoder.rs:565-581) as one batched forward over the n
+        // positions: the weights are read once, not n times.
+        int rc = d->regrow(&d->pf_rows, &d->pf_rows_bytes, (size_t)n * d->V * 4);
+        if (!rc) rc = d->prefill_batched(tokens, n, start_offset, d->pf_rows);
+        if (!rc)
+            TB_HIP(hipMemcpy(logits_out, d->pf_rows, (size_t)n * d->V * 4, hipMemcpyDeviceToHost));
+        if (rc != TB_ERR_MEMORY) return rc;
     }
-    // verify_tokens (decoder.rs:565-581) as one batched forward over the n
-    // positions: the weights are read once, not n times.
-    int rc;
-    if (n > d->pf_rows_n) {
-        if ((rc = d->alloc(&d->pf_rows, (size_t)n * d->V * 4))) return rc;
-        d->pf_rows_n = n;
+    for (int64_t i = 0; i < n; ++i) {
+        int rc = d->step(tokens[i], start_offset + i, true, nullptr);
+        if (rc) return rc;
+        memcpy(logits_out + (size_t)i * d->V, d->host_logits, (size_t)d->V * 4);
     }
-    if ((rc = d->prefill_batched(tokens, n, start_offset, d->pf_rows))) return rc;
-    TB_HIP(hipMemcpy(logits_out, d->pf_rows, (size_t)n * d->V * 4, hipMemcpyDeviceToHost));
     return TB_OK;
 }
 
@@ -1481,15 +1539,15 @@ int tb_decoder_prefill(tb_decoder *d, const int64_t *tokens, int64_t n, int64_t 
     TB_REQUIRE(start_offset >= 0 && start_offset + n <= d->max_seq, TB_ERR_VALUE,
                "prefill " + std::to_string(n) + " tokens at offset " + std::to_string(start_offset) +
                    " exceeds max_seq_len " + std::to_string(d->max_seq));
-    if (d->prefill_batchable(tokens, n, start_offset)) {
-        int rc = d->prefill_batched(tokens, n, start_offset);
-        if (rc) return rc;
-    } else {
-        for (int64_t i = 0; i < n; ++i) {
-            int rc = d->step(tokens[i], start_offset + i, i + 1 == n, nullptr);
-            if (rc) return rc;
-        }
+    int rc = TB_ERR_MEMORY;   // no room for a batch: step by step, as where none is taken
+    if (d->prefill_batchable(tokens, n, start_offset))
+        rc = d->prefill_batched(tokens, n, start_offset);
+    if (rc == TB_ERR_MEMORY) {
+        rc = TB_OK;
+        for (int64_t i = 0; i < n && !rc; ++i)
+            rc = d->step(tokens[i], start_offset + i, i + 1 == n, nullptr);
     }
+    if (rc) return rc;
     *offset_out = start_offset + n;
     return TB_OK;
 }
