@@ -7,6 +7,7 @@ import pytest
 
 from oracle import oracle as O
 from torchburn_amd import synth
+from torchburn_amd._lib import UnsupportedOpError
 from torchburn_amd.decoder import decoder_from_weights
 
 pytestmark = pytest.mark.gpu
@@ -91,4 +92,28 @@ def test_int8_verify_rows(cuda, lmkind, n):
     want = np.stack([ref.step(t, 9 + i).copy() for i, t in enumerate(toks)])
     assert rel(dec.verify_tokens(9, toks), want) < TOL
     ref.close()
+    dec.close()
+
+
+@pytest.mark.parametrize("wkind,refused,taken", [(4, (3, 15), (16,)), (8, (3, 16), ())])
+def test_layers_without_steps(cuda, wkind, refused, taken):
+    """Layers wider than a GEMV pass, whose steps are refused: so are the prompts
+    and verify_tokens that steps stand for."""
+    print(f"case wide layers wkind={wkind}", flush=True)
+    cfg = dict(num_layers=1, hidden=256, intermediate=16416, num_heads=4, num_kv_heads=2,
+               head_dim=64, vocab=1000, eps=1e-6, rope_theta=1e6, qkv_bias=True)
+    dec = decoder_from_weights(synth.decoder_weights(cfg, 94, wkind, wkind, 32), cfg,
+                               group_size=32, max_seq_len=64)
+    with pytest.raises(UnsupportedOpError, match="K <= 16384"):
+        dec._step(1, 0, True)
+    for n in refused:
+        with pytest.raises(UnsupportedOpError, match="K <= 16384"):
+            dec.prefill_tokens(list(range(n)), 0)
+    for n in taken:
+        assert dec.prefill_tokens(list(range(n)), 0) == n
+    if wkind == 8:
+        with pytest.raises(UnsupportedOpError, match="K <= 16384"):
+            dec.verify_tokens(0, [1, 2, 3, 4])
+    else:
+        assert np.isfinite(dec.verify_tokens(0, [1, 2, 3, 4])).all()
     dec.close()

@@ -763,7 +763,7 @@ struct Decoder {
     int rows_w8(const float *xin, const void *w, const float *s, const float *b, const void *w2,
                 const float *s2, const float *res, float *y, int m, int n, int k, int epi,
                 void *scratch, size_t cap) {
-        if (qgemm_w8_wins(m, (int64_t)n * k * (w2 ? 2 : 1)) || k > kMaxGemvElems) {
+        if (qgemm_w8_wins(m, (int64_t)n * k * (w2 ? 2 : 1))) {
             QGemmParams q{};
             q.x = xin; q.w0 = w; q.s0 = s; q.b0 = b; q.w1 = w2; q.s1 = s2; q.res = res; q.y = y;
             q.m = m; q.n = n; q.k = k; q.fmt = Q_W8; q.s0_len = q.s1_len = n;
@@ -810,11 +810,15 @@ struct Decoder {
     // Qwen2.5-0.5B 1399 / 2546 and 1358 / 2530; for 2 tokens the INT4 layers
     // 1193 / 1014).
     static constexpr int kBatchPrompt = 3;
-    static constexpr int kMaxGemvElems = 16384;   // K of one streaming GEMV pass
+    // Layers wider than one GEMV pass have no steps: INT8 prompts are refused as the
+    // steps are, INT4 ones run from 16 tokens.
+    static constexpr int kMaxGemvK = 16384, kBatchPromptWide = 16;
+    bool wide_layers() const { return std::max({H, I, hq * hd}) > kMaxGemvK; }
     bool prefill_batchable(const int64_t *tokens, int64_t n, int64_t start) const {
         static const bool loop_only = getenv("TB_PREFILL_LOOP") != nullptr;
         // W4A8 rounds each token's projection inputs: the step loop does that
         if (loop_only || n < kBatchPrompt || !under_cap(start, n) || a8_wanted()) return false;
+        if (wide_layers() && (wbits == 8 || n < kBatchPromptWide)) return false;
         for (int64_t i = 0; i < n; ++i)
             if (tokens[i] < 0 || tokens[i] >= V) return false;   // the step's zero-logit rule
         return true;
@@ -1484,7 +1488,8 @@ int tb_decoder_verify(tb_decoder *d, int64_t start_offset, const int64_t *tokens
     TB_REQUIRE(start_offset >= 0 && start_offset + n <= d->max_seq, TB_ERR_VALUE,
                "verify exceeds max_seq_len");
     if (n == 0) return TB_OK;
-    bool batch = n >= 2 && d->under_cap(start_offset, n) && !d->a8_wanted();
+    bool batch = n >= 2 && d->under_cap(start_offset, n) && !d->a8_wanted() &&
+                 !(d->wbits == 8 && d->wide_layers());
     for (int64_t i = 0; i < n && batch; ++i) batch = tokens[i] >= 0 && tokens[i] < d->V;
     if (batch) {
         // verify_tokens (decoder.rs:565-581) as one batched forward over the n
