@@ -898,18 +898,25 @@ QPlan plan(int m, int n, int k, int fmt, bool grouped, bool pair, size_t cap) {
     return pl;
 }
 
+// SwiGLU pairs come as INT4 with group scales and as INT8.
+constexpr bool takes_pair(int fmt, bool grouped) { return fmt == Q_W8 || (fmt == Q_W4 && grouped); }
+
 template <int FMT, int SM>
 int launch(const QArgs &a, const QPlan &pl, bool pair, hipStream_t st) {
+    constexpr bool PAIRS = takes_pair(FMT, SM != 2);
     const long tiles = (long)pl.mz * pl.nbx * pl.splits;
     const dim3 grid((unsigned)((tiles + 7) / 8 * 8)), block(256);
     if (pl.direct) {
         const size_t lds = (size_t)std::min(pl.slen, kDirectGroups) * kGroupBytes;
 #define TB_QDIRECT(LONG_)                                                                        \
     do {                                                                                         \
-        if (pair)                                                                                \
-            hipLaunchKernelGGL((k_qdirect<FMT, 2, SM, true, LONG_>), grid, block, lds, st, a);   \
-        else                                                                                     \
-            hipLaunchKernelGGL((k_qdirect<FMT, 1, SM, false, LONG_>), grid, block, lds, st, a);  \
+        if constexpr (PAIRS) {                                                                   \
+            if (pair) {                                                                          \
+                hipLaunchKernelGGL((k_qdirect<FMT, 2, SM, true, LONG_>), grid, block, lds, st, a); \
+                break;                                                                           \
+            }                                                                                    \
+        }                                                                                        \
+        hipLaunchKernelGGL((k_qdirect<FMT, 1, SM, false, LONG_>), grid, block, lds, st, a);      \
     } while (0)
         if (pl.slen > kDirectGroups) TB_QDIRECT(true);
         else TB_QDIRECT(false);
@@ -932,8 +939,14 @@ int launch(const QArgs &a, const QPlan &pl, bool pair, hipStream_t st) {
             return TB_OK;
         }
     }
-    if (pair) TB_QGO(1, 2, true);
-    else if (pl.mt == 2) TB_QGO(2, 1, false);
+    if constexpr (PAIRS) {
+        if (pair) {
+            TB_QGO(1, 2, true);
+            TB_LAUNCHED();
+            return TB_OK;
+        }
+    }
+    if (pl.mt == 2) TB_QGO(2, 1, false);
     else if (pl.nt == 2) TB_QGO(1, 2, false);
     else TB_QGO(1, 1, false);
 #undef TB_QGO
@@ -959,6 +972,8 @@ int qgemm(const QGemmParams &p, const QPlan &pl, void *scratch, hipStream_t st) 
     const bool pair = p.w1 != nullptr;
     TB_REQUIRE(qgemm_shape_ok(p.m, p.n, p.k, p.fmt), TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: batched projection needs K % 32 == 0");
+    TB_REQUIRE(!pair || takes_pair(p.fmt, p.grouped != 0), TB_ERR_UNSUPPORTED,
+               "TB_UNSUPPORTED: batched SwiGLU pairs are INT8, or INT4 with group scales");
     uint8_t *rec = static_cast<uint8_t *>(scratch);
     float *inv = nullptr, *part = reinterpret_cast<float *>(rec);
     if (!pl.direct) {
