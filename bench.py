@@ -313,18 +313,15 @@ def int4_set(torch, dev, gen, n, k, gs=32):
 
 
 def batched_kernel(M, N, K):
-    """The kernel tb_w4a32_grouped_linear runs for an M x N x K v1 g32
-    projection (the selection in csrc/capi.hip linear_w4 and csrc/qgemm.hip
-    plan): M = 3..16 on more than 16 Mi weights takes the small-batch f16-MFMA
-    limb kernel (exact products from f16 limbs of x), else from M = 5 the
-    batched f16-limb GEMM, which builds the limbs in its blocks for few rows.
+    """The kernel tb_w4a32_grouped_linear runs for an M x N x K v1 g32 projection.
     Every entry's frac_fp32_mfma_peak is its f32-contraction rate over the
     FP32-MFMA peak; the limb kernels get there on f16 MFMA."""
-    if 3 <= M <= 16 and N * K > 1 << 24:
-        return "k_limb_prep + k_w4_limb (f16 MFMA on exact limbs of x) + k_limb_reduce"
-    if M <= 32:
-        return "k_qdirect (f16 MFMA on two f16 limbs of x) + k_qreduce"
-    return "k_qsplit + k_qgemm (f16 MFMA on two f16 limbs of x) + k_qreduce"
+    from torchburn_amd import _lib
+    name = _lib.lib().tb_w4_kernel(0, M, N, K, 32).decode()
+    return {"k_w4_limb": "k_limb_prep + k_w4_limb (f16 MFMA on exact limbs of x) + k_limb_reduce",
+            "k_qdirect": "k_qdirect (f16 MFMA on two f16 limbs of x) + k_qreduce",
+            "k_qsplit + k_qgemm": "k_qsplit + k_qgemm (f16 MFMA on two f16 limbs of x) + k_qreduce",
+            }.get(name, name)
 
 
 def batched_section(torch, args, dev):

@@ -30,6 +30,14 @@ TB_API int tb_decoder_time_greedy(tb_decoder *d, int64_t first_token, int64_t of
 TB_API int tb_read_probe(const void *buf, int64_t bytes, int64_t blocks, int64_t loads,
                          uint32_t *out, int64_t *bytes_read, void *stream);
 
+/* Measurement aid (no reference counterpart): the name of the kernel that an INT4
+ * call of these sizes runs on, for 16-byte aligned operands and W4A8 semantics
+ * off; host only.  op 0: tb_w4a32_grouped_linear, 1: tb_w4a32_linear (scales per
+ * row or scalar), 2: tb_w4a32_grouped_linear_v2, 3: tb_swiglu_w4a32 (n = inter),
+ * 4: the gate/up pair of tb_fused_swiglu_mlp_w4a32 from K to n and back to K.
+ * NULL for sizes or a group size that no call takes. */
+TB_API const char *tb_w4_kernel(int64_t op, int64_t m, int64_t n, int64_t k, int64_t group_size);
+
 #ifdef __cplusplus
 }
 #endif

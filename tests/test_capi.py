@@ -120,3 +120,29 @@ def test_noalloc_scratch_limit_before_any_gpu_call():
     for m in (55, 64, 89, 128):
         assert call(m) == _lib.TB_ERR_UNSUPPORTED, m
         assert b"static scratch holds 16777216" in L.tb_last_error()
+
+
+@pytest.mark.parametrize("op,m,n,k,gs,kernel", [
+    (0, 1, 14336, 4096, 32, "k_w4_gemv"), (0, 2, 14336, 4096, 32, "k_w4_gemv"),
+    (0, 3, 14336, 4096, 32, "k_w4_limb"), (0, 16, 4097, 4096, 32, "k_w4_limb"),
+    (0, 16, 4096, 4096, 32, "k_qdirect"),              # 2^24 weights are not more than 2^24
+    (0, 3, 4096, 4096, 32, "k_w4_gemv"), (0, 4, 4096, 4096, 32, "k_w4_gemv"),
+    (0, 4, 300, 20480, 32, "k_w4_limb"),               # K past one GEMV pass
+    (0, 3, 300, 16416, 32, "k_gemv_generic"),          # ... and not in whole batches of 128
+    (0, 5, 300, 16416, 32, "k_qsplit + k_qgemm"), (0, 17, 14336, 4096, 32, "k_qsplit + k_qgemm"),
+    (0, 64, 14336, 4096, 32, "k_qsplit + k_qgemm"), (0, 8, 14336, 4000, 32, "k_qsplit + k_qgemm"),
+    (0, 4, 100, 33, 32, "k_gemv_generic"), (0, 4, 100, 96, 64, "k_gemv_generic"),
+    (1, 4, 16411, 1024, 0, "k_w4_limb"), (1, 12, 777, 1024, 0, "k_qdirect"),
+    (2, 4, 4805, 1600, 64, "k_w4_gemv"), (2, 37, 4805, 1600, 64, "k_qdirect"),
+    (3, 8, 14336, 4096, 32, "k_w4_limb"), (3, 12, 4096, 2048, 32, "k_qdirect"),
+    (4, 8, 14336, 4096, 32, "k_w4_limb"), (4, 16, 2048, 1024, 64, "k_qdirect"),
+    (4, 512, 14336, 4096, 64, "k_qsplit + k_qgemm")])
+def test_int4_routes(op, m, n, k, gs, kernel):
+    assert _lib.lib().tb_w4_kernel(op, m, n, k, gs).decode() == kernel
+
+
+def test_int4_routes_of_impossible_calls():
+    L = _lib.lib()
+    for args in ((5, 1, 1, 32, 32), (0, 0, 1, 32, 32), (0, 1, 1, 32, 9), (2, 1, 1, 96, 64),
+                 (2, 1, 1, 64, 32)):
+        assert L.tb_w4_kernel(*args) is None, args

@@ -1,5 +1,7 @@
-"""Parity of the small-batch INT4 projection (3..16 activation rows on f16
-MFMA, csrc/w4_limb.hip) with the CPU oracle.
+"""Parity of INT4 projections of 3..16 activation rows with the CPU oracle: the
+small-batch kernel (csrc/w4_limb.hip) on weights of more than 2^24 elements, and
+the GEMV passes and the batched kernel (csrc/qgemm.hip) that smaller ones take.
+Every case names the kernel it is there for, and checks that the call runs it.
 
 The oracle restates the reference's gemm_w4a32_grouped / w4a32_grouped_linear
 (src/quantization/gemv.rs:1690-1725, packed_v2.rs:557-624), one GEMV per row,
@@ -12,12 +14,19 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from torchburn_amd import synth
+from torchburn_amd import _lib, synth
 import torchburn_amd as tb
 
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-4
+
+LIMB, GEMV, DIRECT = "k_w4_limb", "k_w4_gemv", "k_qdirect"
+LINEAR, PER_ROW, PAIR, MLP = 0, 1, 3, 4   # operations of tb_w4_kernel
+
+
+def runs(kernel, op, m, n, k, gs=32):
+    assert _lib.lib().tb_w4_kernel(op, m, n, k, gs).decode() == kernel
 
 
 def rel_rows(a, b):
@@ -33,13 +42,17 @@ def T(a, dev):
     return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
 
 
-@pytest.mark.parametrize("m,n,k,gs", [
-    (3, 1000, 2048, 32), (7, 4096, 4096, 64), (8, 45, 256, 32),
-    (9, 1000, 2048, 32), (12, 300, 1024, 128), (16, 4096, 4096, 32), (5, 14336, 4096, 32),
-    (16, 1, 128, 32), (3, 33, 128, 64),
+@pytest.mark.parametrize("kernel,m,n,k,gs", [
+    (LIMB, 3, 4101, 4096, 32), (LIMB, 7, 4100, 4096, 64), (LIMB, 8, 16391, 1024, 32),
+    (LIMB, 9, 8197, 2048, 32), (LIMB, 12, 16421, 1024, 128), (LIMB, 16, 4133, 4096, 32),
+    (LIMB, 5, 14336, 4096, 32), (LIMB, 16, 131079, 128, 32), (LIMB, 3, 131105, 128, 64),
+    (GEMV, 3, 1000, 2048, 32), (DIRECT, 7, 4096, 4096, 64), (DIRECT, 8, 45, 256, 32),
+    (DIRECT, 9, 1000, 2048, 32), (DIRECT, 12, 300, 1024, 128), (DIRECT, 16, 4096, 4096, 32),
+    (DIRECT, 16, 1, 128, 32), (GEMV, 3, 33, 128, 64),
 ])
-def test_limb_linear_matches_oracle(cuda, m, n, k, gs):
-    print(f"case limb linear m={m} n={n} k={k} gs={gs}", flush=True)
+def test_few_rows_linear_matches_oracle(cuda, kernel, m, n, k, gs):
+    print(f"case few rows linear {kernel} m={m} n={n} k={k} gs={gs}", flush=True)
+    runs(kernel, LINEAR, m, n, k, gs)
     g = synth.rng(71, m, n, k, gs)
     x = synth.activations(g, m, k)
     w, s = synth.int4_weight(g, n, k, gs)
@@ -50,11 +63,12 @@ def test_limb_linear_matches_oracle(cuda, m, n, k, gs):
     assert rel_rows(y.cpu().numpy(), ref) < TOL
 
 
-@pytest.mark.parametrize("m", [4, 13])
-def test_limb_residual(cuda, m):
-    print(f"case limb residual m={m}", flush=True)
+@pytest.mark.parametrize("kernel,m,n,k", [(LIMB, 4, 4130, 4096), (LIMB, 13, 8210, 2048),
+                                          (GEMV, 4, 2048, 2048), (DIRECT, 13, 2048, 2048)])
+def test_few_rows_residual(cuda, kernel, m, n, k):
+    print(f"case few rows residual {kernel} m={m}", flush=True)
+    runs(kernel, LINEAR, m, n, k)
     g = synth.rng(72, m)
-    n, k = 2048, 2048
     x = synth.activations(g, m, k)
     r = synth.activations(g, m, n)
     w, s = synth.int4_weight(g, n, k, 32)
@@ -66,12 +80,15 @@ def test_limb_residual(cuda, m):
     assert rel_rows(out.cpu().numpy(), ref) < TOL
 
 
-@pytest.mark.parametrize("m,scalar", [(4, False), (12, True), (3, True)])
-def test_limb_per_channel(cuda, m, scalar):
+@pytest.mark.parametrize("kernel,m,n,k,scalar", [
+    (LIMB, 4, 16411, 1024, False), (LIMB, 12, 4105, 4096, True), (LIMB, 3, 16411, 1024, True),
+    (LIMB, 15, 8200, 2048, False),
+    (GEMV, 4, 777, 1024, False), (DIRECT, 12, 777, 1024, True), (GEMV, 3, 777, 1024, True)])
+def test_few_rows_per_channel(cuda, kernel, m, n, k, scalar):
     """w4a32_linear with one scale per row or one scalar (gemv.rs:1114-1180)."""
-    print(f"case limb w4a32_linear m={m} scalar={scalar}", flush=True)
+    print(f"case few rows w4a32_linear {kernel} m={m} scalar={scalar}", flush=True)
+    runs(kernel, PER_ROW, m, n, k)
     g = synth.rng(73, m, int(scalar))
-    n, k = 777, 1024
     x = synth.activations(g, m, k)
     w = g.integers(0, 256, size=(n, k // 2), dtype=np.uint8)
     s = (np.abs(g.normal(0, 0.02, 1 if scalar else n)) + 1e-3).astype(np.float32)
@@ -81,11 +98,13 @@ def test_limb_per_channel(cuda, m, scalar):
     assert rel_rows(y, ref) < TOL
 
 
-@pytest.mark.parametrize("m,k,inter,gs", [(3, 1024, 2048, 32), (8, 4096, 14336, 32),
-                                          (16, 1024, 2048, 64), (11, 512, 1024, 32),
-                                          (4, 4096, 14336, 64)])
-def test_limb_swiglu_mlp_with_biases(cuda, m, k, inter, gs):
-    print(f"case limb MLP m={m} k={k} inter={inter} gs={gs}", flush=True)
+@pytest.mark.parametrize("kernel,m,k,inter,gs", [
+    (LIMB, 8, 4096, 14336, 32), (LIMB, 4, 4096, 14336, 64), (LIMB, 16, 2048, 4224, 64),
+    (LIMB, 11, 1024, 8320, 32),
+    (GEMV, 3, 1024, 2048, 32), (DIRECT, 16, 1024, 2048, 64), (DIRECT, 11, 512, 1024, 32)])
+def test_few_rows_swiglu_mlp_with_biases(cuda, kernel, m, k, inter, gs):
+    print(f"case few rows MLP {kernel} m={m} k={k} inter={inter} gs={gs}", flush=True)
+    runs(kernel, MLP, m, inter, k, gs)
     g = synth.rng(74, m, k, inter, gs)
     x = synth.activations(g, m, k)
     r = synth.activations(g, m, k)
@@ -104,15 +123,22 @@ def test_limb_swiglu_mlp_with_biases(cuda, m, k, inter, gs):
     assert rel_rows(out.cpu().numpy(), ref) < TOL
 
 
-def test_limb_non_finite_propagate(cuda):
-    """NaN / Inf rows: the flagged batches take the f32 path; other rows stay exact."""
+@pytest.mark.parametrize("kernel,m,n,k", [
+    (LIMB, 6, 8201, 2048), (LIMB, 6, 4105, 4096),   # the second in K splits
+    (LIMB, 13, 8201, 2048), (LIMB, 6, 24576, 4096),  # two tiles; all of K in one block
+    (DIRECT, 6, 300, 2048)])
+def test_few_rows_non_finite_propagate(cuda, kernel, m, n, k):
+    """NaN / Inf rows: the flagged batches of the small-batch kernel take the f32
+    path; other rows stay exact."""
+    print(f"case few rows non-finite {kernel} m={m} n={n}", flush=True)
+    runs(kernel, LINEAR, m, n, k)
     g = synth.rng(75)
-    m, n, k = 6, 300, 2048
     w, s = synth.int4_weight(g, n, k, 32)
     x = synth.activations(g, m, k)
     x[1, 1234] = np.nan
     x[3, 77] = np.inf
     x[4, 500] = -np.inf
+    x[m - 1, 3] = np.inf if m > 8 else x[m - 1, 3]
     ref = O.gemm_w4(x, w, s, None, group_size=32)
     y = tb.w4a32_grouped_linear(T(x, cuda), T(w, cuda), T(s, cuda), None, 32).cpu().numpy()
     assert np.array_equal(np.isnan(y), np.isnan(ref))
@@ -120,14 +146,18 @@ def test_limb_non_finite_propagate(cuda):
     assert np.array_equal(np.sign(y[np.isinf(ref)]), np.sign(ref[np.isinf(ref)]))
     fin = np.isfinite(ref).all(axis=1)
     assert fin[[0, 2, 5]].all()
+    assert m <= 8 or not fin[m - 1]
     assert rel_rows(y[fin], ref[fin]) < TOL
 
 
-def test_limb_extreme_ranges_and_zero_rows(cuda):
+@pytest.mark.parametrize("kernel,m,n,k", [
+    (LIMB, 5, 8201, 2048), (LIMB, 5, 4105, 4096), (LIMB, 12, 8201, 2048), (DIRECT, 5, 256, 2048)])
+def test_few_rows_extreme_ranges_and_zero_rows(cuda, kernel, m, n, k):
     """Groups spanning 1e-30..1e30, all-zero groups, an all-zero row, and a
-    row above 2^100 (the f32 path)."""
+    row above 2^100 (the f32 paths)."""
+    print(f"case few rows extremes {kernel} m={m} n={n}", flush=True)
+    runs(kernel, LINEAR, m, n, k)
     g = synth.rng(76)
-    m, n, k = 5, 256, 2048
     w, s = synth.int4_weight(g, n, k, 32)
     b = g.normal(0, 0.1, n).astype(np.float32)
     x = synth.activations(g, m, k)
@@ -145,9 +175,11 @@ def test_limb_extreme_ranges_and_zero_rows(cuda):
     assert rel_rows(y, ref) < TOL
 
 
-def test_limb_deterministic(cuda):
+@pytest.mark.parametrize("kernel,n", [(LIMB, 4160), (DIRECT, 4096)])
+def test_few_rows_deterministic(cuda, kernel, n):
+    m, k = 8, 4096
+    runs(kernel, LINEAR, m, n, k)
     g = synth.rng(77)
-    m, n, k = 8, 4096, 4096
     x = T(synth.activations(g, m, k), cuda)
     w, s = synth.int4_weight(g, n, k, 32)
     w, s = T(w, cuda), T(s, cuda)
@@ -163,6 +195,7 @@ def test_limb_whole_k_pair_partial_quad_and_nan(cuda):
     print("case limb whole-K MLP m=6 k=3968 inter=14336 + NaN row", flush=True)
     g = synth.rng(78)
     m, k, inter, gs = 6, 3968, 14336, 32
+    runs(LIMB, MLP, m, inter, k)
     x = synth.activations(g, m, k)
     gw, gsc = synth.int4_weight(g, inter, k, gs)
     uw, usc = synth.int4_weight(g, inter, k, gs)
@@ -184,6 +217,7 @@ def test_limb_whole_k_single_projection(cuda):
     print("case limb whole-K linear m=5 n=24576 k=4096", flush=True)
     g = synth.rng(79)
     m, n, k = 5, 24576, 4096
+    runs(LIMB, LINEAR, m, n, k)
     w, s = synth.int4_weight(g, n, k, 32)
     b = g.normal(0, 0.1, n).astype(np.float32)
     x = synth.activations(g, m, k)
@@ -192,19 +226,21 @@ def test_limb_whole_k_single_projection(cuda):
     assert rel_rows(y.cpu().numpy(), ref) < TOL
 
 
-@pytest.mark.parametrize("m,k,inter,gs,bias", [
-    (5, 4096, 14336, 32, True),    # whole-K pair, h only (no records for a next projection)
-    (8, 4096, 12288, 32, False),   # whole-K pair at the plan's smallest size class
-    (3, 4096, 10752, 64, True),    # whole-K pair, group-64 scales (one dword per group)
-    (7, 2048, 14336, 128, False),  # whole-K pair, group 128, a short K
-    (12, 2048, 4096, 32, True),    # two tiles: split partials and the pair reduce
-    (3, 1024, 2048, 64, False),    # one tile, split partials
+@pytest.mark.parametrize("kernel,m,k,inter,gs,bias", [
+    (LIMB, 5, 4096, 14336, 32, True),    # whole-K pair, h only (no records for a next projection)
+    (LIMB, 8, 4096, 12288, 32, False),   # whole-K pair at the plan's smallest size class
+    (LIMB, 3, 4096, 10752, 64, True),    # whole-K pair, group-64 scales (one dword per group)
+    (LIMB, 7, 2048, 14336, 128, False),  # whole-K pair, group 128, a short K
+    (LIMB, 12, 2048, 4224, 32, True),    # two tiles: split partials and the pair reduce
+    (LIMB, 3, 4096, 2176, 64, False),    # one tile, split partials
+    (DIRECT, 12, 2048, 4096, 32, True), (GEMV, 3, 1024, 2048, 64, False),
 ])
-def test_limb_swiglu_pair_entry(cuda, m, k, inter, gs, bias):
+def test_few_rows_swiglu_pair_entry(cuda, kernel, m, k, inter, gs, bias):
     """tb_swiglu_w4a32, the neuron loop of fused_swiglu_mlp_w4a32
     (src/quantization/fused_ops.rs:244-407) on its own: h against the oracle."""
-    from torchburn_amd import _lib
-    print(f"case limb SwiGLU pair m={m} k={k} inter={inter} gs={gs} bias={bias}", flush=True)
+    print(f"case few rows SwiGLU pair {kernel} m={m} k={k} inter={inter} gs={gs} bias={bias}",
+          flush=True)
+    runs(kernel, PAIR, m, inter, k, gs)
     g = synth.rng(83, m, k, inter, gs)
     x = synth.activations(g, m, k)
     gw, gsc = synth.int4_weight(g, inter, k, gs)

@@ -73,6 +73,7 @@ _SIGS = {
 def declared_symbols() -> list:
     """Every entry point the Python layer binds (all are declared in include/tbhip.h)."""
     return ["tb_last_error", "tb_version", "tb_x_records_bytes", "tb_sample_uniform",
+            "tb_w4_kernel",
             *_SIGS.keys()]
 
 
@@ -91,6 +92,8 @@ def lib():
             L.tb_version.restype = C.c_char_p
             L.tb_x_records_bytes.restype = C.c_int64
             L.tb_x_records_bytes.argtypes = [C.c_int64, C.c_int64]
+            L.tb_w4_kernel.restype = C.c_char_p
+            L.tb_w4_kernel.argtypes = [C.c_int64] * 5
             L.tb_sample_uniform.restype = C.c_float
             L.tb_sample_uniform.argtypes = [C.c_uint64, C.c_uint64]
             for name, args in _SIGS.items():

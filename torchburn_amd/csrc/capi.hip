@@ -23,6 +23,7 @@
 #include "w4_limb.hpp"
 #include "v2_layout.hpp"
 #include "qgemm.hpp"
+#include "../../include/tbhip_bench.h"
 #include "quantize.hpp"
 #include "sample.hpp"
 
@@ -1003,6 +1004,35 @@ int tb_xquant(const float *x, uint32_t *xq, int64_t m, int64_t k, void *stream) 
     TB_REQUIRE(aligned(x, 16) && aligned(xq, 16), TB_ERR_UNSUPPORTED,
                "TB_UNSUPPORTED: xquant: 16-byte aligned device pointers required");
     return xquant(x, xq, (int)m, (int)k, (hipStream_t)stream);
+}
+
+const char *tb_w4_kernel(int64_t op, int64_t m, int64_t n, int64_t k, int64_t group_size) {
+    const bool rows = op == 1, v2 = op == 2, pair = op >= 3;
+    if (op < 0 || op > 4 || m < 1 || n < 1 || k < 1 || m >= (1ll << 24) || n >= (1ll << 31) - 512 ||
+        k > (1 << 30) || (!rows && (group_size < 2 || group_size % 2)) ||
+        (v2 && (group_size != 64 || k % 64)))
+        return nullptr;
+    const float *x = reinterpret_cast<const float *>(256);   // aligned, never read
+    const uint8_t *w = reinterpret_cast<const uint8_t *>(256);
+    const int64_t gs = rows ? 32 : group_size;
+    int route;   // as mlp_w4_route()
+    if (op == 4) {
+        MlpW4 a{};
+        a.x = x; a.gate_w = a.up_w = a.down_w = w;
+        a.m = m; a.k = a.n_out = k; a.inter = n; a.gs = gs;
+        route = mlp_w4_path(a);
+    } else if (!v2 && limb_fast(x, w, m, n, k, gs, rows, pair)) {
+        route = 3;
+    } else if (!v2 && !w4_fast(x, w, m, k, gs, rows)) {
+        route = 0;
+    } else {
+        route = m >= mfma_min_m() ? 1 : 2;
+    }
+    if (route == 0) return "k_gemv_generic";
+    if (route == 2) return "k_w4_gemv";
+    if (route == 3) return "k_w4_limb";
+    return qgemm_plan((int)m, (int)n, (int)k, v2 ? Q_V2 : Q_W4, !rows, pair).direct
+               ? "k_qdirect" : "k_qsplit + k_qgemm";
 }
 
 int tb_w4a32_gemv_xq(const float *x, const uint32_t *xq, const uint8_t *w_packed,
