@@ -1,4 +1,6 @@
-"""Parity of the batched INT4 projection (FP32 MFMA from M = 5) with the CPU oracle.
+"""Parity of batched INT4 projections (5 rows and more: the batched f16-MFMA kernel
+of csrc/qgemm.hip, or up to 16 rows on more than 2^24 weights the small-batch kernel
+of csrc/w4_limb.hip) with the CPU oracle.
 
 The oracle's gemm_w4 restates the reference's gemm_w4a32_grouped
 (src/quantization/gemv.rs:1690-1725: one full GEMV per activation row), and
@@ -36,19 +38,19 @@ SHAPES = [
     (16, 14336, 4096, 32),    # config 3
     (64, 4096, 4096, 32),     # config 3
     (64, 14336, 4096, 32),    # config 3
-    (15, 1000, 2048, 32),     # last GEMV row count
+    (15, 1000, 2048, 32),     # half a 32-row slab, ragged N
     (17, 1000, 2048, 32),     # ragged M and N
-    (33, 517, 1024, 64),      # group 64, three M tiles
-    (130, 96, 4096, 32),      # two M blocks of 64 plus a tail
-    (16, 7, 32, 32),          # one group per row, N below a wave's 16 rows
-    (20, 64, 96, 32),         # K not a multiple of the 128-wide step
-    (48, 200, 192, 64),       # K = 1.5 steps, group 64
+    (33, 517, 1024, 64),      # group 64, a second slab of one row
+    (130, 96, 4096, 32),      # four slabs and a tail of two rows
+    (16, 7, 32, 32),          # one group per row, N below a wave's 32 weight rows
+    (20, 64, 96, 32),         # K not a multiple of the 128-wide stage
+    (48, 200, 192, 64),       # K = 1.5 stages, group 64
     (5, 4096, 4096, 32),      # verify-sized batches
     (8, 14336, 4096, 32),
     (7, 1000, 2048, 64),      # group 64
-    (9, 517, 1024, 32),       # four-row tiles 3 of 4 used, ragged N
+    (9, 517, 1024, 32),       # ragged N
     (12, 96, 14336, 32),      # K split over many blocks
-    (6, 33, 96, 32),          # 3 chunks, N below a wave's 16 rows
+    (6, 33, 96, 32),          # 3 groups, one weight row past a wave's 32
 ]
 
 
@@ -67,15 +69,15 @@ def test_mfma_linear_matches_oracle(cuda, m, n, k, gs):
     assert err < TOL
 
 
-# Up to 16 rows in shapes the small-batch limb path does not take (K % 128 != 0,
-# or M = 16 with N, K <= 4096): the FP32-MFMA split-K projection, with and
-# without the residual epilogue.
+# Up to 16 rows in shapes that the small-batch kernel does not take (K % 128 != 0)
+# or leaves to the batched one (at most 2^24 weights), with and without the
+# residual epilogue.
 SMALL_M_SHAPES = [
     # (m, n, k, gs)
     (11, 300, 4064, 32),      # ragged N, K % 128 != 0
-    (16, 4096, 1056, 32),     # 8.25 steps: the last K split ends inside a step
+    (16, 4096, 1056, 32),     # 8.25 stages: the last K split ends inside a stage
     (13, 77, 2112, 64),       # group 64
-    (5, 2000, 160, 32),       # 2 steps
+    (5, 2000, 160, 32),       # 2 stages
     (16, 4160, 4000, 32),     # N past 4096 with K % 128 != 0
     (16, 33, 4096, 128),      # group 128, one row block
 ]
@@ -128,7 +130,7 @@ def test_mfma_residual_matches_oracle(cuda, m):
 
 @pytest.mark.parametrize("m,k,inter,gs", [(16, 4096, 14336, 32), (64, 4096, 14336, 32),
                                           (24, 896, 4864, 32), (16, 512, 1024, 64),
-                                          (12, 1056, 1120, 32),   # K % 128 != 0: FP32 MFMA
+                                          (12, 1056, 1120, 32),   # K % 128 != 0
                                           (16, 2112, 3136, 64)])
 def test_mfma_swiglu_mlp_matches_oracle(cuda, m, k, inter, gs):
     print(f"case mfma fused_swiglu_mlp m={m} k={k} inter={inter} gs={gs}", flush=True)
@@ -203,9 +205,8 @@ def test_mfma_special_cases(cuda):
 
 @pytest.mark.parametrize("m", [16, 6, 40, 70])
 def test_mfma_non_finite_propagate(cuda, m):
-    """NaN / Inf in one 16-row slab take the f32 path for that slab's batch
-    (M = 40: the third slab of a block; M = 70: the fifth slab, a second block
-    along M); the other slabs stay on the limbs."""
+    """NaN / Inf travel through the first limb of their own row (M = 40 and 70: in the
+    first slab of 32 rows and in a later one); every other row is as ever."""
     g = synth.rng(34, m)
     n, k = 128, 1024
     w, s = synth.int4_weight(g, n, k, 32)

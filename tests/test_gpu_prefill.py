@@ -2,9 +2,8 @@
 
 The reference's prefill_tokens (src/llm/decoder.rs:431-447) runs one decoder
 step per prompt token and keeps the last step's logits.  The gfx950 decoder
-runs prompts of 16 or more in-vocabulary tokens (INT4 projections) as batches:
-row RMSNorms, the QKV / O / gate-up / down projections on the FP32-MFMA GEMM,
-RoPE + KV append for every row and causal attention over the cache.  The
+runs prompts of 3 or more in-vocabulary tokens as batches: row RMSNorms, the QKV /
+O / gate-up / down projections on the few-row and batched kernels, RoPE + KV append for every row and causal attention over the cache.  The
 oracle steps through the same prompt; the prefill's logits, the KV cache it
 leaves (through the decode steps that read it) and the greedy continuation
 must match.  Metric max|d| / max|ref| (tests/parity/int4.rs:131-141).
@@ -78,8 +77,7 @@ def test_prefill_small(cuda):
 
 
 def test_prefill_chunks_after_cached_prefix(cuda):
-    """A 300-token prompt after 20 cached positions: two 256-row chunks, the
-    second attending over the first chunk's KV rows."""
+    """300 tokens after 20 cached positions, one batch in buffers of 512 rows."""
     run_prefill(small(), 22, 300, start=20, max_seq=400)
 
 
@@ -94,8 +92,8 @@ def test_prefill_threshold_g64_int8_lm_head(cuda):
 
 
 def test_prefill_group64_v2_blocks(cuda):
-    """Group 64, vocab 1024: the batched projections read v2 blocks for QKV, O
-    and down and the lm_head (MFMA V2 path)."""
+    """Group 64, vocab 1024: QKV, O, down and the lm_head have binary16 scales, as
+    the reference's v2 blocks hold them."""
     run_prefill(small(vocab=1024), 28, 100, start=7, gs=64)
 
 
@@ -111,5 +109,7 @@ def test_prefill_mha_and_wide_groups(cuda, heads):
     run_prefill(cfg, 26, 65, start=3)
 
 
-def test_prefill_short_prompt_uses_steps(cuda):
-    run_prefill(small(), 27, 15)
+@pytest.mark.parametrize("n", [2, 3, 15])
+def test_prefill_short_prompt(cuda, n):
+    """2 tokens are steps, 3 and 15 a batch of few rows."""
+    run_prefill(small(), 27, n)

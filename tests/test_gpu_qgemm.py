@@ -1,7 +1,7 @@
-"""The batched f16-limb projection (INT4 from 17 rows, INT8 from 3 or 5) at the edges of its tiles:
-rows around 32 and 64, column blocks of 128 and 256, K that is no whole number
-of 128-element stages, K splits, every scale form, and rows of extreme or
-non-finite activations.  Against float64; the bound follows the kernel: two f16
+"""The batched f16-limb projection (INT4 from 5 rows, INT8 from 4, or 3 on 32 Mi
+weights) at the edges of its tiles: rows around 32 and 64, column blocks of 128 and
+256, K that is no whole number of 128-element stages, K splits, every scale form,
+and rows of extreme or non-finite activations.  Against float64; the bound follows the kernel: two f16
 limbs hold an activation to 2^-22, and every sum is f32, one addition per 32
 elements of K plus the splits', so an output is off by at most
 (K / 32 + 16) 2^-24 sum |w x|."""

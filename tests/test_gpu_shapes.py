@@ -34,14 +34,14 @@ def T(a, dev):
 @pytest.mark.parametrize("m,n,k,scalar", [
     (1, 4096, 4096, False),     # streaming GEMV, one scale per row
     (3, 300, 896, False),       # GEMV pass of 3 rows
-    (7, 512, 4096, True),       # FP32-MFMA projection, one per-tensor scale
+    (7, 512, 4096, True),       # batched kernel, one per-tensor scale
     (1, 77, 1001, False),       # odd K: any-shape GEMV
     (2, 50, 31, True),          # K below one chunk
     (1, 256, 20480, False),     # K past one GEMV pass
-    (24, 512, 4096, False),     # limb GEMM (M >= 17), one scale per row
-    (40, 300, 1024, True),      # limb GEMM, one per-tensor scale, ragged N
-    (16, 1000, 4064, False),    # FP32-MFMA projection (K % 128 != 0), one scale per row
-    (9, 300, 2080, True),       # FP32-MFMA projection (K % 128 != 0), one per-tensor scale
+    (24, 512, 4096, False),     # ... one scale per row
+    (40, 300, 1024, True),      # two slabs of rows, one per-tensor scale, ragged N
+    (16, 1000, 4064, False),    # K % 128 != 0, one scale per row
+    (9, 300, 2080, True),       # K % 128 != 0, one per-tensor scale
 ])
 def test_w4a32_linear_per_channel(cuda, m, n, k, scalar):
     print(f"case w4a32_linear m={m} n={n} k={k} scalar={scalar}", flush=True)
@@ -87,12 +87,12 @@ def test_quantize_weight_int4_non_finite(cuda):
 @pytest.mark.parametrize("m,n,k,gs", [
     (1, 300, 1000, 40),     # group 40, K % 32 != 0
     (2, 256, 4096, 128),    # power-of-two group 128 on the streaming GEMV
-    (6, 256, 4096, 128),    # ... and on the MFMA projection
+    (6, 256, 4096, 128),    # ... and on the batched kernel
     (1, 128, 28672, 32),    # K past one GEMV pass (Llama-70B intermediate)
     (1, 64, 1001, 32),      # odd K, short last group
     (5, 96, 100, 20),       # 5 rows, odd shape: any-shape GEMV
-    (40, 256, 4096, 128),   # group 128 on the limb GEMM (M >= 17)
-    (18, 130, 384, 64),     # group 64, two slabs (one of 2 rows), ragged N
+    (40, 256, 4096, 128),   # ... with two slabs of rows
+    (18, 130, 384, 64),     # group 64, a partial slab, ragged N
 ])
 def test_w4_grouped_general_shapes(cuda, m, n, k, gs):
     print(f"case w4a32_grouped_linear m={m} n={n} k={k} gs={gs}", flush=True)

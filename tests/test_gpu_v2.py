@@ -188,7 +188,7 @@ def test_vnni_semantics_fused_mlp(cuda, m, k, inter):
     """fused_swiglu_mlp_w4a32 at group 64 under W4A8 semantics: x's bytes into the
     gate / up pair, h's bytes into the down projection (fused_ops.rs:215-232,
     409-421), on each MLP path (M = 1 GEMV, 2 GEMV passes, 4 small-batch f16
-    MFMA, 32 FP32 MFMA, K % 32 != 0 any-shape), with biases and a residual."""
+    MFMA, 32 batched f16 MFMA, K % 32 != 0 any-shape), with biases and a residual."""
     print(f"case vnni fused mlp m={m} k={k} inter={inter}", flush=True)
     g = synth.rng(98, m, k, inter)
     x = synth.activations(g, m, k)

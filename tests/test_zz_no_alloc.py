@@ -44,9 +44,8 @@ def call(name, t, m, k, inter, gs, dev):
 
 def test_noalloc_matches_allocating_entry(cuda):
     # first Llama-3-8B MLPs at M = 16 and 8 (small-batch f16 MFMA; M = 16 needs
-    # 11.3 MB of the 16 MiB scratch), then smaller ones at M = 3 (same path) and
-    # M = 1 (the GEMV record path): the scratch keeps the previous call's
-    # contents.
+    # 11.3 MB of the 16 MiB scratch), then smaller ones at M = 3 and M = 1 (the
+    # GEMV record path): the scratch keeps the previous call's contents.
     for seed, m, k, inter in ((65, 16, 4096, 14336), (61, 8, 4096, 14336), (63, 3, 1024, 2048),
                               (62, 1, 1024, 2048)):
         print(f"case noalloc mlp m={m} k={k} inter={inter}", flush=True)
@@ -62,7 +61,7 @@ def test_noalloc_matches_allocating_entry(cuda):
 
 
 def test_noalloc_rejects_oversized_scratch(cuda):
-    # M = 64 runs the FP32-MFMA pair, whose split-K partials exceed the 16 MiB scratch
+    # the count that the entry point promises for M = 64 exceeds the 16 MiB scratch
     m, k, inter = 64, 4096, 14336
     print(f"case noalloc size limit m={m} k={k} inter={inter}", flush=True)
     dev = cuda
