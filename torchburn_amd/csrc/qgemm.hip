@@ -22,7 +22,8 @@
 // 22 bits, and where the large ones meet zero codes nothing else is left of the
 // sum.  A row in whose K range more than one in 16 nonzero elements is that small,
 // or whose largest is past 2^100, is marked by a negative 2^-e, and its slab of
-// 32 rows is multiplied from the f32 activations on f32 MFMA instead (wide_slab).
+// 32 rows is multiplied from the f32 activations on three bf16 limbs, which hold
+// an f32 whole (wide_slab).
 // Under that share the small elements' error, 2^-39 of the largest each, stays
 // below the f32 rounding of the sum of the others, 15 times as many and each at
 // least 2^-17 of the largest.  N(0, 1) rows are marked from a channel of 5100 to
@@ -78,6 +79,7 @@ using namespace gemv;
 namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -313,32 +315,45 @@ struct QTile {
         }
     }
 
-    // Group g of the stage at g0 for one slab (MT 1) in f32: xg is element 16 h of
-    // the group in the lane's row, scaled by up.
-    __device__ __forceinline__ void compute_wide(const float *xg, float up, int g, int g0,
+    // Group g of the stage at g0 for one slab (MT 1) on three bf16 limbs: x is the
+    // lane's half of the group (elements 16 h .. 16 h + 15 of its row), up its 2^e.
+    __device__ __forceinline__ void compute_wide(const f32x4 (&x)[4], float up, int g, int g0,
                                                  const Stage &st, f32x16 (&acc)[1][NT],
                                                  f32x16 (&run)[1][NT]) const {
-        f32x4 v[4];
+        const float sgn = negated(g0 + g) ? -1.f : 1.f;
+        h8 H[NT][2];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = reinterpret_cast<const f32x4 *>(xg)[j] * up;
+        for (int nt = 0; nt < NT; ++nt) expand(st, nt, g, g0, H[nt]);
+        f32x16 D[NT] = {};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            b8 A[3];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int el = 8 * u + (FMT == Q_W8 ? e : slot_elem(e));
+                const float v = x[el >> 2][el & 3] * (sgn * up);
+                const float r1 = fabsf(v) < INFINITY ? v - (float)(__bf16)v : 0.f;
+                A[0][e] = (__bf16)v;
+                A[1][e] = (__bf16)r1;
+                A[2][e] = (__bf16)(r1 - (float)(__bf16)r1);
+            }
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                b8 B;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) B[e] = (__bf16)(float)H[nt][u][e];
+#pragma unroll
+                for (int l = 2; l >= 0; --l)
+                    D[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[l], B, D[nt], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);   // one step's limbs in registers at a time
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
-            h8 B[2];
-            expand(st, nt, g, g0, B);
-            f32x16 D = {};
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int el = 8 * u + (FMT == Q_W8 ? e : slot_elem(e));
-                    D = __builtin_amdgcn_mfma_f32_32x32x2f32(v[el >> 2][el & 3], (float)B[u][e], D,
-                                                             0, 0, 0);
-                }
-            const float s = scale(st, nt, g);
+            const float s = sgn * scale(st, nt, g);
             f32x16 &to = SM == 2 ? run[0][nt] : acc[0][nt];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) to[r] = fmaf(D[r], s, to[r]);
-            __builtin_amdgcn_sched_barrier(0);   // few registers rather than overlap
+            for (int r = 0; r < 16; ++r) to[r] = fmaf(D[nt][r], s, to[r]);
         }
     }
 
@@ -485,9 +500,13 @@ __device__ __forceinline__ int store_tile(const QArgs &a, const QTile<FMT, MT, N
     return left;
 }
 
-// The results of one slab with rows of wide range, from the f32 activations: K
-// range and columns as the block's, 16 f32 MFMAs per group in place of 4 in f16 (8
-// times the matrix time; only such slabs pay it, after the block's other work).
+// The results of one slab with rows of wide range, on three bf16 limbs: K range and
+// columns as the block's, 6 MFMAs per group in place of 4.  The waves read the
+// activations themselves, one group ahead, and split them: bound by those reads and
+// the splitting.  Only such slabs pay for it, after the block's other work.  us for
+// INT4, group 32, without such rows / with one / all of them: 64 x 14336 x 4096 34 /
+// 100 / 99, 512 rows 137 / 290 / 452 (on 16 f32 MFMAs per group, without reading
+// ahead: 126 / 125 and 478 / 814).
 template <int FMT, int NT, int SM, bool PAIR>
 __device__ __forceinline__ void wide_slab(const QArgs &a, int bx, int split, int slab,
                                           const float *inv) {
@@ -496,17 +515,29 @@ __device__ __forceinline__ void wide_slab(const QArgs &a, int bx, int split, int
     const int gb = split * a.slen, ge = min(gb + a.slen, a.groups);
     T t(a);
     t.rows(bx);
-    // rows past m repeat the last one and are not stored
+    // rows past m repeat the last one and are not stored, groups past K the last one
+    // and are not added
     const float *xr = a.x + (size_t)min(slab * kSlab + t.i, a.m - 1) * a.k + 16 * t.h;
+    auto fetch = [&](int g, f32x4 (&v)[4]) {
+        const f32x4 *p = reinterpret_cast<const f32x4 *>(xr + 32 * (size_t)min(g, t.chunks - 1));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = p[j];
+    };
     const float up = 1.0f / fabsf(inv[t.i]);   // a power of two
     f32x16 acc[1][NT] = {}, run[1][NT] = {};
+    f32x4 xa[4], xb[4];
+    typename T::Stage st;
+    fetch(gb, xa);
 #pragma unroll 1
     for (int g = gb; g < ge; g += SG) {
-        typename T::Stage st;
         t.load(g, st);
 #pragma unroll
-        for (int j = 0; j < SG; ++j)
-            if (g + j < t.chunks) t.compute_wide(xr + 32 * (size_t)(g + j), up, j, g, st, acc, run);
+        for (int j = 0; j < SG; j += 2) {
+            fetch(g + j + 1, xb);
+            if (g + j < t.chunks) t.compute_wide(xa, up, j, g, st, acc, run);
+            fetch(g + j + 2, xa);
+            if (g + j + 1 < t.chunks) t.compute_wide(xb, up, j + 1, g, st, acc, run);
+        }
         if (((g - gb) & (kRun / 32 - 1)) == kRun / 32 - SG) T::flush(acc, run);
     }
     T::flush(acc, run);
