@@ -620,9 +620,11 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
 // kernel (FP32 MFMA with split K, which this replaced: 9.8), 16 x 4096 x 4096
 // 13.9 / 14.8 (14.7), 37 x 4805 x 1600 in v2 15.2 / 16.6 (19.3), 13 x 4605 x 1984
 // in INT8 12.5 / 13.8 (35 as GEMV passes).
-// (Three blocks a CU where the registers allow it, by the LDS they take.)
+// (Three blocks a CU, as many as their LDS allows, where the registers do; the LONG
+// form spills at three: 20 rows, N 2048, K 8192 13.4 us against 12.2.)
 template <int FMT, int NT, int SM, bool PAIR, bool LONG>
-__global__ __launch_bounds__(256, NT == 1 && (FMT == Q_W8 || (FMT == Q_W4 && SM != 2)) ? 3 : 2)
+__global__ __launch_bounds__(
+    256, NT == 1 && !LONG && (FMT == Q_W8 || (FMT == Q_W4 && SM != 2)) ? 3 : 2)
     void k_qdirect(QArgs a) {
     using T = QTile<FMT, 1, NT, SM, PAIR>;
     constexpr int SG = T::SG, PC = kDirectGroups * 32 / 64;   // pieces of 8 per lane
