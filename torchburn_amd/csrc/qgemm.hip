@@ -20,14 +20,17 @@
 //
 // Rows of wide range.  Elements below 2^-17 of the row's largest keep fewer than
 // 22 bits, and where the large ones meet zero codes nothing else is left of the
-// sum.  A row in whose K range more than one in 16 nonzero elements is that small,
-// or whose largest is past 2^100, is marked by a negative 2^-e, and its slab of
-// 32 rows is multiplied from the f32 activations on three bf16 limbs, which hold
-// an f32 whole (wide_slab).
-// Under that share the small elements' error, 2^-39 of the largest each, stays
-// below the f32 rounding of the sum of the others, 15 times as many and each at
-// least 2^-17 of the largest.  N(0, 1) rows are marked from a channel of 5100 to
-// 10300 on.  Counting takes 0 to 0.3 us of a call (37 x 4805 x 1600 in v2 14.6 ->
+// sum.  A row in whose K range more than one in 16 nonzero elements is that small
+// and fewer than 8 lie between them and 2^-10 of the largest, or whose largest is
+// past 2^100, is marked by a negative 2^-e, and its slab of 32 rows is multiplied
+// from the f32 activations on three bf16 limbs, which hold an f32 whole (wide_slab).
+// N(0, 1) rows of K = 4096 are marked from a channel of 250000 to 500000 on; just
+// below, the small elements' error, up to 2^-39 of the largest each, adds 2e-7 to the
+// results' f32 rounding of about 1.3e-7, and with a channel of 1e5 6e-8 (rms).  The
+// gap tells such rows from those of silu(g) u with large g, most of whose elements
+// all but vanish beside the others (511 rows of 14336, a few hundred of them within
+// 2^-17: a prompt of synthetic weights 30.4 ms with such rows marked, not marked 20.1).
+// Counting takes 0 to 0.3 us of a call (37 x 4805 x 1600 in v2 14.6 ->
 // 14.9 us, 64 x 14336 x 4096 31.2 -> 31.3).
 // Inf and NaN travel through the first limb, as in the reference's
 // unpack-and-fma.  An MFMA step rounds its sum down, which over a long row adds
@@ -50,16 +53,16 @@
 // h, so K slot (u, h, e) of a group (step u of two) is element
 // 16 h + 8 u + e, and the records hold x in that order.
 //
-// Bound: the matrix cores, at the clock this card holds under a dense f16
-// product (a large library product in bf16 runs at 1.2 PFLOP/s, half the
-// nominal rate).  Measured on whole calls, against the kernel on fixed-point
+// Bound, from 256 rows: 950-1020 TFLOP/s of MFMA work (a large library product in
+// bf16 runs at 1.2 PFLOP/s, half the nominal rate), with the matrix cores busy 0.49
+// of the time and the waves waiting 0.43 of theirs.  Measured on whole calls, against the kernel on fixed-point
 // limbs with an exponent per 64 elements and two more MFMAs per group for the
 // -8 of the weights that this one replaced:
 //   Llama-3-8B gate/up pair, 512 rows, group 32    251 us, 479 TFLOP/s (958 in
 //                                                  MFMA work)
-//   Llama-3-8B MLP, 512 rows, group 64             942 -> 382 us
-//   64 rows, N = 14336, K = 4096, group 32         54.0 -> 31.0 us
-//   Llama-3-8B MLP in INT8, 128 rows               2559 -> 154 us, against GEMV
+//   Llama-3-8B MLP, 512 rows, group 64             942 -> 393 us
+//   64 rows, N = 14336, K = 4096, group 32         54.0 -> 31.1 us
+//   Llama-3-8B MLP in INT8, 128 rows               2559 -> 151 us, against GEMV
 //                                                  passes of 2 rows each
 // The error against 64 bits went from 6.2e-7 to 1.4e-7 for INT4 (activations
 // with large channels: the limbs follow each element's own size) and from
@@ -370,6 +373,13 @@ struct QTile {
     }
 };
 
+// The sum over 8 consecutive lanes.
+__device__ __forceinline__ float sum8(float v) {
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) v += shfl_xor_u(v, o);
+    return v;
+}
+
 // Consecutive tiles (row blocks of the same columns first) on one XCD: blocks
 // go to the 8 XCDs round robin, the grid is a multiple of 8.
 __device__ __forceinline__ int block_tile() {
@@ -378,11 +388,10 @@ __device__ __forceinline__ int block_tile() {
 }
 
 // The limbs of 8 consecutive elements a, b of a row, scaled by sc (2^e, negated
-// for the groups negated() names), W4: slots in nibble order.  A row is of wide
-// range when the sum of `lack`, 15 for an element that keeps fewer than 22 bits
-// and -1 for another, is positive over its nonzero elements; here zeros count as
-// short too, an upper bound that ordinary rows keep negative in every wave, so
-// that only others pay for counting their zeros (zeros8).
+// for the groups negated() names), W4: slots in nibble order.  `lack` sums 15 for
+// an element that keeps fewer than 22 bits, or is zero, and -1 for another: ordinary
+// rows keep it negative in every wave, so that only others pay for a closer look
+// (Spread).
 template <bool W4>
 __device__ __forceinline__ void limbs8(const f32x4 &a, const f32x4 &b, float sc, h8 &l1, h8 &l2,
                                        int &lack) {
@@ -400,12 +409,19 @@ __device__ __forceinline__ void limbs8(const f32x4 &a, const f32x4 &b, float sc,
     asm("" : "+v"(lack));   // summed here, not kept as 8 flags for later
 }
 
-__device__ __forceinline__ int zeros8(const f32x4 &a, const f32x4 &b) {
-    int z = 0;
+// What decides on a row whose lack is positive: its zeros, and the elements from
+// 2^-17 to 2^-10 of the largest (scaled: 2^-2 to 2^5).
+struct Spread {
+    int zeros = 0, mid = 0;
+    __device__ __forceinline__ void add(const f32x4 &a, const f32x4 &b, float sc) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) z += (a[e] == 0.f) + (b[e] == 0.f);
-    return z;
-}
+        for (int e = 0; e < 8; ++e) {
+            const float v = fabsf((e < 4 ? a : b)[e & 3]);
+            zeros += v == 0.f;
+            mid += v * sc >= 0.25f && v * sc < 32.f;
+        }
+    }
+};
 
 // The largest finite magnitude of a, b and mx.
 __device__ __forceinline__ float max_finite(float mx, const f32x4 &a, const f32x4 &b) {
@@ -427,10 +443,11 @@ __device__ __forceinline__ int row_exp(float mx) {
     return mx > kLargest ? 100 - E : mx > 0.f ? min(15 - E, 126) : 0;
 }
 
-// 2^-e as stored: negative for a row of wide range.
-__device__ __forceinline__ float row_inv(int e, float mx, float score) {
-    const float v = ldexpf(1.f, -e);
-    return mx > kLargest || score > 0.f ? -v : v;
+// 2^-e as stored: negative for a row of wide range, which has more than one short
+// element in 16 (lack, over the nonzero ones, positive) and a gap above them.
+__device__ __forceinline__ float row_inv(float mx, float lack = 0.f, float mid = 0.f) {
+    const float v = ldexpf(1.f, -row_exp(mx));
+    return mx > kLargest || (lack > 0.f && mid < 8.f) ? -v : v;
 }
 
 // The block's results, scaled by their rows' 2^-e (inv: of slab0's first row
@@ -613,8 +630,8 @@ __global__ __launch_bounds__(256, 2) void k_qgemm(QArgs a) {
 // The same projection for few rows: the block builds the limbs of its 32 rows
 // itself, straight into LDS and while its first weights are on their way, 12
 // groups at a time, and needs no record kernel before it.  Up to 12 groups per
-// split x is read once and the loop has no barrier; a longer range (LONG, for
-// calls with little scratch) reads x once more before, for the rows' maxima.
+// split x is read once and the loop has no barrier; a longer range (LONG) reads x
+// once more before, for the rows' maxima.
 // Wave w converts rows 8 w .. 8 w + 7, eight lanes each.  Small calls are bound
 // by their launches: 41 x 904 x 1088 takes 8.9 us here, 12.4 with the record
 // kernel (FP32 MFMA with split K, which this replaced: 9.8), 16 x 4096 x 4096
@@ -699,23 +716,20 @@ __global__ __launch_bounds__(
         }
         T::flush(acc, run);
     }
-    float sc = row < a.m ? (float)lack : 0.f;
-#pragma unroll
-    for (int o = 1; o < 8; o <<= 1) sc += shfl_xor_u(sc, o);
+    float sc = row < a.m ? (float)lack : 0.f, mid = 0.f;
+    sc = sum8(sc);
     if (__any(sc > 0.f)) {
-        int z = 0;
+        Spread sp;
 #pragma unroll 1
         for (int kk = gb * 32 + 8 * c0; kk < min(ge * 32, a.k); kk += 64) {
             f32x4 va, vb;
             piece(kk, va, vb);
-            z += zeros8(va, vb);
+            sp.add(va, vb, up);
         }
-        float zc = (float)(15 * z);
-#pragma unroll
-        for (int o = 1; o < 8; o <<= 1) zc += shfl_xor_u(zc, o);
-        sc -= zc;
+        sc -= 15.f * sum8((float)sp.zeros);
+        mid = sum8((float)sp.mid);
     }
-    if (c0 == 0) inv[r] = row_inv(row_exp(mx), mx, sc);
+    if (c0 == 0) inv[r] = row_inv(mx, sc, mid);
     __syncthreads();
     if (store_tile<false>(a, t, acc, bx, split, mz, inv))
         wide_slab<FMT, NT, SM, PAIR>(a, bx, split, mz, inv);
@@ -727,14 +741,15 @@ __global__ __launch_bounds__(
 // Bound by how many CUs take part (a row's largest magnitude ties its K range to
 // one block) against the length of the stores (16 R bytes).  us at 8 / 4 / 2 rows:
 // 64 x 4096 5.7 / 4.9 / 4.1, 128 rows of 4096 and 14336 8.2 / 6.4 / 6.4 on average,
-// 512 rows 11.6 / 9.6 / 12.4.
+// 512 rows 11.6 / 9.6 / 12.4 (without the count of short elements; with it, at the
+// chosen rows, 4.5, 5.9 and 9.8).
 template <bool W4, int R>
 __global__ __launch_bounds__(1024, 8) void k_qsplit(const float *__restrict__ x,
                                                  uint8_t *__restrict__ rec,
                                                  float *__restrict__ inv, int m, int k, int slabs,
                                                  int groups, int slen) {
     constexpr int PC = 4;   // pieces kept in registers
-    __shared__ float red[16][R];
+    __shared__ float red[16][R], mids[16][R];
     __shared__ int any_short;
     const int t = threadIdx.x, tpr = blockDim.x / R, p0 = t / R;
     const int row = blockIdx.x * R + t % R, split = blockIdx.y;
@@ -772,7 +787,7 @@ __global__ __launch_bounds__(1024, 8) void k_qsplit(const float *__restrict__ x,
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t % R]);
     const int e = row_exp(mx);
     const float up = ldexpf(1.f, e);
-    if (t < R) inv[(size_t)split * slabs * kSlab + row] = row_inv(e, mx, 0.f);
+    if (t < R) inv[(size_t)split * slabs * kSlab + row] = row_inv(mx);
     int lack = 0;
     auto put = [&](int p, const f32x4 &a, const f32x4 &b) {
         const int kk = k0 + 8 * p, g = kk >> 5, q = (kk >> 3) & 3;
@@ -803,22 +818,32 @@ __global__ __launch_bounds__(1024, 8) void k_qsplit(const float *__restrict__ x,
     mx = 0.f;
     for (int w = 0; w < (int)(blockDim.x >> 6); ++w) mx = fmaxf(mx, red[w][t % R]);
     __syncthreads();
-    int z = 0;
+    Spread sp;
+    const float scale = ldexpf(1.f, row_exp(mx));
 #pragma unroll 1
     for (int p = p0; p < pieces; p += tpr) {
         f32x4 a, b;
         fetch(p, a, b);
-        if (k0 + 8 * p < k) z += zeros8(a, b);
+        if (k0 + 8 * p < k) sp.add(a, b, scale);
     }
-    float zc = (float)(15 * z);
+    float zc = (float)sp.zeros, mc = (float)sp.mid;
 #pragma unroll
-    for (int o = R; o < 64; o <<= 1) zc += shfl_xor_u(zc, o);
-    if ((t & 63) < R) red[t >> 6][t % R] = sc - zc;
+    for (int o = R; o < 64; o <<= 1) {
+        zc += shfl_xor_u(zc, o);
+        mc += shfl_xor_u(mc, o);
+    }
+    if ((t & 63) < R) {
+        red[t >> 6][t % R] = sc - 15.f * zc;
+        mids[t >> 6][t % R] = mc;
+    }
     __syncthreads();
     if (t >= R) return;
-    sc = 0.f;
-    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) sc += red[w][t];
-    inv[(size_t)split * slabs * kSlab + row] = row_inv(row_exp(mx), mx, sc);
+    sc = mc = 0.f;
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) {
+        sc += red[w][t];
+        mc += mids[w][t];
+    }
+    inv[(size_t)split * slabs * kSlab + row] = row_inv(mx, sc, mc);
 }
 
 // Sum of the split-K partials in split order, then the epilogue.  res may be y

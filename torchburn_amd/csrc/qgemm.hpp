@@ -26,7 +26,7 @@ struct QGemmParams {
     int s0_len, s1_len;    // 1 or n scales (not grouped)
 };
 
-// Shapes the kernel takes: m >= 1, k a multiple of 32 (v2: of 64) up to 2^24.
+// Shapes the kernel takes: k a multiple of 32 (v2: of 64) up to 2^30, m below 2^24.
 bool qgemm_shape_ok(int64_t m, int64_t n, int64_t k, int fmt);
 
 // Whether INT8 rows go to this kernel rather than to GEMV passes of 2 rows that
