@@ -17,8 +17,8 @@ ONE, RUN = 5, slice(64, 96)   # channels of zero codes: a single one, a group of
 
 
 def close(y, x, w):
-    """check(), and every row's 2-norm within what f32 sums show (1.3e-7 at K = 4096)
-    and the limbs' part just below the line (2e-7) come to, with half as much again."""
+    """check(), and every row's 2-norm within 3.5 times what f32 sums show (1.4e-7 at
+    K = 14336, measured with and without large channels)."""
     check(y, x, w)
     ref = x.astype(np.float64) @ w.T
     assert (np.linalg.norm(y - ref, axis=1) <= 5e-7 * np.linalg.norm(ref, axis=1)).all()

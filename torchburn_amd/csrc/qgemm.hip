@@ -24,14 +24,15 @@
 // and fewer than 8 lie between them and 2^-10 of the largest, or whose largest is
 // past 2^100, is marked by a negative 2^-e, and its slab of 32 rows is multiplied
 // from the f32 activations on three bf16 limbs, which hold an f32 whole (wide_slab).
-// N(0, 1) rows of K = 4096 are marked from a channel of 250000 to 500000 on; just
-// below, the small elements' error, up to 2^-39 of the largest each, adds 2e-7 to the
-// results' f32 rounding of about 1.3e-7, and with a channel of 1e5 6e-8 (rms).  The
-// gap tells such rows from those of silu(g) u with large g, most of whose elements
-// all but vanish beside the others (511 rows of 14336, a few hundred of them within
-// 2^-17: a prompt of synthetic weights 30.4 ms with such rows marked, not marked 20.1).
-// Counting takes 0 to 0.3 us of a call (37 x 4805 x 1600 in v2 14.6 ->
-// 14.9 us, 64 x 14336 x 4096 31.2 -> 31.3).
+// Rows of N(0, 1) with one channel of 1e3 to 1e9 on zero codes are off by 0.8e-7 to
+// 1.4e-7 of their 2-norm throughout, K from 512 to 14336, INT4 and INT8, as without
+// the channel (two limbs alone, INT4: 1.5e-6 at 1e6, 1.6e-3 at 1e9).  The gap tells
+// such rows from those of silu(g) u with large g, most of whose elements all but
+// vanish beside the others (511 rows of 14336, a few hundred of them within 2^-17: a
+// prompt of synthetic weights 30.4 ms with such rows marked, not marked 20.1).
+// Counting takes 0 to 0.3 us of a call (37 x 4805 x 1600 in v2 14.6 -> 14.9 us,
+// 64 x 14336 x 4096 31.2 -> 31.3).
+//
 // Inf and NaN travel through the first limb, as in the reference's
 // unpack-and-fma.  An MFMA step rounds its sum down, which over a long row adds
 // up (a mean error of 1.3e-7 of the results' size at K = 14336): the records
