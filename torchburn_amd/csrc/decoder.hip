@@ -717,11 +717,17 @@ struct Decoder {
     uint8_t *pf_limb = nullptr;
     uint8_t *pf_hrec = nullptr;   // records of h, [kLimbMaxM, I]
     size_t pf_limb_bytes = 0;
+    // Whether the batch may take it: its activations are in fixed point, one step per
+    // 64 elements, where the steps that a prompt of up to 15 tokens stands for have one
+    // per 16 (error of eight Llama-3-8B layers' logits at 9 tokens: steps 1.98e-6, this
+    // 2.15e-6, the GEMM 1.55e-6; us for two layers 1262 / 354 / 407).
+    bool pf_fixed = false;
+    static constexpr int kFixedPrompt = 16;
     bool limb_gemm(const float *xin, const void *w, const float *s, const float *b,
                    const void *w2, const float *s2, const float *res, float *y, int m, int n,
                    int k, int &rc, uint8_t *rec_out = nullptr, const uint8_t *rec_in = nullptr) {
         const bool pair = w2 != nullptr;
-        if (!pf_limb || m < 3 || m > kLimbMaxM || !limb_shape_ok(m, n, k, pair) ||
+        if (!pf_limb || !pf_fixed || m < 3 || m > kLimbMaxM || !limb_shape_ok(m, n, k, pair) ||
             !limb_wins((int64_t)n * k * (pair ? 2 : 1)))
             return false;
         const size_t rb = up256(limb_records_bytes(m, k));
@@ -806,7 +812,7 @@ struct Decoder {
     bool under_cap(int64_t start, int64_t n) const { return start + n <= (int64_t)attn_cap; }
 
     // Prompts from this length run as batches (us for 3 tokens, batched / step
-    // by step: eight Llama-3-8B layers in INT4 808 / 1496, in INT8 1129 / 1829,
+    // by step: eight Llama-3-8B layers in INT4 913 / 1316, in INT8 1000 / 1549,
     // Qwen2.5-0.5B 1399 / 2546 and 1358 / 2530; for 2 tokens the INT4 layers
     // 1193 / 1014).
     static constexpr int kBatchPrompt = 3;
@@ -873,6 +879,7 @@ struct Decoder {
                         float *rows_out = nullptr) {
         int rc = layers_set(), rows = 0;
         if (rc || (rc = prefill_alloc(n, start, &rows))) return rc;
+        pf_fixed = rows_out || n >= kFixedPrompt;
         const int nq = (hq + 2 * hkv) * hd;
         // Host copy of the whole prompt, alive until the closing synchronize.
         std::vector<int> tok32(tokens, tokens + n);
